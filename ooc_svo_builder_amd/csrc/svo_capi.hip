@@ -289,7 +289,7 @@ void svo_ctx_destroy(svo_ctx* ctx) {
   c.glog.clear();
   DevBuf* bufs[] = {&c.tris, &c.jobdev, &c.batch_tris, &c.hitbox, &c.part_lists, &c.unitdev,
                     &c.table, &c.pool, &c.pool8, &c.grid8, &c.counters, &c.large_unit,
-                    &c.large_tri, &c.large_cols, &c.large_off, &c.occ_list, &c.bcount,
+                    &c.large_tri, &c.large_rows, &c.large_jobs, &c.occ_list, &c.bcount,
                     &c.wprefix, &c.winner, &c.scan_scratch, &c.codes, &c.records, &c.nodes,
                     &c.lvl_code, &c.lvl_size, &c.lvl_mask, &c.lvl_first, &c.lvl_start,
                     &c.lvl_aux, &c.lvl_leafp, &c.lvl_pidx, &c.lvl_isize, &c.lvl_cache,

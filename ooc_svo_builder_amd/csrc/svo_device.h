@@ -49,13 +49,13 @@ __host__ __device__ __forceinline__ void unmorton3(uint64_t m, uint32_t& x, uint
 // Scalar semantics of the reference's x86 build
 // ------------------------------------------------------------------------------------
 // static_cast<int>(float) as cvttss2si: NaN / out of range -> INT_MIN
-__device__ __forceinline__ int trunc_i32_x86(float f) {
+__host__ __device__ __forceinline__ int trunc_i32_x86(float f) {
   if (!(f >= -2147483648.0f && f < 2147483648.0f)) return (int)0x80000000;
   return (int)f;
 }
-__device__ __forceinline__ float min_std(float a, float b) { return (b < a) ? b : a; }
-__device__ __forceinline__ float max_std(float a, float b) { return (a < b) ? b : a; }
-__device__ __forceinline__ int clamp_i(int v, int lo, int hi) {
+__host__ __device__ __forceinline__ float min_std(float a, float b) { return (b < a) ? b : a; }
+__host__ __device__ __forceinline__ float max_std(float a, float b) { return (a < b) ? b : a; }
+__host__ __device__ __forceinline__ int clamp_i(int v, int lo, int hi) {
   return v < lo ? lo : (v > hi ? hi : v);
 }
 
@@ -173,6 +173,17 @@ __device__ __forceinline__ uint32_t wave_incl_scan<uint32_t>(uint32_t v) {
   x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);  // row_bcast:15
   x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
   return (uint32_t)x;
+}
+// inclusive maximum over the lanes of a wave: the same moves
+__device__ __forceinline__ uint32_t wave_incl_max(uint32_t v) {
+  auto up = [](uint32_t a, int b) { return max(a, (uint32_t)b); };
+  v = up(v, __builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true));
+  v = up(v, __builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true));
+  v = up(v, __builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true));
+  v = up(v, __builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true));
+  v = up(v, __builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));
+  v = up(v, __builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));
+  return v;
 }
 // 64-bit form: the same moves on both halves of the value, 64-bit adds
 template <int CTRL, int ROWS, bool BOUND>

@@ -103,7 +103,7 @@ enum Counter : int {
   kCtrNumOcc = 3,     // occupied bricks after compaction
   kCtrNumVox = 4,     // voxels of the current pass
   kCtrLevelN = 5,     // node count of the level being built
-  kCtrCols = 6,       // columns of the large tier
+  kCtrLargeJobs = 6,  // jobs of the large tier past its triangles' first ones
   kCtrError = 15,     // sticky: internal consistency failures (cleared per job)
   kCtrPartTotal = 16, // partition list length
   kNumCounters = 32
@@ -132,7 +132,7 @@ struct VoxTuning {
   int small_cols = 1024;    // columns above which a triangle goes to the large tier
   int direct_cols = 16;     // columns up to which a triangle's own thread walks them
   int tile_blocks = 1024;   // persistent grid of the small tier
-  int large_blocks = 2048;  // grid of the large tier (grid-stride)
+  int large_blocks = 1024;  // grid of the large tier (grid-stride)
 };
 
 struct StageTimes {
@@ -265,8 +265,8 @@ struct Context {
   uint64_t pool_cap = 0;        // slots of pool8 (and of pool) on the touch path
   uint64_t dense_limit = 0;     // largest dense grid in bytes (set from free HBM)
   DevBuf counters;
-  DevBuf large_unit, large_tri, large_cols, large_off;
-  DevBuf large_walk;  // walk constants of large triangles (44 words each, capped)
+  DevBuf large_unit, large_tri, large_rows, large_jobs;
+  DevBuf large_walk;  // set-up of large triangles (capped)
   DevBuf occ_list, bcount, wprefix, winner;
   DevBuf scan_scratch;
   DevBuf scan_status;  // status words of the single-pass scans of a voxelize pass

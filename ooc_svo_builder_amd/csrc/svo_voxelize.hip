@@ -7,9 +7,9 @@
 //
 // Voxelize (voxelizer.cpp:138-307): the Schwarz-Seidel conservative triangle/box test in
 // FP32 with the reference's expression order. Work is split in two tiers:
-//   * small triangles: one thread walks all columns of its triangle's clamped bbox;
-//   * large triangles: one thread per column, the columns of all large triangles laid
-//     out by an exclusive scan of their column counts.
+//   * small triangles: a wave takes up to 64 of them, a lane walking its own triangle or all
+//     lanes sharing the tile's columns;
+//   * large triangles: jobs of some rows of a triangle each, a wave per job.
 // Columns run along the axis of the triangle's dominant normal component. Per column the
 // projection test in the plane across that axis is evaluated once (it does not depend
 // on the position along the column), and only the voxels of the plane slab, widened by
@@ -32,235 +32,11 @@
 #include "svo_device.h"
 #include "svo_internal.h"
 #include "svo_scan.h"
+#include "svo_walk.h"
 
 namespace svo {
 
 typedef unsigned long long ull;
-
-// One voxelize unit: one Morton-range partition of one job (a mesh). A batch voxelizes
-// many units in the same launches.
-struct VoxParams {
-  const float* tris;
-  const uint32_t* list;  // partition's triangle indices, nullptr = identity
-  uint32_t n;
-  int stride;  // floats per record: 9 binary, 21 payload
-  uint64_t mstart;
-  uint64_t bstart;  // mstart rounded down to a brick: origin of the brick table segment
-  int pmin[3], pmax[3];
-  float unit, unit_div;
-  float coord_limit;  // |vertex| beyond this walks full columns
-  double slab_margin; // voxels added on each side of the exact plane slab
-  double inv_unit;    // 1 / unit in double
-  int small_cols;
-  int direct_cols;     // triangles with at most this many columns: walked by their thread
-  uint32_t job;        // tag of the unit's codes (bits kJobShift and up)
-  int dense;           // 1: voxels in grid8; 0: in pool slots flagged by the touch pass
-  int wide;            // dense payload unit: 4-byte cells holding ~(first triangle)
-  uint64_t table_base; // first entry of the unit's segment of the brick table
-  uint8_t* grid8;      // dense byte grid of the unit (nullptr on the touch path)
-};
-
-struct Setup {
-  float n[3];
-  float d1, d2;
-  float ne[9][2];  // edge normals: xy e0..e2, yz e0..e2, zx e0..e2
-  float de[9];
-  int g0[3], g1[3];
-  int w;          // column axis
-  bool slab;      // restrict columns to the plane slab
-  double nv0, nc, nm;
-};
-
-// voxelizer.cpp:189-254 (bbox, clamp, normal, critical point, edge functions)
-__device__ __forceinline__ void setup_tri(const float* __restrict__ p, const VoxParams& P,
-                                          Setup& S) {
-  const float v0x = p[0], v0y = p[1], v0z = p[2];
-  const float v1x = p[3], v1y = p[4], v1z = p[5];
-  const float v2x = p[6], v2y = p[7], v2z = p[8];
-  const float u = P.unit;
-  {
-    const float mn0 = min_std(v0x, min_std(v1x, v2x)), mx0 = max_std(v0x, max_std(v1x, v2x));
-    const float mn1 = min_std(v0y, min_std(v1y, v2y)), mx1 = max_std(v0y, max_std(v1y, v2y));
-    const float mn2 = min_std(v0z, min_std(v1z, v2z)), mx2 = max_std(v0z, max_std(v1z, v2z));
-    S.g0[0] = clamp_i(trunc_i32_x86(mn0 * P.unit_div), P.pmin[0], P.pmax[0]);
-    S.g0[1] = clamp_i(trunc_i32_x86(mn1 * P.unit_div), P.pmin[1], P.pmax[1]);
-    S.g0[2] = clamp_i(trunc_i32_x86(mn2 * P.unit_div), P.pmin[2], P.pmax[2]);
-    S.g1[0] = clamp_i(trunc_i32_x86(mx0 * P.unit_div), P.pmin[0], P.pmax[0]);
-    S.g1[1] = clamp_i(trunc_i32_x86(mx1 * P.unit_div), P.pmin[1], P.pmax[1]);
-    S.g1[2] = clamp_i(trunc_i32_x86(mx2 * P.unit_div), P.pmin[2], P.pmax[2]);
-  }
-  const float e0x = v1x - v0x, e0y = v1y - v0y, e0z = v1z - v0z;
-  const float e1x = v2x - v1x, e1y = v2y - v1y, e1z = v2z - v1z;
-  const float e2x = v0x - v2x, e2y = v0y - v2y, e2z = v0z - v2z;
-  const float cx = e0y * e1z - e1y * e0z;
-  const float cy = e0z * e1x - e1z * e0x;
-  const float cz = e0x * e1y - e1x * e0y;
-  const float ss = (cx * cx + cy * cy) + cz * cz;
-  const float inv = 1.0f / sqrtf(ss);
-  const float nx = cx * inv, ny = cy * inv, nz = cz * inv;
-  S.n[0] = nx;
-  S.n[1] = ny;
-  S.n[2] = nz;
-  const float ccx = (nx > 0) ? u : 0.0f;
-  const float ccy = (ny > 0) ? u : 0.0f;
-  const float ccz = (nz > 0) ? u : 0.0f;
-  S.d1 = (nx * (ccx - v0x) + ny * (ccy - v0y)) + nz * (ccz - v0z);
-  S.d2 = (nx * ((u - ccx) - v0x) + ny * ((u - ccy) - v0y)) + nz * ((u - ccz) - v0z);
-
-  const float E[3][3] = {{e0x, e0y, e0z}, {e1x, e1y, e1z}, {e2x, e2y, e2z}};
-  const float V[3][3] = {{v0x, v0y, v0z}, {v1x, v1y, v1z}, {v2x, v2y, v2z}};
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    // XY plane (voxelizer.cpp:220-230)
-    float a = -1.0f * E[k][1], b = E[k][0];
-    if (nz < 0.0f) {
-      a = -1.0f * a;
-      b = -1.0f * b;
-    }
-    S.ne[k][0] = a;
-    S.ne[k][1] = b;
-    S.de[k] = ((-1.0f * (a * V[k][0] + b * V[k][1])) + max_std(0.0f, u * a)) + max_std(0.0f, u * b);
-    // YZ plane (:232-242)
-    a = -1.0f * E[k][2];
-    b = E[k][1];
-    if (nx < 0.0f) {
-      a = -1.0f * a;
-      b = -1.0f * b;
-    }
-    S.ne[3 + k][0] = a;
-    S.ne[3 + k][1] = b;
-    S.de[3 + k] = ((-1.0f * (a * V[k][1] + b * V[k][2])) + max_std(0.0f, u * a)) + max_std(0.0f, u * b);
-    // ZX plane (:244-254)
-    a = -1.0f * E[k][0];
-    b = E[k][2];
-    if (ny < 0.0f) {
-      a = -1.0f * a;
-      b = -1.0f * b;
-    }
-    S.ne[6 + k][0] = a;
-    S.ne[6 + k][1] = b;
-    S.de[6 + k] = ((-1.0f * (a * V[k][2] + b * V[k][0])) + max_std(0.0f, u * a)) + max_std(0.0f, u * b);
-  }
-
-  // column axis and slab restriction
-  const float ax = fabsf(nx), ay = fabsf(ny), az = fabsf(nz);
-  S.w = (az >= ax && az >= ay) ? 2 : (ax >= ay ? 0 : 1);
-  const float L = P.coord_limit;
-  const bool finite = (ax <= 2.0f) && (ay <= 2.0f) && (az <= 2.0f);  // false for NaN/inf
-  const bool near = fabsf(v0x) <= L && fabsf(v0y) <= L && fabsf(v0z) <= L && fabsf(v1x) <= L &&
-                    fabsf(v1y) <= L && fabsf(v1z) <= L && fabsf(v2x) <= L && fabsf(v2y) <= L &&
-                    fabsf(v2z) <= L;
-  S.slab = finite && near && fmaxf(ax, fmaxf(ay, az)) >= 0.5f;
-  S.nv0 = ((double)nx * v0x + (double)ny * v0y) + (double)nz * v0z;
-  S.nc = ((double)nx * ccx + (double)ny * ccy) + (double)nz * ccz;
-  S.nm = ((double)nx * (u - ccx) + (double)ny * (u - ccy)) + (double)nz * (u - ccz);
-}
-
-// ---------------------------------------------------------------- column walk
-// A triangle's voxels are tested column by column along its column axis w (the axis of
-// the dominant normal component); a column is fixed by its coordinates (a, b) on the two
-// other axes ua < va. The per-triangle constants are re-slotted once so that one
-// branch-free code path serves all three axes:
-//   * plane test t = (n0*px + n1*py) + n2*pz becomes t = (nw*pc + Ka) + Kb with
-//     Ka, Kb per column (Kb = +0 when w = z; a zero's sign never changes the decision);
-//   * the projection test in the plane across w (3 edges) depends on (pa, pb) only and
-//     is evaluated once per column: (h0*pa + h1*pb) + hd;
-//   * each edge of the two other planes is (cv*pc + cc*pconst) + de per voxel, where
-//     pconst is pb for one of them (plane P) and pa for the other (plane Q).
-// Every product and sum is the reference's own (voxelizer.cpp:257-287); only operands of
-// single additions are swapped, which is exact in IEEE arithmetic. The products of pb
-// (h1*pb, cc*pb of plane P, the plane-test term of b, the slab term of b) are the same
-// along a row of columns and are computed once per row.
-enum WalkF {
-  F_NW = 0, F_D1, F_D2, F_NUA, F_NVA,
-  F_H0 = 5, F_H1 = 8, F_HD = 11,
-  F_PV = 14, F_PC = 17, F_PD = 20,
-  F_QV = 23, F_QC = 26, F_QD = 29,
-  F_KA = 32, F_KB, F_ALO, F_AHI,
-  kWalkF = 36
-};
-enum WalkI { I_G0U = 0, I_G1U, I_G0V, I_G1V, I_G0W, I_G1W, I_WS, I_TRI, kWalkI = 8 };
-constexpr int kWalkWords = kWalkF + kWalkI;
-
-struct Walk {
-  float f[kWalkF];
-  int i[kWalkI];
-  __device__ __forceinline__ int w() const { return i[I_WS] & 3; }
-  __device__ __forceinline__ bool slab() const { return (i[I_WS] >> 2) & 1; }
-  __device__ __forceinline__ uint64_t columns() const {
-    return (uint64_t)(i[I_G1U] - i[I_G0U] + 1) * (uint64_t)(i[I_G1V] - i[I_G0V] + 1);
-  }
-  __device__ __forceinline__ uint64_t work() const {
-    return slab() ? columns() : columns() * (uint64_t)(i[I_G1W] - i[I_G0W] + 1);
-  }
-};
-
-// The plane roles for column axis w, as value selects: the hoisted plane's edges (H0, H1
-// in operand order (pa, pb), HD), plane P (its other coordinate is pb) and plane Q (pa)
-// with their column-coordinate factor (PV, QV), the other factor (PC, QC) and the offset
-// (PD, QD). Edges: xy = ne[0..2], yz = ne[3..5], zx = ne[6..8].
-//   w = 2: hoisted xy(pa, pb); P = yz(pb, pc); Q = zx(pc, pa)
-//   w = 0: hoisted yz(pa, pb); P = zx(pb, pc); Q = xy(pc, pa)
-//   w = 1: hoisted zx(pb, pa); P = yz(pc, pb); Q = xy(pa, pc)
-// (A branch per axis is merged by the compiler into an index on the edge arrays, which
-// puts them in scratch memory.)
-__device__ __forceinline__ void fill_planes(const Setup& S, Walk& K, int w) {
-  const bool w2 = (w == 2), w0 = (w == 0);
-  auto pick = [&](float a2, float a0, float a1) { return w2 ? a2 : (w0 ? a0 : a1); };
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    K.f[F_H0 + k] = pick(S.ne[k][0], S.ne[3 + k][0], S.ne[6 + k][1]);
-    K.f[F_H1 + k] = pick(S.ne[k][1], S.ne[3 + k][1], S.ne[6 + k][0]);
-    K.f[F_HD + k] = pick(S.de[k], S.de[3 + k], S.de[6 + k]);
-    K.f[F_PV + k] = pick(S.ne[3 + k][1], S.ne[6 + k][1], S.ne[3 + k][0]);
-    K.f[F_PC + k] = pick(S.ne[3 + k][0], S.ne[6 + k][0], S.ne[3 + k][1]);
-    K.f[F_PD + k] = pick(S.de[3 + k], S.de[6 + k], S.de[3 + k]);
-    K.f[F_QV + k] = pick(S.ne[6 + k][0], S.ne[k][0], S.ne[k][1]);
-    K.f[F_QC + k] = pick(S.ne[6 + k][1], S.ne[k][1], S.ne[k][0]);
-    K.f[F_QD + k] = pick(S.de[6 + k], S.de[k], S.de[k]);
-  }
-}
-
-// Re-slot a triangle's setup (voxelizer.cpp:189-254, see setup_tri) for the column walk.
-__device__ __forceinline__ void make_walk(const Setup& S, const VoxParams& P, uint32_t tri,
-                                          Walk& K) {
-  const int w = S.w;
-  const int ua = (w == 0) ? 1 : 0;
-  const int va = (w == 2) ? 1 : 2;
-  fill_planes(S, K, w);
-  const float n0 = S.n[0], n1 = S.n[1], n2 = S.n[2];
-  const float nw = (w == 0) ? n0 : (w == 1 ? n1 : n2);
-  const float nua = (ua == 0) ? n0 : n1;
-  const float nva = (va == 1) ? n1 : n2;
-  K.f[F_NW] = nw;
-  K.f[F_D1] = S.d1;
-  K.f[F_D2] = S.d2;
-  K.f[F_NUA] = nua;
-  K.f[F_NVA] = nva;
-  // plane slab in index space along w: c in [ka*a + kb*b + alpha_lo, ... + alpha_hi]
-  if (S.slab) {
-    const double inw = 1.0 / (double)nw, iu = P.inv_unit;
-    const double a1 = -(S.nc - S.nv0) * inw * iu, a2 = -(S.nm - S.nv0) * inw * iu;
-    K.f[F_KA] = (float)(-(double)nua * inw);
-    K.f[F_KB] = (float)(-(double)nva * inw);
-    K.f[F_ALO] = (float)(fmin(a1, a2) - P.slab_margin);
-    K.f[F_AHI] = (float)(fmax(a1, a2) + P.slab_margin);
-  } else {
-    K.f[F_KA] = K.f[F_KB] = K.f[F_ALO] = K.f[F_AHI] = 0.0f;
-  }
-  // bbox along (ua, va, w) by value selects (a branch per axis would let the compiler
-  // index the bbox arrays with w, which puts them in scratch memory)
-  const int x0 = S.g0[0], y0 = S.g0[1], z0 = S.g0[2];
-  const int x1 = S.g1[0], y1 = S.g1[1], z1 = S.g1[2];
-  K.i[I_G0U] = (w == 0) ? y0 : x0;
-  K.i[I_G1U] = (w == 0) ? y1 : x1;
-  K.i[I_G0V] = (w == 2) ? y0 : z0;
-  K.i[I_G1V] = (w == 2) ? y1 : z1;
-  K.i[I_G0W] = (w == 0) ? x0 : (w == 1 ? y0 : z0);
-  K.i[I_G1W] = (w == 0) ? x1 : (w == 1 ? y1 : z1);
-  K.i[I_WS] = w | (S.slab ? 4 : 0);
-  K.i[I_TRI] = (int)tri;
-}
 
 // The terms of a row of columns (fixed b) that do not depend on a: pb, the hoisted
 // plane's h1*pb, plane P's cc*pb, the plane test's term of pb and the slab's term of b.
@@ -492,12 +268,10 @@ struct ActArgs {
 // flagged bricks in Morton order (table entry = slot + 1) and lists them.
 struct TouchAction {
   static constexpr bool kTouch = true;
-  // columns of a row per item of the small tier, per unit: with more than one, an item
-  // walks its segment narrowed to the row's interval; atomic updates take one (the
-  // lanes of a wave then update neighbouring cells, whose atomics share cache lines)
-  __device__ static int seg_cols(const VoxParams&) { return 8; }
-  // one-column items of a unit laid out over its rows' intervals only (see k_vox_tile)
-  static constexpr bool kCompact = false;
+  // the same action for lanes in no order of their triangles (queued columns)
+  using Unordered = TouchAction;
+  // whether a direct walk narrows its rows to their intervals
+  __device__ static bool narrow(const VoxParams&) { return true; }
   uint32_t* table;
   uint64_t brick0;  // first brick of the unit's table segment
   __device__ static TouchAction make(const ActArgs& A, const VoxParams& P) {
@@ -530,12 +304,8 @@ typedef __attribute__((address_space(1))) uint32_t gword_t;
 template <bool kWide, bool kLaneOrder = true>
 struct MarkDenseT {
   static constexpr bool kTouch = false;
-  __device__ static int seg_cols(const VoxParams& P) {
-    if (!kWide) return 16;
-    if (kLaneOrder) return 1;  // the single-unit payload pass: its unit is wide
-    return P.wide ? 1 : 16;
-  }
-  static constexpr bool kCompact = kWide;
+  using Unordered = MarkDenseT<kWide, false>;
+  __device__ static bool narrow(const VoxParams& P) { return !kWide || (!kLaneOrder && !P.wide); }
   gword_t* table;
   gbyte_t* bytes;
   uint64_t base;  // code of the first voxel of the unit's first brick
@@ -585,8 +355,8 @@ using MarkDenseWideBatchAction = MarkDenseT<true, false>;
 
 struct MarkPoolAction {
   static constexpr bool kTouch = false;
-  __device__ static int seg_cols(const VoxParams&) { return 8; }
-  static constexpr bool kCompact = false;
+  using Unordered = MarkPoolAction;
+  __device__ static bool narrow(const VoxParams&) { return true; }
   const gword_t* table;
   gbyte_t* bytes;  // the slot pool
   ull* ctr;
@@ -625,8 +395,8 @@ struct MarkPoolAction {
 // Second payload pass: lowest triangle index per voxel rank.
 struct WinnerAction {
   static constexpr bool kTouch = false;
-  __device__ static int seg_cols(const VoxParams&) { return 1; }
-  static constexpr bool kCompact = false;
+  using Unordered = WinnerAction;
+  __device__ static bool narrow(const VoxParams&) { return false; }
   const uint32_t* table;
   const ull* pool;  // bit form of the bricks, written by the compaction
   const uint32_t* wprefix;
@@ -670,32 +440,40 @@ __device__ __forceinline__ uint32_t upper_index(const T* __restrict__ a, uint32_
   return lo;
 }
 
-// Small tier, persistent: blocks take tiles of tt <= kTileTris consecutive triangles of one
-// unit from a device work queue (tile_off[u] = first tile of unit u); tt is smaller for
-// passes with few triangles, so that their tiles still spread over the CUs. For a tile, each thread builds
-// its triangle's walk constants into LDS; a block scan lays out the (triangle, row
-// segment) items, a segment being Act::seg_cols neighbouring columns of one row; then the
-// threads share the items, so the work per lane is a few voxel tests regardless of
-// triangle size. Triangles with more than small_cols columns
-// (or non-slab triangles with more than small_cols * 8 tests) go to the column-parallel
-// tier. Triangles with at most direct_cols columns skip the item layout: their own
-// thread walks their columns from registers (the per-item lookup and constant loads
-// would cost more than the walk). Units the pass does not apply to (skip mask)
-// contribute no items.
-constexpr int kTile = 256;      // threads per block
-constexpr int kTileTris = 192;  // triangles per tile: 35 KB of walk constants in LDS, so
-                                // that four blocks fit a CU
-// Actions with kCompact (atomic payload marks, one column per item) lay out the items of a
-// triangle of at most kCompactRows rows and 255 columns per row over its rows' intervals
-// only (row_interval: the columns outside fail the projection test), 255 items at most;
-// the rows' first columns and item offsets take 32 bytes of LDS per triangle, so their
-// tiles hold kTileTrisCompact triangles (four blocks still fit a CU).
-constexpr int kCompactRows = 16;
-constexpr int kTileTrisCompact = 160;
+// Small tier, persistent: waves take tiles of tt <= 64 consecutive triangles of one unit from
+// device work queues (tile_off[u] = first tile of unit u); tt is smaller for passes with few
+// triangles, so that their tiles still spread over the chip. Lane l sets up triangle l of
+// the tile. A tile whose triangles all have at most direct_cols columns, of about as many
+// each, is walked from registers, a lane a triangle. Triangles with more than small_cols columns (or non-slab triangles with more
+// than small_cols * 8 tests) go to the column-parallel tier. Otherwise a tile is laid out in two
+// steps, each giving every lane of the wave one element whatever the triangles' shapes:
+//   * rows: 64 rows of the tile's triangles at a time; a lane finds its row's interval of
+//     columns, and the terms of its bounds that do not change along it (fast_row);
+//   * columns: the columns of these 64 rows, 64 at a time; a lane finds the run of voxels
+//     its column holds (fast_column) and marks it without testing them one by one.
+// A column whose run is not certain (a bound within its error of an integer: a few in a
+// thousand at 2048; most where faces lie on voxel planes) is queued, and the queue walked
+// with the reference's own tests once 64 are there. Units the pass does not apply to (skip mask) contribute nothing.
+//
+// Bound by vector instructions (binary meshes) or by the winner atomics (payload). Testing
+// every candidate voxel of a row segment per lane left 64% of the lanes of a rough mesh's waves
+// idle and took ~43 instructions a candidate: 64 mixed meshes 4.35 -> 2.75 ms, a 1.3M-triangle
+// rough sphere at 1024 987 -> 438 us, a 6M-triangle soup at 4096 in 8 partitions 1.71 -> 1.19
+// ms, the 2.1M-triangle terrain at 2048 (lanes walking their own triangles) 154 -> 141 us.
+// 128 registers and 40 KB of LDS a block keep four blocks on a CU: three cost 10%.
+constexpr int kTile = 256;     // threads per block
+constexpr int kTileWaves = kTile / kWave;
+constexpr int kTileTris = 64;  // triangles per tile: one per lane
+constexpr int kRowWords = 8;   // LDS words of a row
+constexpr int kTriQuads = (int)sizeof(FastTri) / 16;
+constexpr int kRowQuads = (int)(sizeof(FastTri) - sizeof(FastCol)) / 16;  // per-row part of a triangle
+constexpr int kQueueCap = 2 * kWave;  // uncertain columns waiting per wave
+constexpr uint32_t kColMask = (1u << 26) - 1u;  // columns of a triangle of the small tier, or of a job
 constexpr uint32_t kQueues = 8;        // tile queues per persistent launch
+constexpr uint32_t kTileRun = 16;      // neighbouring tiles in one queue
 constexpr uint32_t kQueueStride = 16;  // words between their counters (own cache lines)
 constexpr uint32_t kQueueWords = kQueues * kQueueStride;
-constexpr uint64_t kLargeWalkMax = 1u << 18;  // large triangles with stored walk constants
+constexpr uint64_t kLargeWalkMax = 1u << 18;  // large triangles with stored constants
 constexpr int kSkipDense = 1;   // units voxelized in a dense grid (touch pass)
 constexpr int kSkipBinary = 2;  // geometry-only units (payload winner pass)
 
@@ -703,241 +481,348 @@ __device__ __forceinline__ bool skipped(const VoxParams& P, int skip) {
   return ((skip & kSkipDense) && P.dense) || ((skip & kSkipBinary) && P.stride == 9);
 }
 
+// Per wave: the tile's triangles, the current rows, a 64-entry slot array and the queue of
+// uncertain columns (lane of the triangle << 26 | (j - row0) * (number of i) + i).
+struct WalkLds {
+  uint4 tri[kTileTris][kTriQuads];
+  uint4 row[kWave][kRowWords / 4];
+  uint32_t q[kQueueCap];
+  uint8_t slot[kWave];
+};
+
+// The element of lane's position k0 + lane among elements laid out by their start positions
+// (lane e holds element e's start, has = it is not empty): the last one that starts at or
+// before it. carry: the element the previous window ended in (0 before the first), as
+// index + 1.
+__device__ __forceinline__ uint32_t locate(uint8_t* slot, uint32_t start, bool has, uint32_t k0,
+                                           uint32_t& carry) {
+  const int lane = lane_id();
+  slot[lane] = (uint8_t)(lane == 0 ? carry : 0u);
+  wave_lds_sync();
+  if (has && start - k0 < (uint32_t)kWave) slot[start - k0] = (uint8_t)(lane + 1);
+  wave_lds_sync();
+  const uint32_t v = wave_incl_max(slot[lane]);
+  wave_lds_sync();  // (the next call clears the slots)
+  carry = (uint32_t)__builtin_amdgcn_readlane((int)v, kWave - 1);
+  return v - 1u;
+}
+
+// Up to 64 queued columns through the reference's tests: lane l's walk is K.
+template <typename Act>
+__device__ __forceinline__ void walk_queued(const VoxParams& P, const ActArgs& A, const Walk& K,
+                                            uint32_t row0, const uint32_t* q, uint32_t n) {
+  const uint32_t e = (uint32_t)lane_id() < n ? q[lane_id()] : 0u;
+  const int src = (int)(e >> 26);
+  Walk Q;  // the walk of lane src
+#pragma unroll
+  for (int f = 0; f < kWalkF; f++) Q.f[f] = __shfl(K.f[f], src, kWave);
+#pragma unroll
+  for (int f = 0; f < kWalkI; f++) Q.i[f] = __shfl(K.i[f], src, kWave);
+  if ((uint32_t)lane_id() >= n) return;
+  typename Act::Unordered act = Act::Unordered::make(A, P);
+  const uint32_t col = e & kColMask, na = (uint32_t)(Q.i[I_G1U] - Q.i[I_G0U] + 1);
+  const int a = Q.i[I_G0U] + (int)(col % na);
+  walk_row_span<false>(Q, P, Q.i[I_G0V] + (int)(row0 + col / na), a, a, act);
+  act.flush();
+}
+
+// Rows [row0, row0 + nrows) of the lanes' triangles (nall rows each; their walks K, their linear forms in
+// L.tri).
+template <typename Act>
+__device__ __forceinline__ void walk_rows(WalkLds& L, const VoxParams& P, const ActArgs& A,
+                                          const Walk& K, uint32_t nall, uint32_t nrows, uint32_t row0) {
+  uint32_t nq = 0;
+  const int lane = lane_id();
+  const uint32_t rend = wave_incl_scan<uint32_t>(nrows), rstart = rend - nrows;
+  const uint32_t R = (uint32_t)__builtin_amdgcn_readlane((int)rend, kWave - 1);
+  uint32_t tcarry = 0;
+  for (uint32_t r0 = 0; r0 < R; r0 += kWave) {
+    const uint32_t t = locate(L.slot, rstart, nrows != 0, r0, tcarry);
+    const uint32_t r = r0 + lane;
+    const int j = (int)(r - (uint32_t)__shfl((int)rstart, (int)t, kWave) + row0);
+    const int nb = __shfl((int)nall, (int)t, kWave);
+    uint32_t cnt = 0;
+    FastRow W;
+    if (r < R) {
+      FastTri F;
+      const uint4* src = L.tri[t];
+      uint4* dst = (uint4*)&F;
+#pragma unroll
+      for (int k = 0; k < kRowQuads; k++) dst[k] = src[k];
+      dst[kRowQuads + 2] = src[kRowQuads + 2];  // (the error)
+      fast_row(F, j, nb, W);
+      if (W.i1 >= W.i0) cnt = (uint32_t)(W.i1 - W.i0 + 1);
+      const int w = (int)(F.rf >> 8) & 3;
+      const uint32_t b = (F.rf >> 16) + (uint32_t)j;
+      const uint64_t mb = spread3_s(b) << (w == 2 ? 1 : 2);
+      // the row's columns are known by their position in the row: its end flags by the count
+      L.row[lane][1] = make_uint4(__float_as_uint(W.s_lo), (uint32_t)mb, (uint32_t)(mb >> 32),
+                                  (uint32_t)j | (cnt << 16));
+      L.row[lane][0] = make_uint4(0u, (uint32_t)W.i0 | (t << 16) | (W.first_unsure ? 1u << 24 : 0u) |
+                                          (W.last_unsure ? 1u << 25 : 0u) | (W.all ? 1u << 26 : 0u),
+                                  __float_as_uint(W.p_lo), __float_as_uint(W.p_hi));
+    }
+    const uint32_t cend = wave_incl_scan<uint32_t>(cnt), cstart = cend - cnt;
+    const uint32_t C = (uint32_t)__builtin_amdgcn_readlane((int)cend, kWave - 1);
+    L.row[lane][0].x = cstart;
+    uint32_t ccarry = 0;
+    Act act = Act::make(A, P);
+    for (uint32_t k0 = 0; k0 < C; k0 += kWave) {
+      const uint32_t rr = locate(L.slot, cstart, cnt != 0, k0, ccarry);  // (orders the row stores)
+      const uint32_t k = k0 + lane;
+      bool push = false;
+      uint32_t e = 0;
+      if (k < C) {
+        const uint4 ra = L.row[rr][0], rb = L.row[rr][1];
+        const uint32_t t = (ra.y >> 16) & 0xFFu;
+        FastCol F;
+        const uint4* src = &L.tri[t][kRowQuads];
+        uint4* dst = (uint4*)&F;
+#pragma unroll
+        for (int q = 0; q < (int)sizeof(FastCol) / 16; q++) dst[q] = src[q];
+        const uint32_t at = k - ra.x;
+        const int i = (int)((ra.y & 0xFFFFu) + at);
+        const int w = (int)(F.qf >> 8) & 3;
+        const uint32_t a = (F.qf >> 16) + (uint32_t)i;
+        int lo, hi;
+        bool sure = fast_column(F, __uint_as_float(ra.z), __uint_as_float(ra.w),
+                                __uint_as_float(rb.x), i, lo, hi);
+        sure = sure && !((ra.y & (1u << 24)) && at == 0) &&
+               !((ra.y & (1u << 25)) && at + 1 == (rb.w >> 16)) && !(ra.y & (1u << 26));
+        const bool careful = F.qf & kFastCareful;
+        if (lo <= hi || careful) {
+          const uint64_t mb = ((uint64_t)rb.z << 32) | rb.y;
+          const int c0 = (int)(F.ck & 0xFFFFu);
+          if (Act::kTouch ? careful : !sure) {
+            push = true;
+            const uint32_t na = L.tri[t][kRowQuads - 1].w & 0xFFFFu;
+            e = (t << 26) | (((rb.w & 0xFFFFu) - row0) * na + (uint32_t)i);
+          } else if constexpr (Act::kTouch) {
+            const uint32_t b = (uint32_t)compact3(mb >> (w == 2 ? 1 : 2));
+            const uint64_t bb = (spread3(a >> 4) << (w == 0 ? 1 : 0)) |
+                                (spread3(b >> 4) << (w == 2 ? 1 : 2));
+            for (int cb = (c0 + lo) >> 4; cb <= (c0 + hi) >> 4; cb++)
+              act.touch(bb | (spread3((uint32_t)cb) << w));
+          } else {
+            const uint64_t cbase = mb + (spread3_s(a) << (w == 0 ? 1 : 0));
+            uint64_t mc = spread3_s((uint32_t)(c0 + lo)) << w;
+            for (int c = lo; c <= hi; c++, mc = morton_step(mc, w)) act.add(cbase + mc, F.tri);
+          }
+        }
+      }
+      const uint64_t pm = __ballot(push);
+      if (pm) {  // uniform
+        if (push) L.q[nq + (uint32_t)__popcll(pm & ((1ull << lane) - 1ull))] = e;
+        nq += (uint32_t)__popcll(pm);
+        wave_lds_sync();
+        if (nq >= (uint32_t)kWave) {
+          walk_queued<Act>(P, A, K, row0, L.q + (nq - kWave), kWave);
+          nq -= kWave;
+          wave_lds_sync();
+        }
+      }
+    }
+    act.flush();
+    wave_lds_sync();  // the next rows overwrite these
+  }
+  if (nq) walk_queued<Act>(P, A, K, row0, L.q, nq);
+  wave_lds_sync();
+}
+
+// The triangles of the large tier: unit, triangle, rows per job, the linear form and walk of
+// the first walk_cap of them (the others are set up again by each of their jobs), and the jobs
+// after each triangle's first one (triangle's index here, first row).
+constexpr uint32_t kLargeJobs = 1u << 20;  // places for those
+constexpr uint32_t kJobCols = 1024;        // columns of a job, roughly
+constexpr int kLargeQuads = kTriQuads + kWalkWords / 4;
+static_assert(kWalkWords % 4 == 0 && sizeof(Walk) == kWalkWords * 4, "walk words");
+struct LargeList {
+  uint32_t* unit;
+  uint32_t* tri;
+  uint32_t* rows;
+  uint2* jobs;
+  uint4* walk;
+  uint64_t walk_cap;
+};
+// Rows per job of a triangle with nu x nv columns, its further jobs appended; with no room
+// for them (kAllRows) its one job takes all rows, that many at a time.
+constexpr uint32_t kAllRows = 1u << 31;
+__device__ __forceinline__ uint32_t large_jobs(const LargeList& B, ull* ctr, uint32_t idx,
+                                               uint32_t nu, uint32_t nv) {
+  const uint32_t rows = max(1u, min((uint32_t)kWave, kJobCols / nu));
+  const uint32_t more = (nv + rows - 1) / rows - 1;
+  if (!more) return rows;
+  const ull at = atomicAdd(&ctr[kCtrLargeJobs], (ull)more);
+  const bool fits = at + more <= kLargeJobs;
+  for (uint32_t q = 0; q < more && at + q < kLargeJobs; q++)
+    B.jobs[at + q] = make_uint2(fits ? idx : 0xFFFFFFFFu, (q + 1) * rows);
+  return fits ? rows : rows | kAllRows;
+}
+
 template <typename Act>
 __global__ __launch_bounds__(kTile, 4) void k_vox_tile(const VoxParams* __restrict__ units,
-                                                    uint32_t n_units,
-                                                    const uint32_t* __restrict__ tile_off,
-                                                    ActArgs A, ull* queue,
-                                                    uint32_t* large_unit, uint32_t* large_tri,
-                                                    uint32_t* large_cols, uint32_t* large_walk,
-                                                    uint32_t walk_cap, uint32_t tt, int collect,
-                                                    int skip) {
-  constexpr bool kCompact = Act::kCompact;
-  constexpr int kTT = kCompact ? kTileTrisCompact : kTileTris;
-  __shared__ uint32_t sk[kWalkWords][kTT];
-  __shared__ uint32_t soff[kTT + 1];
-  __shared__ uint32_t wsum[kTile / kWave];
-  __shared__ uint32_t s_tile;
-  // compact layout, per triangle: items before each row, each row's first column - g0u,
-  // and whether the triangle uses the layout
-  __shared__ uint8_t s_rpre[kCompact ? kTT : 1][kCompactRows];
-  __shared__ uint8_t s_ri0[kCompact ? kTT : 1][kCompactRows];
-  __shared__ uint8_t s_cmp[kCompact ? kTT : 1];
-  fill_spread_table();  // read after the first barrier of the tile loop
+                                                       uint32_t n_units,
+                                                       const uint32_t* __restrict__ tile_off,
+                                                       ActArgs A, ull* queue, LargeList B,
+                                                       uint32_t tt, int collect, int skip) {
+  __shared__ WalkLds s_walk[kTileWaves];
+  __shared__ uint32_t s_empty[kQueues];  // ranges found empty
+  if (threadIdx.x < kQueues) s_empty[threadIdx.x] = 0;
+  fill_spread_table();
+  __syncthreads();  // the waves part here
+  WalkLds& L = s_walk[threadIdx.x / kWave];
   ull* ctr = A.ctr;
-  const uint32_t total_tiles = tile_off[n_units];
-  const uint32_t tid = threadIdx.x;
-  // kQueues interleaved tile classes (tile % kQueues), each with its own counter: one
-  // counter's atomics serialize (~14 ns each), which bounds a single queue at ~70 M
-  // tiles/s. A block starts on class blockIdx % kQueues and moves on when it is empty.
-  uint32_t cls = blockIdx.x % kQueues, tried = 0;
+  const int lane = lane_id();
+  const uint32_t total = tile_off[n_units];
+  // Runs of kTileRun tiles are dealt to kQueues classes (one per XCD: blocks are dealt to
+  // them in turn), each with its own counter in its own cache line: a run's tiles, neighbours
+  // in space, mark lines of one L2, and the classes hold about the same work. One counter's
+  // returning atomics serialize (~14 ns each), those that find a class empty included, so a
+  // wave looks into one other class only, and a block's waves tell each other which classes
+  // are empty. A pass with no more tiles than waves needs no counter.
+  const bool one_each = total <= gridDim.x * kTileWaves;
+  uint32_t cls = blockIdx.x % kQueues;
+  uint32_t next = one_each ? blockIdx.x * kTileWaves + threadIdx.x / kWave : total;
   for (;;) {
-    if (tid == 0) {
-      uint32_t tl = total_tiles;
-      while (tried < kQueues) {
-        const uint32_t k = (uint32_t)atomicAdd(queue + kQueueStride * cls, 1ull);
-        const uint32_t cand = cls + kQueues * k;
-        if (cand < total_tiles) {
-          tl = cand;
-          break;
+    if (!one_each) {
+      for (uint32_t tried = 0; tried < 2; tried++) {
+        if (!*(volatile uint32_t*)&s_empty[cls]) {
+          uint32_t k = 0;
+          if (lane == 0) k = (uint32_t)atomicAdd(queue + kQueueStride * cls, 1ull);
+          k = (uint32_t)__builtin_amdgcn_readfirstlane((int)k);
+          next = (k / kTileRun * kQueues + cls) * kTileRun + k % kTileRun;
+          if (next < total) break;
+          *(volatile uint32_t*)&s_empty[cls] = 1u;
         }
         cls = (cls + 1) % kQueues;
-        tried++;
       }
-      s_tile = tl;
     }
-    __syncthreads();
-    // the block's tile in a scalar register: the unit search and the unit's parameters
-    // then run on scalar loads
-    const uint32_t tile = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_tile);
-    if (tile >= total_tiles) break;
+    // in a scalar register: the unit search and the unit's parameters run on scalar loads
+    const uint32_t tile = (uint32_t)__builtin_amdgcn_readfirstlane((int)next);
+    if (tile >= total) return;
+    next = total;
     const uint32_t u = upper_index<uint32_t>(tile_off, n_units + 1, tile);
     const VoxParams P = units[u];
-    const bool active = !skipped(P, skip);
-    const uint32_t i = (tile - tile_off[u]) * tt + tid;
-    uint32_t items = 0;
-    if (active && tid < tt && i < P.n) {
+    if (skipped(P, skip)) continue;
+    const uint32_t i = (tile - tile_off[u]) * tt + lane;
+    Walk K;
+    uint32_t ncols = 0, nu = 0, nv = 0;  // columns of a triangle of this tier; its sides
+    bool large = false;
+    if ((uint32_t)lane < tt && i < P.n) {
       const uint32_t t = P.list ? P.list[i] : i;
       Setup S;
       setup_tri(P.tris + (uint64_t)t * P.stride, P, S);
-      Walk K;
       make_walk(S, P, t, K);
-      const uint64_t ncols = K.columns();
+      const uint64_t nc = K.columns();
       const uint64_t lim = (uint64_t)P.small_cols;
-      if (K.slab() ? (ncols > lim) : (K.work() > lim * 8)) {
-        if (collect) {
-          const ull idx = atomicAdd(&ctr[kCtrLargeCount], 1ull);
-          large_unit[idx] = u;
-          large_tri[idx] = t;
-          large_cols[idx] = (uint32_t)ncols;
-          if (idx < walk_cap) {  // its walk constants, for the column threads
-            uint32_t* dst = large_walk + idx * kWalkWords;
+      nu = (uint32_t)(K.i[I_G1U] - K.i[I_G0U] + 1);
+      nv = (uint32_t)(K.i[I_G1V] - K.i[I_G0V] + 1);
+      large = (K.slab() ? (nc > lim) : (K.work() > lim * 8)) || nc > (uint64_t)kColMask;
+      if (!large) ncols = (uint32_t)nc;
+    }
+    // A lane walking its own triangle takes ~100 instructions a column, in as many steps as
+    // the tile's largest triangle has columns; the rows and columns of the whole tile take
+    // ~1200 and ~4 a column (headline, 64 triangles of 9.4 columns: 141 us by lanes, 268 by
+    // columns; 16-triangle tiles of the same, 178,802 triangles at 1024: 56 and 55).
+    uint32_t all = wave_incl_scan<uint32_t>(min(ncols, 0xFFFFu));
+    all = (uint32_t)__builtin_amdgcn_readlane((int)all, kWave - 1);
+    uint32_t most = wave_incl_max(ncols);
+    most = (uint32_t)__builtin_amdgcn_readlane((int)most, kWave - 1);
+    const bool direct = most <= (uint32_t)P.direct_cols && most * 100u <= 1200u + all * 4u;
+    uint32_t rows = 0;
+    if ((large && collect) || (ncols && !direct)) {
+      FastTri F;
+      make_fast(K, P, F);
+      const uint4* src = (const uint4*)&F;
+      if (!large) {
 #pragma unroll
-            for (int f = 0; f < kWalkF; f++) dst[f] = __float_as_uint(K.f[f]);
+        for (int k = 0; k < kTriQuads; k++) L.tri[lane][k] = src[k];
+        rows = nv;
+      } else {
+        const ull idx = atomicAdd(&ctr[kCtrLargeCount], 1ull);
+        B.unit[idx] = u;
+        B.tri[idx] = (uint32_t)K.i[I_TRI];
+        B.rows[idx] = large_jobs(B, ctr, (uint32_t)idx, nu, nv);
+        if (idx < B.walk_cap) {
+          uint4* dst = B.walk + idx * kLargeQuads;
 #pragma unroll
-            for (int f = 0; f < kWalkI; f++) dst[kWalkF + f] = (uint32_t)K.i[f];
-          }
+          for (int k = 0; k < kTriQuads; k++) dst[k] = src[k];
+          const uint4* wk = (const uint4*)&K;
+#pragma unroll
+          for (int k = 0; k < kWalkWords / 4; k++) dst[kTriQuads + k] = wk[k];
         }
-      } else if (ncols <= (uint64_t)P.direct_cols) {
-        // few columns: this thread walks them now, from registers
+      }
+    }
+    if (direct) {
+      if (ncols) {
         Act act = Act::make(A, P);
-        walk_all_columns(K, P, act, Act::seg_cols(P) > 1);
+        walk_all_columns(K, P, act, Act::narrow(P));
         act.flush();
-      } else {
-        // items: the rows' segments of seg columns
-        const uint32_t seg = (uint32_t)Act::seg_cols(P);
-        const uint32_t eu = (uint32_t)(K.i[I_G1U] - K.i[I_G0U] + 1);
-        const uint32_t nrows = (uint32_t)(K.i[I_G1V] - K.i[I_G0V] + 1);
-        items = nrows * ((eu + seg - 1) / seg);
-        if constexpr (kCompact) {
-          // one-column items over the rows' intervals only
-          bool cmp = false;
-          if (seg == 1 && nrows <= (uint32_t)kCompactRows && eu <= 255u) {
-            uint32_t cum = 0;
-            for (uint32_t r = 0; r < nrows; r++) {
-              const ColRow R = col_row(K, P, K.i[I_G0V] + (int)r);
-              int i0, i1;
-              row_interval(K, R, P.unit, i0, i1);
-              s_rpre[tid][r] = (uint8_t)min(cum, 255u);
-              s_ri0[tid][r] = (uint8_t)min(i0 - K.i[I_G0U], 255);
-              if (i1 >= i0) cum += (uint32_t)(i1 - i0 + 1);
-            }
-            if (cum <= 255u) {
-              cmp = true;
-              items = cum;
-            }
-          }
-          s_cmp[tid] = cmp ? 1 : 0;
-        }
-#pragma unroll
-        for (int f = 0; f < kWalkF; f++) sk[f][tid] = __float_as_uint(K.f[f]);
-#pragma unroll
-        for (int f = 0; f < kWalkI; f++) sk[kWalkF + f][tid] = (uint32_t)K.i[f];
       }
+      continue;
     }
-    uint32_t total;
-    const uint32_t inc = block_incl_scan<uint32_t, kTile>(items, wsum, total);
-    if (tid < tt) soff[tid] = inc - items;
-    if (tid == tt - 1) soff[tt] = total;
-    __syncthreads();
-    Act act = Act::make(A, P);
-    for (uint32_t it = tid; it < total; it += kTile) {
-      // owner: last j with soff[j] <= it (triangles without items have empty ranges)
-      const uint32_t lo = upper_index<uint32_t>(soff, tt, it);
-      Walk K;
-#pragma unroll
-      for (int f = 0; f < kWalkF; f++) K.f[f] = __uint_as_float(sk[f][lo]);
-#pragma unroll
-      for (int f = 0; f < kWalkI; f++) K.i[f] = (int)sk[kWalkF + f][lo];
-      const uint32_t local = it - soff[lo];
-      const uint32_t eu = (uint32_t)(K.i[I_G1U] - K.i[I_G0U] + 1);
-      const int seg = Act::seg_cols(P);  // the tile's unit: uniform
-      if (kCompact && s_cmp[kCompact ? lo : 0]) {
-        // row: the last r with s_rpre[r] <= local among the triangle's rows (an empty
-        // row shares its offset with the next one, which is the one taken)
-        const uint32_t nrows = (uint32_t)(K.i[I_G1V] - K.i[I_G0V] + 1);
-        uint32_t r0 = 0, r1 = nrows - 1;
-        while (r0 < r1) {
-          const uint32_t mid = (r0 + r1 + 1) >> 1;
-          if (s_rpre[lo][mid] <= local)
-            r0 = mid;
-          else
-            r1 = mid - 1;
-        }
-        const int a = K.i[I_G0U] + (int)s_ri0[lo][r0] + (int)(local - s_rpre[lo][r0]);
-        walk_row_span<false>(K, P, K.i[I_G0V] + (int)r0, a, a, act);
-      } else if (seg > 1) {
-        const uint32_t nseg = (eu + seg - 1) / seg;
-        const int a = K.i[I_G0U] + (int)(local % nseg) * seg;
-        const int b = K.i[I_G0V] + (int)(local / nseg);
-        walk_row_span<true>(K, P, b, a, min(a + seg - 1, K.i[I_G1U]), act);
-      } else {
-        const int a = K.i[I_G0U] + (int)(local % eu);
-        const int b = K.i[I_G0V] + (int)(local / eu);
-        walk_row_span<false>(K, P, b, a, a, act);
-      }
+    if (__ballot(rows != 0)) {
+      wave_lds_sync();
+      walk_rows<Act>(L, P, A, K, nv, rows, 0u);
     }
-    act.flush();
-    __syncthreads();  // LDS (setups, offsets, s_tile) is reused by the next tile
   }
 }
 
-// Column-parallel tier: one thread per column of the deferred triangles; the counts live
-// on the device (ctr[kCtrLargeCount] triangles, ctr[kCtrCols] columns), the grid strides.
-// walk constants stored as 44 words (kWalkF floats, then kWalkI ints)
-__device__ __forceinline__ void load_walk(const uint32_t* __restrict__ src, Walk& K) {
-#pragma unroll
-  for (int f = 0; f < kWalkF; f++) K.f[f] = __uint_as_float(src[f]);
-#pragma unroll
-  for (int f = 0; f < kWalkI; f++) K.i[f] = (int)src[kWalkF + f];
-}
-
+// Column-parallel tier: a wave per job, a job being some rows of one deferred triangle (at most
+// 64, about kJobCols columns), laid out over the wave's lanes as in the small tier; the counts
+// live on the device, the grid strides. Triangle idx has its first job at idx, its others at
+// n_large + (their place in B.jobs). (A thread per bbox column took 219 us on 20,480 triangles
+// of ~2,200 columns, after a launch that scanned the column counts; in rows 160.)
 template <typename Act>
-__global__ __launch_bounds__(256) void k_vox_large(const VoxParams* __restrict__ units, ActArgs A,
-                                                   const uint32_t* __restrict__ large_unit,
-                                                   const uint32_t* __restrict__ large_tri,
-                                                   const uint64_t* __restrict__ large_off,
-                                                   const uint32_t* __restrict__ large_walk,
-                                                   uint32_t walk_cap, int skip) {
+__global__ __launch_bounds__(kTile, 3) void k_vox_large(const VoxParams* __restrict__ units,
+                                                        ActArgs A, LargeList B, int skip) {
+  __shared__ WalkLds s_walk[kTileWaves];
+  const ull* ctr = A.ctr;
+  const uint64_t n_large = ctr[kCtrLargeCount];
+  const uint64_t total = n_large + min(ctr[kCtrLargeJobs], (ull)kLargeJobs);
+  if ((uint64_t)blockIdx.x * kTileWaves >= total) return;  // uniform per block
   fill_spread_table();
   __syncthreads();
-  __shared__ uint32_t s_j0;
-  const ull* ctr = A.ctr;
-  const uint32_t n_large = (uint32_t)ctr[kCtrLargeCount];
-  const uint64_t total = ctr[kCtrCols];
-  // each block walks one contiguous range of the columns, 256 at a time: the owner of its
-  // first column comes from one binary search, and a thread's owner only moves forward
-  // (a triangle here has more than small_cols columns), one offset compare per step
-  const uint64_t per = (total + gridDim.x - 1) / gridDim.x;
-  const uint64_t beg = (uint64_t)blockIdx.x * per;
-  const uint64_t end = min(total, beg + per);
-  if (beg >= end) return;  // uniform per block
-  if (threadIdx.x == 0) s_j0 = upper_index<uint64_t>(large_off, n_large, beg);
-  __syncthreads();
-  uint32_t j = s_j0;
-  for (uint64_t g = beg + threadIdx.x; g < end; g += blockDim.x) {
-    while (j + 1 < n_large && large_off[j + 1] <= g) j++;
-    // the lanes of a wave nearly always share their triangle: then its unit parameters
-    // and walk constants come in with scalar loads (one per 16 words) instead of some 60
-    // vector loads per column, which bound this kernel
-    // (a wave that straddles two triangles sets its lanes' walks up again)
-    const uint32_t jf = (uint32_t)__builtin_amdgcn_readfirstlane((int)j);
-    VoxParams P;
-    Walk K;
-    uint32_t t;
-    uint64_t local;
-    bool stored = false;
-    if (__all(j == jf)) {
-      P = units[large_unit[jf]];
-      t = large_tri[jf];
-      local = g - large_off[jf];
-      if (jf < walk_cap) {
-        load_walk(large_walk + (uint64_t)jf * kWalkWords, K);
-        stored = true;
-      }
-    } else {
-      P = units[large_unit[j]];
-      t = large_tri[j];
-      local = g - large_off[j];
+  WalkLds& L = s_walk[threadIdx.x / kWave];
+  const int lane = lane_id();
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(
+      (int)(blockIdx.x * kTileWaves + threadIdx.x / kWave));
+  for (uint64_t g = wave; g < total; g += (uint64_t)gridDim.x * kTileWaves) {
+    uint32_t idx = (uint32_t)g, row0 = 0;
+    if (g >= n_large) {
+      const uint2 e = B.jobs[g - n_large];
+      idx = e.x;
+      row0 = e.y;
+      if (idx == 0xFFFFFFFFu) continue;  // a place left empty
     }
+    const VoxParams P = units[B.unit[idx]];
     if (skipped(P, skip)) continue;
-    if (!stored) {
-      Setup S;
-      setup_tri(P.tris + (uint64_t)t * P.stride, P, S);
-      make_walk(S, P, t, K);
-    }
-    const uint32_t eu = (uint32_t)(K.i[I_G1U] - K.i[I_G0U] + 1);
-    int a, b;
-    if (local <= 0xFFFFFFFFull) {  // 32-bit division (a 64-bit one is a long routine)
-      a = K.i[I_G0U] + (int)((uint32_t)local % eu);
-      b = K.i[I_G0V] + (int)((uint32_t)local / eu);
+    Walk K;  // (the same in every lane)
+    if (idx < B.walk_cap) {
+      const uint4* src = B.walk + (uint64_t)idx * kLargeQuads;
+      if (lane < kTriQuads) L.tri[0][lane] = src[lane];
+      uint4* wk = (uint4*)&K;
+#pragma unroll
+      for (int k = 0; k < kWalkWords / 4; k++) wk[k] = src[kTriQuads + k];
     } else {
-      a = K.i[I_G0U] + (int)(local % eu);
-      b = K.i[I_G0V] + (int)(local / eu);
+      Setup S;
+      setup_tri(P.tris + (uint64_t)B.tri[idx] * P.stride, P, S);
+      make_walk(S, P, B.tri[idx], K);
+      FastTri F;
+      make_fast(K, P, F);
+      const uint4* src = (const uint4*)&F;
+      if (lane == 0) {
+#pragma unroll
+        for (int k = 0; k < kTriQuads; k++) L.tri[0][k] = src[k];
+      }
     }
-    Act act = Act::make(A, P);
-    walk_row_span<false>(K, P, b, a, a, act);
-    act.flush();
+    wave_lds_sync();
+    const uint32_t nb = (uint32_t)(K.i[I_G1V] - K.i[I_G0V] + 1);
+    const uint32_t rows = B.rows[idx] & ~kAllRows;
+    do {
+      walk_rows<Act>(L, P, A, K, nb, lane == 0 ? min(rows, nb - row0) : 0u, row0);
+      row0 += rows;
+    } while ((B.rows[idx] & kAllRows) && row0 < nb);
   }
 }
 
@@ -1129,10 +1014,6 @@ struct BrickOffStore {
     bvoff[i] = s0 + (ex & kVoxMask);
     if (last) *total = (ull)(ex + v);
   }
-};
-struct ColLoad {
-  const uint32_t* a;
-  __device__ uint64_t operator()(uint64_t i) const { return a[i]; }
 };
 
 // The brick stream entry of every non-empty flagged brick and, with kCodes, for payload
@@ -1713,29 +1594,30 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
   std::vector<uint64_t> ubase(nu + 1);
   std::vector<uint32_t> toff(nu + 1);
   uint64_t ntab = 0, ntiles = 0, ntri = 0;
-  // triangles per tile: kTileTris once the pass has about four tiles of them per block of
-  // the persistent grid, else fewer (a multiple of 32, at least 32)
-  // (passes with payload units: kTileTrisCompact, the tile of the compact item layout)
+  // triangles per tile: kTileTris once the pass has about four tiles of them per wave of the
+  // persistent grid, else fewer; up to 16 a wave, one tile for each wave
   uint32_t tt = (uint32_t)kTileTris;
   int small_cols = c.tune.small_cols;
   {
     uint64_t all = 0;
-    bool any_payload_unit = false;
-    for (uint32_t u = 0; u < nu; u++) {
-      all += units[u].n;
-      any_payload_unit |= units[u].stride == 21;
-    }
-    const uint64_t cap = any_payload_unit ? kTileTrisCompact : kTileTris;
+    for (uint32_t u = 0; u < nu; u++) all += units[u].n;
     const uint64_t blocks = (uint64_t)std::max(1, c.tune.tile_blocks);
-    const uint64_t want = all / (4 * blocks);
-    tt = (uint32_t)std::min<uint64_t>(cap, std::max<uint64_t>(32, (want + 31) / 32 * 32));
+    const uint64_t waves = kTileWaves * blocks;
+    if (all <= 16 * waves) {
+      tt = (uint32_t)std::max<uint64_t>(1, (all + waves - 1) / waves);
+      // (a wave has few triangles: it keeps those of four times as many columns, which saves
+      // their trip through the large tier's list; 20,480 triangles at 2048: 137 + 161 us in
+      // the two tiers, 138 in this one)
+      small_cols = (int)std::max<int64_t>(small_cols, std::min<int64_t>(4ll * small_cols, 1 << 16));
+    } else
+      tt = (uint32_t)std::min<uint64_t>(kTileTris, (all / (4 * waves) + 7) / 8 * 8);
     // A pass of one mesh with 16 or more tiles per block of the persistent grid has the
     // parallelism to walk triangles of up to 16 x small_cols columns in the small tier (rows
     // narrowed to their intervals, a triangle's segments shared by its block's threads),
     // which is faster than the large tier's thread per bbox column (the soup of 5x10^7
     // triangles at 8192, 8 partitions: 68.6 -> 61.1 ms per step). Batches keep their
     // autotuned threshold.
-    if (!batch && all >= 16 * blocks * tt)
+    if (!batch && all >= 16 * blocks * 192)
       small_cols = std::max(small_cols, (int)std::min<int64_t>(16ll * small_cols, 1 << 16));
   }
   for (uint32_t u = 0; u < nu; u++) {
@@ -1845,17 +1727,19 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
   ull* pool_words = dense ? c.bwords.as<ull>() + nb0 * kBrickWords : c.pool.as<ull>();
   SVO_TRY(ensure(c.large_unit, ntri * 4));
   SVO_TRY(ensure(c.large_tri, ntri * 4));
-  SVO_TRY(ensure(c.large_cols, ntri * 4));
-  SVO_TRY(ensure(c.large_off, ntri * 8 + 8));
-  // walk constants of the first kLargeWalkMax large triangles of a pass (the others are
-  // set up again by each of their column threads)
-  const uint32_t walk_cap = (uint32_t)std::min<uint64_t>(ntri, kLargeWalkMax);
-  SVO_TRY(ensure(c.large_walk, (size_t)walk_cap * kWalkWords * 4 + 4));
+  SVO_TRY(ensure(c.large_rows, ntri * 4));
+  SVO_TRY(ensure(c.large_jobs, (size_t)kLargeJobs * sizeof(uint2)));
+  const uint64_t walk_cap = std::min<uint64_t>(ntri, kLargeWalkMax);
+  SVO_TRY(ensure(c.large_walk, (size_t)walk_cap * kLargeQuads * sizeof(uint4)));
   SVO_TRY(ensure(c.occ_list, ntab * 4));
-  SVO_TRY(ensure_scan_scratch(c, std::max<uint64_t>(ntri, ntab), 8));
+  SVO_TRY(ensure_scan_scratch(c, ntab, 8));
   ull* ctr = c.counters.as<ull>();
   ull hc[kNumCounters];
-  const unsigned tile_grid = (unsigned)std::min<uint64_t>(ntiles, c.tune.tile_blocks);
+  // (one payload mesh: half the waves, whose winner atomics meet on the same cells less often;
+  // 320,000 triangles at 512: mark 73 -> 67 us)
+  const unsigned tile_grid = (unsigned)std::min<uint64_t>(
+      (ntiles + kTileWaves - 1) / kTileWaves,
+      std::max(1, nu == 1 && !geometry_only ? c.tune.tile_blocks / 2 : c.tune.tile_blocks));
   const unsigned large_grid = (unsigned)c.tune.large_blocks;
   auto brick_grid = [&](uint64_t bricks) {
     return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((bricks * kWave + 255) / 256, 8192));
@@ -1871,17 +1755,14 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     A.pool_cap = c.pool_cap;
     return A;
   };
-  uint32_t* l_unit = c.large_unit.as<uint32_t>();
-  uint32_t* l_tri = c.large_tri.as<uint32_t>();
-  uint32_t* l_cols = c.large_cols.as<uint32_t>();
-  uint64_t* l_off = c.large_off.as<uint64_t>();
-  uint32_t* l_walk = c.large_walk.as<uint32_t>();
+  const LargeList large{c.large_unit.as<uint32_t>(), c.large_tri.as<uint32_t>(),
+                        c.large_rows.as<uint32_t>(), c.large_jobs.as<uint2>(),
+                        c.large_walk.as<uint4>(),    walk_cap};
   auto tile_pass = [&](auto tag, const char* name, ull* queue, int collect, int skip) {
     using Act = decltype(tag);
     ktimer_begin(c, name);
     SVO_LAUNCH((k_vox_tile<Act>), dim3(tile_grid), dim3(kTile), 0, c.stream, d_units, nu,
-                       d_toff, args(), queue, l_unit, l_tri, l_cols, l_walk, walk_cap, tt,
-                       collect, skip);
+                       d_toff, args(), queue, large, tt, collect, skip);
     ktimer_end(c);
     return hipGetLastError();
   };
@@ -1889,15 +1770,13 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     using Act = decltype(tag);
     ktimer_begin(c, name);
     SVO_LAUNCH((k_vox_large<Act>), dim3(large_grid), dim3(256), 0, c.stream, d_units,
-                       args(), l_unit, l_tri, l_off, l_walk, walk_cap, skip);
+                       args(), large, skip);
     ktimer_end(c);
     return hipGetLastError();
   };
-  // single-pass scans, each with its own zeroed status words: large-triangle columns,
-  // flagged bricks, brick counts (the last only while its packed prefixes stay below 2^62:
+  // single-pass scans, each with its own zeroed status words: flagged bricks, brick counts (the last only while its packed prefixes stay below 2^62:
   // at most bricks * (2^kNonEmptyShift + 4096))
-  const uint64_t w_col = scan_single_words(ntri), w_occ = scan_single_words(ntab);
-  ull* st_col = nullptr;
+  const uint64_t w_occ = scan_single_words(ntab);
   ull* st_occ = nullptr;
   ull* st_bc = nullptr;
   ull* queues = nullptr;  // 3 x kQueueWords: the tile queues of the mark/touch, second and winner passes
@@ -1916,15 +1795,14 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     const uint64_t w_bc = bc_single ? scan_single_words(bc_bound) : 0;
     SVO_TRY(ensure(c.bcount, bc_bound * 8 + 8));
     // status words of the scans, then the tile queues of the three tile passes
-    SVO_TRY(ensure(c.scan_status, (w_col + w_occ + w_bc + 3 * kQueueWords) * 8));
-    st_col = c.scan_status.as<ull>();
-    st_occ = st_col + w_col;
+    SVO_TRY(ensure(c.scan_status, (w_occ + w_bc + 3 * kQueueWords) * 8));
+    st_occ = c.scan_status.as<ull>();
     st_bc = st_occ + w_occ;
     queues = st_bc + w_bc;
     // the pass's kernels up to its read-back: one graph segment
     SVO_TRY(run_segment(c, [&]() -> hipError_t {
       {  // pass counters, scan status words and tile queues
-        const uint64_t ns = w_col + w_occ + w_bc + 3 * kQueueWords;
+        const uint64_t ns = w_occ + w_bc + 3 * kQueueWords;
         SVO_LAUNCH(k_zero2_u64, dim3(fill_grid(kCtrPassClear + ns)), dim3(256), 0,
                            c.stream, (uint64_t*)ctr, (uint64_t)kCtrPassClear,
                            c.scan_status.as<uint64_t>(), ns);
@@ -1942,10 +1820,6 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
         SVO_TRY(tile_pass(MarkDenseWideBatchAction{}, "vox_small_mark", queues, 1, 0));
       else
         SVO_TRY(tile_pass(TouchAction{}, "vox_small_touch", queues, 1, 0));
-      SVO_TRY((scan_single<uint64_t>(ColLoad{l_cols},
-                                     CountStore{l_off, ctr + kCtrCols},
-                                     ntri, st_col, ctr + kCtrError, c.stream,
-                                     ctr + kCtrLargeCount)));
       if (dense) {
         if (geometry_only)
           SVO_TRY(large_pass(MarkDenseAction{}, "vox_large_mark", 0));
