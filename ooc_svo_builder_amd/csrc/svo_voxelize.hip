@@ -1419,6 +1419,8 @@ hipError_t read_back(Context& c, const ReadReq* reqs, int n) {
     c.hread_cap = 0;
     const size_t cap = std::max<size_t>(total, 1u << 20);
     SVO_TRY(hipHostMalloc(&c.hread, cap, hipHostMallocDefault));
+    // memory freed by another context may hold its last flag: a value this one will wait for
+    memset(c.hread, 0, 256);
     c.hread_cap = cap;
   }
   const size_t base = 256;
