@@ -717,8 +717,12 @@ __global__ __launch_bounds__(kTile, 4) void k_vox_tile(const VoxParams* __restri
       const uint64_t lim = (uint64_t)P.small_cols;
       nu = (uint32_t)(K.i[I_G1U] - K.i[I_G0U] + 1);
       nv = (uint32_t)(K.i[I_G1V] - K.i[I_G0V] + 1);
-      large = (K.slab() ? (nc > lim) : (K.work() > lim * 8)) || nc > (uint64_t)kColMask;
-      if (!large) ncols = (uint32_t)nc;
+      // (a bbox end beyond the range of int truncates to INT_MIN, and an end before its start
+      // covers nothing)
+      if (min(min((int)nu, (int)nv), K.i[I_G1W] - K.i[I_G0W] + 1) > 0) {
+        large = (K.slab() ? (nc > lim) : (K.work() > lim * 8)) || nc > (uint64_t)kColMask;
+        if (!large) ncols = (uint32_t)nc;
+      }
     }
     // A lane walking its own triangle takes ~100 instructions a column, in as many steps as
     // the tile's largest triangle has columns; the rows and columns of the whole tile take

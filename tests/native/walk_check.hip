@@ -42,9 +42,10 @@ extern "C" void walk_check(const float* tris, uint64_t n, float unit, uint64_t g
     make_walk(S, P, (uint32_t)q, K);
     FastTri F;
     make_fast(K, P, F);
-    if (F.rf & kFastCareful) out[4]++;
     const int w = K.w(), ua = w == 0 ? 1 : 0, va = w == 2 ? 1 : 2;
     const int nb = K.i[I_G1V] - K.i[I_G0V] + 1, na = K.i[I_G1U] - K.i[I_G0U] + 1, nc = (int)(F.c.ck >> 16);
+    if (na < 1 || nb < 1 || nc < 1) continue;  // nothing to test (an inverted bbox)
+    if (F.rf & kFastCareful) out[4]++;
     for (int j = 0; j < nb; j++) {
       FastRow R;
       fast_row(F, j, nb, R);

@@ -52,6 +52,18 @@ def test_large_triangles_in_jobs(small_cols, aligned):
         assert np.array_equal(_codes(ctx, tris, False, G), _want(tris, False, G))
 
 
+def test_bbox_ends_beyond_int():
+    """A coordinate past the range of int truncates to INT_MIN as on x86: its bbox is inverted
+    or clamped to the grid's first layer."""
+    G = 64
+    tris = _mesh(np.random.default_rng(8), 300, 3.0 / G)
+    tris[::5, 3] = 1e12
+    tris[1::5, 7] = -1e12
+    tris[2::5, 2] = 3e38
+    with SvoContext(0) as ctx:
+        assert np.array_equal(_codes(ctx, tris, False, G), _want(tris, False, G))
+
+
 def test_fresh_context_waits_for_its_own_read_back():
     """A new context's pinned read-back area may be memory a closed context left its completion
     flag in: the first read-back must not take that flag for its own."""
