@@ -288,7 +288,7 @@ void svo_ctx_destroy(svo_ctx* ctx) {
   c.gexec.clear();
   c.glog.clear();
   DevBuf* bufs[] = {&c.tris, &c.jobdev, &c.batch_tris, &c.hitbox, &c.part_lists, &c.unitdev,
-                    &c.table, &c.pool, &c.pool8, &c.grid8, &c.counters, &c.large_unit,
+                    &c.table, &c.pool, &c.pool8, &c.grid8, &c.cflags, &c.counters, &c.large_unit,
                     &c.large_tri, &c.large_rows, &c.large_jobs, &c.occ_list, &c.bcount,
                     &c.wprefix, &c.winner, &c.scan_scratch, &c.codes, &c.records, &c.nodes,
                     &c.lvl_code, &c.lvl_size, &c.lvl_mask, &c.lvl_first, &c.lvl_start,

@@ -260,6 +260,8 @@ struct Context {
   std::vector<uint8_t> unit_img;  // what unitdev holds before uvoff (empty: unknown)
   DevBuf table, pool, pool8;  // pool: bit words per slot; pool8: bytes per slot
   DevBuf grid8;               // dense byte grids of a pass's units (when they fit)
+  DevBuf cflags;              // dense payload units: a byte per 64-voxel word of a table entry
+  uint64_t cflags_zeroed = 0; // bytes of cflags known to be zero
   uint64_t table_entries = 0;
   uint64_t grid_zeroed = 0;     // bytes of grid8 known to be zero
   uint64_t pool_cap = 0;        // slots of pool8 (and of pool) on the touch path

@@ -255,6 +255,7 @@ __device__ __forceinline__ void walk_all_columns(const Walk& K, const VoxParams&
 // Global buffers the actions work on; each action binds its unit's segment.
 struct ActArgs {
   uint32_t* table;    // all units' brick tables, concatenated
+  uint8_t* cflags;    // dense payload units: a byte per 64-voxel word of every table entry
   uint8_t* pool8;     // touch path: 4096 bytes per slot
   ull* pool;          // 64 bit words per slot (written by the compaction)
   uint32_t* wprefix;  // per word: batch rank of its first voxel
@@ -286,11 +287,13 @@ struct TouchAction {
 // same value, so no atomic read-modify-write is needed however many triangles cover it
 // (about three per voxel on a terrain).
 //  * dense units (MarkDenseT): a byte per voxel of the unit's Morton range (the
-//    reference's own layout, voxelizer.cpp:144, kept in HBM); the brick's table entry is
-//    flagged with a plain store when the thread enters a brick. Only flagged bricks are
-//    compacted and cleared afterwards, so the grid is never swept. Dense payload units
+//    reference's own layout, voxelizer.cpp:144, kept in HBM); a byte of the brick's table entry
+//    is set with a plain store when the thread enters a quarter of it (1 KiB). Only flagged
+//    quarters are compacted and cleared afterwards, so the grid is never swept. Dense payload units
 //    keep 4 bytes per voxel and resolve the winning triangle in the same walk (atomicMax
-//    of ~triangle: voxelizer.cpp:263, the first triangle in partition order wins).
+//    of ~triangle: voxelizer.cpp:263, the first triangle in partition order wins); they flag
+//    64-voxel words as well (256 bytes of cells). Flagged words for all units made the
+//    headline's mark 13 us slower for 3 us of its compaction.
 //  * touch units (MarkPoolAction): 4096 bytes per pool slot; the slot comes from the table
 //    (touch pass + table scan), cached per thread.
 // Both store through global (not generic) pointers.
@@ -306,14 +309,16 @@ struct MarkDenseT {
   static constexpr bool kTouch = false;
   using Unordered = MarkDenseT<kWide, false>;
   __device__ static bool narrow(const VoxParams& P) { return !kWide || (!kLaneOrder && !P.wide); }
-  gword_t* table;
+  gbyte_t* table;  // the unit's table segment, a byte per quarter of a brick
+  gbyte_t* words;  // the unit's word flags (payload units)
   gbyte_t* bytes;
   uint64_t base;  // code of the first voxel of the unit's first brick
   int wide;
-  uint32_t cbrick = 0xFFFFFFFFu;
+  uint32_t cquarter = 0xFFFFFFFFu, cword = 0xFFFFFFFFu;  // the last ones marked
   __device__ static MarkDenseT make(const ActArgs& A, const VoxParams& P) {
     MarkDenseT m;
-    m.table = (gword_t*)(A.table + P.table_base);
+    m.table = (gbyte_t*)(A.table + P.table_base);
+    m.words = (gbyte_t*)(A.cflags + P.table_base * kBrickWords);
     m.bytes = (gbyte_t*)P.grid8;
     m.base = P.bstart;
     m.wide = kWide ? P.wide : 0;
@@ -322,7 +327,7 @@ struct MarkDenseT {
   __device__ __forceinline__ void touch(uint64_t) {}
   __device__ __forceinline__ void add(uint64_t code, uint32_t tri) {
     const uint64_t rel = code - base;
-    const uint32_t b = (uint32_t)(rel >> kBrickBits);
+    const uint32_t q = (uint32_t)(rel >> (kBrickBits - 2));
     if (kWide && wide) {
       // the lowest covering triangle as the largest ~tri (0 = unmarked). With kLaneOrder
       // a lane whose left neighbour marks the same cell in the same step holds a triangle
@@ -340,11 +345,16 @@ struct MarkDenseT {
               phi == (uint32_t)(addr >> 32);
       }
       if (!dup) atomicMax(cell, ~tri);
+      const uint32_t w = (uint32_t)(rel >> 6);
+      if (w != cword) {
+        cword = w;
+        words[w] = 1;
+      }
     } else
       bytes[rel] = 1;
-    if (b != cbrick) {
-      cbrick = b;
-      table[b] = 1u;
+    if (q != cquarter) {
+      cquarter = q;
+      table[q] = 1;
     }
   }
   __device__ __forceinline__ void flush() {}
@@ -835,14 +845,31 @@ struct OccLoad {
   const uint32_t* table;
   __device__ uint32_t operator()(uint64_t i) const { return table[i] != 0u; }
 };
+// Touch path: flagged entries become slot + 1 (slots in Morton order).
 struct OccStore {
   uint32_t* occ;
-  uint32_t* table;  // flagged entries become slot + 1 (slots in Morton order)
+  uint32_t* table;
   ull* ctr;
   __device__ void operator()(uint64_t i, uint32_t ex, uint32_t v, bool last) const {
     if (v) {
       occ[ex] = (uint32_t)i;
       table[i] = ex + 1u;
+    }
+    if (last) ctr[kCtrNumOcc] = (ull)(ex + v);
+  }
+};
+// Dense passes: the list entries carry the brick's flagged quarters above its table index
+// (the dense limit, 2^37 cells, keeps that below 2^25).
+constexpr int kOccBits = 28;
+constexpr uint32_t kOccMask = (1u << kOccBits) - 1u;
+struct OccStoreDense {
+  uint32_t* occ;
+  const uint32_t* table;
+  ull* ctr;
+  __device__ void operator()(uint64_t i, uint32_t ex, uint32_t v, bool last) const {
+    if (v) {
+      const uint32_t quarters = __builtin_amdgcn_udot4(table[i], 0x08040201u, 0u, false);
+      occ[ex] = (uint32_t)i | (quarters << kOccBits);
     }
     if (last) ctr[kCtrNumOcc] = (ull)(ex + v);
   }
@@ -859,13 +886,21 @@ __device__ __forceinline__ uint64_t waves_total() {
 
 // Pack each flagged brick's bytes into 64 bit words (lane l = voxels 64l..64l+63) at the
 // brick's rank, count its voxels, and zero the bytes that were set. The bytes live in the
-// unit's dense grid (at the brick's index) or in the slot pool (at its rank).
+// unit's dense grid (at the brick's index; only its flagged quarters, or words of payload
+// cells, are read) or in the slot pool (at its rank). Bound by those reads: an eighth of a
+// soup's bricks in 1771 us with whole bricks read.
 // ubase[u] = first table entry of unit u (n_units + 1 entries).
 // Dense passes flag only bricks that hold voxels, so the rank is the brick's place in the
 // brick stream: there 'pool' is the stream's word array, bcode (non-null) receives the
 // tagged brick codes and the table entries are cleared here.
 // ONE: a single unit (its parameters are uniform, read with scalar loads).
 
+// 16 bytes, each 0 or 1, as 16 bits
+__device__ __forceinline__ uint32_t pack16(uint4 v) {
+  const uint32_t lo = __builtin_amdgcn_udot4(v.y, 0x80402010u, __builtin_amdgcn_udot4(v.x, 0x08040201u, 0u, false), false);
+  const uint32_t hi = __builtin_amdgcn_udot4(v.w, 0x80402010u, __builtin_amdgcn_udot4(v.z, 0x08040201u, 0u, false), false);
+  return lo | (hi << 8);
+}
 // Brick wv (table entry ti, unit u): its tagged code, and its table entry cleared.
 __device__ __forceinline__ void brick_head(uint64_t wv, uint64_t ti, uint32_t u,
                                            const VoxParams* __restrict__ units,
@@ -878,29 +913,19 @@ __device__ __forceinline__ void brick_head(uint64_t wv, uint64_t ti, uint32_t u,
     table[ti] = 0u;
   }
 }
-// The lane's 16-byte pieces of a brick's bytes: load q of lane l is the 16 bytes at
-// q * 1024 + 16 l (each load of the wave one contiguous KiB).
-__device__ __forceinline__ uint4* brick_bytes(uint64_t wv, uint64_t ti, uint32_t u,
-                                              const VoxParams* __restrict__ units,
-                                              const uint64_t* __restrict__ ubase,
-                                              uint8_t* __restrict__ pool8) {
-  uint8_t* base = units[u].dense ? units[u].grid8 + (ti - ubase[u]) * kBrickVox
-                                 : pool8 + wv * kBrickVox;
-  return (uint4*)base + lane_id();
-}
-// The lane's occupancy word from the loaded pieces (piece q of lane l holds bits
-// 16 (l % 4) .. + 15 of word 16 q + l / 4); pieces that held marks are zeroed.
-__device__ __forceinline__ ull pack_brick_bytes(uint4* src, const uint4 (&v)[4]) {
+// A brick of bytes as occupancy words: load q of lane l is the 16 bytes at q * 1024 + 16 l (each
+// load of the wave one contiguous KiB, quarter q of the brick, made if its flag is set); they
+// are packed into the lane's word (piece q of lane l holds bits 16 (l % 4) .. + 15 of word
+// 16 q + l / 4); pieces that held marks are zeroed.
+__device__ __forceinline__ ull pack_bytes(uint4* src, uint32_t quarters) {
   ull parts = 0;  // 16 bits per load
+  uint4 v[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    v[q] = (quarters >> q) & 1u ? src[q * kWave] : make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
   for (int q = 0; q < 4; q++) {
-    const uint32_t w4[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
-#pragma unroll
-    for (int d = 0; d < 4; d++) {
-      const uint32_t x = w4[d];  // four bytes, each 0 or 1
-      const uint32_t nib = (x & 1u) | ((x >> 7) & 2u) | ((x >> 14) & 4u) | ((x >> 21) & 8u);
-      parts |= (ull)nib << (16 * q + 4 * d);
-    }
+    parts |= (ull)pack16(v[q]) << (16 * q);
     if (v[q].x | v[q].y | v[q].z | v[q].w) src[q * kWave] = make_uint4(0u, 0u, 0u, 0u);
   }
   // word L = 16 q + r gathers the parts of load q from lanes 4 r .. 4 r + 3
@@ -912,6 +937,30 @@ __device__ __forceinline__ ull pack_brick_bytes(uint4* src, const uint4 (&v)[4])
     const uint32_t hi = (uint32_t)__shfl((int)(uint32_t)(parts >> 32), 4 * r + k, kWave);
     const ull p = ((ull)hi << 32) | lo;
     m |= ((p >> (16 * q)) & 0xFFFFull) << (16 * k);
+  }
+  return m;
+}
+// A payload brick's cells as occupancy words: the lane's own 64 cells (kept: they hold the
+// winners), read only when their word's flag is set.
+__device__ __forceinline__ ull pack_cells(const uint32_t* cells, uint8_t* flags) {
+  const int lane = lane_id();
+  const bool set = flags[lane] != 0;
+  flags[lane] = 0;
+  ull m = 0;
+  if (!set) return m;
+  const uint4* src = (const uint4*)cells + lane * 16;
+  // four loads at a time: few registers, so that many waves stay resident
+#pragma unroll 1
+  for (int g = 0; g < 16; g += 4) {
+    uint4 v[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) v[q] = src[g + q];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const uint32_t nib = (v[q].x != 0u ? 1u : 0u) | (v[q].y != 0u ? 2u : 0u) |
+                           (v[q].z != 0u ? 4u : 0u) | (v[q].w != 0u ? 8u : 0u);
+      m |= (ull)nib << (4 * (g + q));
+    }
   }
   return m;
 }
@@ -939,6 +988,7 @@ __device__ __forceinline__ void brick_count_body(const uint32_t* __restrict__ oc
                                                  const VoxParams* __restrict__ units,
                                                  const uint64_t* __restrict__ ubase,
                                                  uint32_t n_units, uint8_t* __restrict__ pool8,
+                                                 uint8_t* __restrict__ cflags,
                                                  ull* __restrict__ pool,
                                                  uint64_t* __restrict__ bcount,
                                                  uint64_t* __restrict__ bcode,
@@ -947,34 +997,18 @@ __device__ __forceinline__ void brick_count_body(const uint32_t* __restrict__ oc
   for (uint64_t wv = wave_global(); wv < n_occ; wv += waves_total()) {
     // the brick is the wave's: its table index in a scalar register, so that the unit
     // search below runs on scalar loads
-    const uint64_t ti = (uint32_t)__builtin_amdgcn_readfirstlane((int)occ[wv]);
+    const uint32_t oe = (uint32_t)__builtin_amdgcn_readfirstlane((int)occ[wv]);
+    const uint64_t ti = bcode ? oe & kOccMask : oe;
+    const uint32_t quarters = bcode ? oe >> kOccBits : 15u;
     const uint32_t u = ONE ? 0u : upper_index<uint64_t>(ubase, n_units + 1, ti);
     brick_head(wv, ti, u, units, ubase, bcode, table);
-    ull m = 0;
-    if (units[u].wide) {
-      // 4-byte cells (~winner, 0 = unmarked): kept for k_brick_emit, which clears them
-      const uint4* src = (const uint4*)((const uint32_t*)units[u].grid8 +
-                                        (ti - ubase[u]) * kBrickVox + lane_id() * 64);
-      // four loads at a time: few registers, so that many waves stay resident
-#pragma unroll 1
-      for (int g = 0; g < 16; g += 4) {
-        uint4 v[4];
-#pragma unroll
-        for (int q = 0; q < 4; q++) v[q] = src[g + q];
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-          const uint32_t nib = (v[q].x != 0u ? 1u : 0u) | (v[q].y != 0u ? 2u : 0u) |
-                               (v[q].z != 0u ? 4u : 0u) | (v[q].w != 0u ? 8u : 0u);
-          m |= (ull)nib << (4 * (g + q));
-        }
-      }
-    } else {
-      uint4* src = brick_bytes(wv, ti, u, units, ubase, pool8);
-      uint4 v[4];
-#pragma unroll
-      for (int q = 0; q < 4; q++) v[q] = src[q * kWave];
-      m = pack_brick_bytes(src, v);
-    }
+    const uint64_t bi = ti - ubase[u];
+    ull m;
+    if (units[u].wide)
+      m = pack_cells((const uint32_t*)units[u].grid8 + bi * kBrickVox, cflags + ti * kBrickWords);
+    else
+      m = pack_bytes((uint4*)(units[u].dense ? units[u].grid8 + bi * kBrickVox
+                                             : pool8 + wv * kBrickVox) + lane_id(), quarters);
     brick_tail(wv, m, pool, bcount, bcode, bshape);
   }
 }
@@ -984,6 +1018,7 @@ __global__ __launch_bounds__(256) void k_brick_count(const uint32_t* __restrict_
                                                      const VoxParams* __restrict__ units,
                                                      const uint64_t* __restrict__ ubase,
                                                      uint32_t n_units, uint8_t* __restrict__ pool8,
+                                                     uint8_t* __restrict__ cflags,
                                                      ull* __restrict__ pool,
                                                      uint64_t* __restrict__ bcount,
                                                      uint64_t* __restrict__ bcode,
@@ -992,10 +1027,10 @@ __global__ __launch_bounds__(256) void k_brick_count(const uint32_t* __restrict_
   // more flagged bricks than slots (touch path): the pass is redone with a larger pool
   const uint64_t n_occ = min((uint64_t)ctr[kCtrNumOcc], cap);
   if (n_units == 1)
-    brick_count_body<true>(occ, n_occ, units, ubase, n_units, pool8, pool, bcount, bcode,
+    brick_count_body<true>(occ, n_occ, units, ubase, n_units, pool8, cflags, pool, bcount, bcode,
                            bshape, table);
   else
-    brick_count_body<false>(occ, n_occ, units, ubase, n_units, pool8, pool, bcount, bcode,
+    brick_count_body<false>(occ, n_occ, units, ubase, n_units, pool8, cflags, pool, bcount, bcode,
                             bshape, table);
 }
 
@@ -1045,7 +1080,8 @@ __global__ __launch_bounds__(256) void k_brick_emit(const uint32_t* __restrict__
   extern __shared__ uint32_t s_cells[];  // stage_cells: kBrickVox per wave
   const uint64_t n_occ = ctr[kCtrNumOcc];
   for (uint64_t wv = wave_global(); wv < n_occ; wv += waves_total()) {
-    const uint64_t ti = (uint32_t)__builtin_amdgcn_readfirstlane((int)occ[wv]);  // wave's brick
+    const uint32_t oe = (uint32_t)__builtin_amdgcn_readfirstlane((int)occ[wv]);  // wave's brick
+    const uint64_t ti = write_stream ? oe : oe & kOccMask;
     const uint32_t u = upper_index<uint64_t>(ubase, n_units + 1, ti);
     // a dense pass has its brick stream already (k_brick_count): only the payload units'
     // bricks have work left
@@ -1148,7 +1184,9 @@ __global__ __launch_bounds__(256) void k_brick_clear(const uint32_t* __restrict_
 }
 
 // First voxel (batch rank) of each unit: the offset of its first flagged brick.
-__global__ void k_unit_voxels(const uint32_t* __restrict__ occ, const ull* __restrict__ ctr,
+// (occ_mask: the table index in an occ entry)
+__global__ void k_unit_voxels(const uint32_t* __restrict__ occ, uint32_t occ_mask,
+                              const ull* __restrict__ ctr,
                               const uint64_t* __restrict__ ubase, uint32_t n_units,
                               const uint64_t* __restrict__ boff, uint64_t* __restrict__ uvoff) {
   const uint32_t u = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1163,7 +1201,7 @@ __global__ void k_unit_voxels(const uint32_t* __restrict__ occ, const ull* __res
   uint64_t lo = 0, hi = n_occ;
   while (lo < hi) {
     const uint64_t mid = (lo + hi) >> 1;
-    if ((uint64_t)occ[mid] < ubase[u])
+    if ((uint64_t)(occ[mid] & occ_mask) < ubase[u])
       lo = mid + 1;
     else
       hi = mid;
@@ -1662,7 +1700,8 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
   const bool dense = dense_bytes <= c.dense_limit;
   bool geometry_only = true;  // no unit carries payload records
   for (uint32_t u = 0; u < nu; u++) geometry_only = geometry_only && units[u].stride == 9;
-  // the table, the dense grid and the byte pool are all-zero whenever no pass is running
+  // the table, the word flags, the dense grid and the byte pool are all-zero whenever no pass
+  // is running
   if (c.table_entries < ntab) {
     SVO_TRY(ensure(c.table, ntab * 4));
     SVO_TRY(fill_u32(c.table.as<uint32_t>(), 0, ntab, c.stream));
@@ -1681,6 +1720,11 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
       }
       SVO_TRY(fill_u64(c.grid8.as<uint64_t>(), 0, target / 8, c.stream));
       c.grid_zeroed = target;
+    }
+    if (!geometry_only && c.cflags_zeroed < ntab * kBrickWords) {
+      SVO_TRY(ensure(c.cflags, ntab * kBrickWords));
+      SVO_TRY(fill_u64(c.cflags.as<uint64_t>(), 0, ntab * kBrickWords / 8, c.stream));
+      c.cflags_zeroed = ntab * kBrickWords;
     }
     for (uint32_t u = 0; u < nu; u++) {
       P[u].dense = 1;
@@ -1753,6 +1797,7 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
   auto args = [&]() {
     ActArgs A;
     A.table = c.table.as<uint32_t>();
+    A.cflags = c.cflags.as<uint8_t>();
     A.pool8 = c.pool8.as<uint8_t>();
     A.pool = pool_words;
     A.wprefix = c.wprefix.as<uint32_t>();
@@ -1787,6 +1832,11 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
   ull* st_bc = nullptr;
   ull* queues = nullptr;  // 3 x kQueueWords: the tile queues of the mark/touch, second and winner passes
   auto occ_scan = [&]() {
+    if (dense)
+      return scan_single<uint32_t>(
+          OccLoad{c.table.as<uint32_t>()},
+          OccStoreDense{c.occ_list.as<uint32_t>(), c.table.as<uint32_t>(), ctr}, ntab, st_occ,
+          ctr + kCtrError, c.stream);
     return scan_single<uint32_t>(
         OccLoad{c.table.as<uint32_t>()},
         OccStore{c.occ_list.as<uint32_t>(), c.table.as<uint32_t>(), ctr}, ntab, st_occ,
@@ -1844,8 +1894,8 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
       ktimer_begin(c, "brick_count");
       SVO_LAUNCH(k_brick_count, dim3(brick_grid(bc_bound)), dim3(256), 0, c.stream,
                          c.occ_list.as<uint32_t>(), ctr, bc_bound, d_units, d_ubase, nu,
-                         c.pool8.as<uint8_t>(), pool_words, c.bcount.as<uint64_t>(),
-                         dense ? c.bcode.as<uint64_t>() + nb0 : (uint64_t*)nullptr,
+                         c.pool8.as<uint8_t>(), c.cflags.as<uint8_t>(), pool_words,
+                         c.bcount.as<uint64_t>(), dense ? c.bcode.as<uint64_t>() + nb0 : (uint64_t*)nullptr,
                          dense ? c.bshape.as<uint32_t>() + nb0 : (uint32_t*)nullptr,
                          dense ? c.table.as<uint32_t>() : (uint32_t*)nullptr);
       ktimer_end(c);
@@ -1874,8 +1924,8 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
             c.scan_scratch.as<uint64_t>(), c.stream, ctr + kCtrNumOcc)));
       if (!(nu == 1 && geometry_only)) {
         SVO_LAUNCH(k_unit_voxels, dim3((nu + 256) / 256), dim3(256), 0, c.stream,
-                   c.occ_list.as<uint32_t>(), ctr, d_ubase, nu, c.bcount.as<uint64_t>(),
-                   d_uvoff);
+                   c.occ_list.as<uint32_t>(), dense ? kOccMask : 0xFFFFFFFFu, ctr, d_ubase, nu,
+                   c.bcount.as<uint64_t>(), d_uvoff);
         SVO_TRY(hipGetLastError());
       }
       return hipSuccess;

@@ -64,6 +64,23 @@ def test_bbox_ends_beyond_int():
         assert np.array_equal(_codes(ctx, tris, False, G), _want(tris, False, G))
 
 
+@pytest.mark.parametrize("size", [1.0, 40.0])
+def test_words_and_flags_are_clear_again(size):
+    """The same context over another mesh and back: no mark, flag or cell is left behind."""
+    G = 128
+    rng = np.random.default_rng(3)
+    a, b = _mesh(rng, 500, size / G), _mesh(rng, 700, 2.0 / G)
+    pay = np.concatenate([b, rng.uniform(0, 1, (700, 12)).astype(np.float32)], axis=1)
+    with SvoContext(0) as ctx:
+        want = _want(a, False, G)
+        for mesh, payload in ((a, False), (pay, True), (b, False), (a, False)):
+            got = _codes(ctx, mesh, payload, G)
+            if mesh is a:
+                assert np.array_equal(got, want)
+            else:
+                assert np.array_equal(got, _want(mesh, payload, G))
+
+
 def test_fresh_context_waits_for_its_own_read_back():
     """A new context's pinned read-back area may be memory a closed context left its completion
     flag in: the first read-back must not take that flag for its own."""
