@@ -109,6 +109,15 @@ __device__ __forceinline__ float canon_nan(float f) {
   return (f != f) ? __uint_as_float(0xFFC00000u) : f;
 }
 
+// Pointers to device memory. One read from memory (a unit's or job's) is generic to the
+// compiler otherwise, which then emits flat accesses: every LDS wait becomes one for them and
+// for all memory accesses before them.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(1))) uint8_t gbyte_t;
+typedef __attribute__((address_space(1))) uint32_t gword_t;
+typedef __attribute__((address_space(1))) float gfloat_t;
+typedef __attribute__((address_space(1))) u32x4 gquad_t;
+
 // ------------------------------------------------------------------------------------
 // Wave-level helpers (64 lanes)
 // ------------------------------------------------------------------------------------

@@ -297,8 +297,6 @@ struct TouchAction {
 //  * touch units (MarkPoolAction): 4096 bytes per pool slot; the slot comes from the table
 //    (touch pass + table scan), cached per thread.
 // Both store through global (not generic) pointers.
-typedef __attribute__((address_space(1))) uint8_t gbyte_t;
-typedef __attribute__((address_space(1))) uint32_t gword_t;
 // kWide: some units of the pass carry payload (4-byte cells; the unit's wide flag decides
 // per voxel); otherwise every cell is a byte. kLaneOrder: the lanes of a wave hold
 // non-decreasing triangle indices (the small tier: tile order, item order), and a lane
@@ -333,7 +331,7 @@ struct MarkDenseT {
       // a lane whose left neighbour marks the same cell in the same step holds a triangle
       // no lower than the neighbour's and leaves the atomic to it: on fine meshes
       // neighbouring triangles cover the same voxels
-      uint32_t* cell = (uint32_t*)bytes + rel;
+      gword_t* cell = (gword_t*)bytes + rel;
       bool dup = false;
       if (kLaneOrder) {
         const uint64_t addr = (uint64_t)cell;
@@ -344,7 +342,8 @@ struct MarkDenseT {
         dup = ln > 0 && ((act >> (ln - 1)) & 1ull) && plo == (uint32_t)addr &&
               phi == (uint32_t)(addr >> 32);
       }
-      if (!dup) atomicMax(cell, ~tri);
+      if (!dup)
+        __hip_atomic_fetch_max(cell, ~tri, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const uint32_t w = (uint32_t)(rel >> 6);
       if (w != cword) {
         cword = w;
@@ -676,7 +675,7 @@ __global__ __launch_bounds__(kTile, 4) void k_vox_tile(const VoxParams* __restri
                                                        ActArgs A, ull* queue, LargeList B,
                                                        uint32_t tt, int collect, int skip) {
   __shared__ WalkLds s_walk[kTileWaves];
-  __shared__ uint32_t s_empty[kQueues];  // ranges found empty
+  __shared__ volatile uint32_t s_empty[kQueues];  // classes found empty
   if (threadIdx.x < kQueues) s_empty[threadIdx.x] = 0;
   fill_spread_table();
   __syncthreads();  // the waves part here
@@ -696,13 +695,13 @@ __global__ __launch_bounds__(kTile, 4) void k_vox_tile(const VoxParams* __restri
   for (;;) {
     if (!one_each) {
       for (uint32_t tried = 0; tried < 2; tried++) {
-        if (!*(volatile uint32_t*)&s_empty[cls]) {
+        if (!s_empty[cls]) {
           uint32_t k = 0;
           if (lane == 0) k = (uint32_t)atomicAdd(queue + kQueueStride * cls, 1ull);
           k = (uint32_t)__builtin_amdgcn_readfirstlane((int)k);
           next = (k / kTileRun * kQueues + cls) * kTileRun + k % kTileRun;
           if (next < total) break;
-          *(volatile uint32_t*)&s_empty[cls] = 1u;
+          s_empty[cls] = 1u;
         }
         cls = (cls + 1) % kQueues;
       }
@@ -719,9 +718,9 @@ __global__ __launch_bounds__(kTile, 4) void k_vox_tile(const VoxParams* __restri
     uint32_t ncols = 0, nu = 0, nv = 0;  // columns of a triangle of this tier; its sides
     bool large = false;
     if ((uint32_t)lane < tt && i < P.n) {
-      const uint32_t t = P.list ? P.list[i] : i;
+      const uint32_t t = P.list ? ((const gword_t*)P.list)[i] : i;
       Setup S;
-      setup_tri(P.tris + (uint64_t)t * P.stride, P, S);
+      setup_tri((const gfloat_t*)P.tris + (uint64_t)t * P.stride, P, S);
       make_walk(S, P, t, K);
       const uint64_t nc = K.columns();
       const uint64_t lim = (uint64_t)P.small_cols;
@@ -820,7 +819,7 @@ __global__ __launch_bounds__(kTile, 3) void k_vox_large(const VoxParams* __restr
       for (int k = 0; k < kWalkWords / 4; k++) wk[k] = src[kTriQuads + k];
     } else {
       Setup S;
-      setup_tri(P.tris + (uint64_t)B.tri[idx] * P.stride, P, S);
+      setup_tri((const gfloat_t*)P.tris + (uint64_t)B.tri[idx] * P.stride, P, S);
       make_walk(S, P, B.tri[idx], K);
       FastTri F;
       make_fast(K, P, F);
@@ -896,7 +895,7 @@ __device__ __forceinline__ uint64_t waves_total() {
 // ONE: a single unit (its parameters are uniform, read with scalar loads).
 
 // 16 bytes, each 0 or 1, as 16 bits
-__device__ __forceinline__ uint32_t pack16(uint4 v) {
+__device__ __forceinline__ uint32_t pack16(u32x4 v) {
   const uint32_t lo = __builtin_amdgcn_udot4(v.y, 0x80402010u, __builtin_amdgcn_udot4(v.x, 0x08040201u, 0u, false), false);
   const uint32_t hi = __builtin_amdgcn_udot4(v.w, 0x80402010u, __builtin_amdgcn_udot4(v.z, 0x08040201u, 0u, false), false);
   return lo | (hi << 8);
@@ -917,16 +916,18 @@ __device__ __forceinline__ void brick_head(uint64_t wv, uint64_t ti, uint32_t u,
 // load of the wave one contiguous KiB, quarter q of the brick, made if its flag is set); they
 // are packed into the lane's word (piece q of lane l holds bits 16 (l % 4) .. + 15 of word
 // 16 q + l / 4); pieces that held marks are zeroed.
-__device__ __forceinline__ ull pack_bytes(uint4* src, uint32_t quarters) {
+__device__ __forceinline__ ull pack_bytes(gquad_t* src, uint32_t quarters) {
   ull parts = 0;  // 16 bits per load
-  uint4 v[4];
+  u32x4 v[4];
 #pragma unroll
-  for (int q = 0; q < 4; q++)
-    v[q] = (quarters >> q) & 1u ? src[q * kWave] : make_uint4(0u, 0u, 0u, 0u);
+  for (int q = 0; q < 4; q++) {
+    v[q] = u32x4{0u, 0u, 0u, 0u};
+    if ((quarters >> q) & 1u) v[q] = src[q * kWave];
+  }
 #pragma unroll
   for (int q = 0; q < 4; q++) {
     parts |= (ull)pack16(v[q]) << (16 * q);
-    if (v[q].x | v[q].y | v[q].z | v[q].w) src[q * kWave] = make_uint4(0u, 0u, 0u, 0u);
+    if (v[q].x | v[q].y | v[q].z | v[q].w) src[q * kWave] = u32x4{0u, 0u, 0u, 0u};
   }
   // word L = 16 q + r gathers the parts of load q from lanes 4 r .. 4 r + 3
   const int L = lane_id(), q = L >> 4, r = L & 15;
@@ -942,17 +943,17 @@ __device__ __forceinline__ ull pack_bytes(uint4* src, uint32_t quarters) {
 }
 // A payload brick's cells as occupancy words: the lane's own 64 cells (kept: they hold the
 // winners), read only when their word's flag is set.
-__device__ __forceinline__ ull pack_cells(const uint32_t* cells, uint8_t* flags) {
+__device__ __forceinline__ ull pack_cells(const gquad_t* cells, uint8_t* flags) {
   const int lane = lane_id();
   const bool set = flags[lane] != 0;
   flags[lane] = 0;
   ull m = 0;
   if (!set) return m;
-  const uint4* src = (const uint4*)cells + lane * 16;
+  const gquad_t* src = cells + lane * 16;
   // four loads at a time: few registers, so that many waves stay resident
 #pragma unroll 1
   for (int g = 0; g < 16; g += 4) {
-    uint4 v[4];
+    u32x4 v[4];
 #pragma unroll
     for (int q = 0; q < 4; q++) v[q] = src[g + q];
 #pragma unroll
@@ -1005,10 +1006,11 @@ __device__ __forceinline__ void brick_count_body(const uint32_t* __restrict__ oc
     const uint64_t bi = ti - ubase[u];
     ull m;
     if (units[u].wide)
-      m = pack_cells((const uint32_t*)units[u].grid8 + bi * kBrickVox, cflags + ti * kBrickWords);
+      m = pack_cells((const gquad_t*)units[u].grid8 + bi * (kBrickVox / 4), cflags + ti * kBrickWords);
     else
-      m = pack_bytes((uint4*)(units[u].dense ? units[u].grid8 + bi * kBrickVox
-                                             : pool8 + wv * kBrickVox) + lane_id(), quarters);
+      m = pack_bytes((gquad_t*)(units[u].dense ? units[u].grid8 + bi * kBrickVox
+                                               : pool8 + wv * kBrickVox) + lane_id(),
+                     quarters);
     brick_tail(wv, m, pool, bcount, bcode, bshape);
   }
 }
@@ -1055,12 +1057,9 @@ struct BrickOffStore {
   }
 };
 
-// The brick stream entry of every non-empty flagged brick and, with kCodes, for payload
-// units the sorted codes of its voxels, tagged with the unit's job in bits kJobShift+
-// (and the payload winners of dense payload units). stage_cells: the launch gives each
-// wave kBrickVox words of dynamic LDS, into which a dense payload brick's 4-byte cells
-// are copied with coalesced loads (and cleared in the grid) before its voxels read their
-// winners from there, instead of one dependent global load per voxel.
+// Touched-brick passes: the brick stream entry of every non-empty flagged brick and, with
+// kCodes, for payload units the sorted codes of its voxels, tagged with the unit's job in bits
+// kJobShift+.
 template <bool kCodes>
 __global__ __launch_bounds__(256) void k_brick_emit(const uint32_t* __restrict__ occ,
                                                     const ull* __restrict__ ctr,
@@ -1074,25 +1073,18 @@ __global__ __launch_bounds__(256) void k_brick_emit(const uint32_t* __restrict__
                                                     uint64_t s0, uint64_t* __restrict__ bwords,
                                                     uint64_t* __restrict__ bcode,
                                                     uint64_t* __restrict__ bvoff,
-                                                    uint32_t* __restrict__ bshape,
-                                                    uint32_t* __restrict__ winner,
-                                                    int stage_cells, int write_stream) {
-  extern __shared__ uint32_t s_cells[];  // stage_cells: kBrickVox per wave
+                                                    uint32_t* __restrict__ bshape) {
   const uint64_t n_occ = ctr[kCtrNumOcc];
   for (uint64_t wv = wave_global(); wv < n_occ; wv += waves_total()) {
-    const uint32_t oe = (uint32_t)__builtin_amdgcn_readfirstlane((int)occ[wv]);  // wave's brick
-    const uint64_t ti = write_stream ? oe : oe & kOccMask;
+    const uint64_t ti = (uint32_t)__builtin_amdgcn_readfirstlane((int)occ[wv]);  // wave's brick
     const uint32_t u = upper_index<uint64_t>(ubase, n_units + 1, ti);
-    // a dense pass has its brick stream already (k_brick_count): only the payload units'
-    // bricks have work left
-    if (!write_stream && units[u].stride == 9) continue;
     const uint64_t slot = wv * kBrickWords + lane_id();
     ull word = pool[slot];
     const uint64_t bo = boff[wv];
     const uint64_t tag = (uint64_t)units[u].job << kJobShift;
     const uint64_t b0 = units[u].bstart + ((ti - ubase[u]) << kBrickBits);
     // the brick stream (non-empty bricks, appended in stream order)
-    if (write_stream && __ballot(word != 0ull)) {
+    if (__ballot(word != 0ull)) {
       const uint64_t sb = bo >> kNonEmptyShift;
       bwords[sb * kBrickWords + lane_id()] = word;
       const BrickShape B = brick_shape_of(word);
@@ -1107,45 +1099,10 @@ __global__ __launch_bounds__(256) void k_brick_emit(const uint32_t* __restrict__
     const uint32_t c = (uint32_t)__popcll(word);
     const uint32_t inc = wave_incl_scan<uint32_t>(c);
     uint64_t pos = (bo & kVoxMask) + (inc - c);
-    if (wprefix) wprefix[slot] = (uint32_t)pos;
+    wprefix[slot] = (uint32_t)pos;
     const uint64_t cb = (b0 + ((uint64_t)lane_id() << 6)) | tag;
-    // dense payload unit: each voxel's winner from its cell, which is cleared
-    if (units[u].wide && stage_cells) {
-      uint32_t* sc = s_cells + (threadIdx.x / kWave) * kBrickVox;
-      uint4* src = (uint4*)((uint32_t*)units[u].grid8 + (ti - ubase[u]) * kBrickVox);
-      uint4 v[kBrickVox / 4 / kWave];
-      // uint4 r * 64 + l holds cells of word 4 r + l / 16: the cells of an empty word are
-      // all zero, so only those of non-empty words are read
-      const uint64_t ne = __ballot(word != 0ull);
-#pragma unroll
-      for (int r = 0; r < kBrickVox / 4 / kWave; r++)
-        v[r] = ((ne >> (4 * r + (lane_id() >> 4))) & 1ull) ? src[r * kWave + lane_id()]
-                                                           : make_uint4(0u, 0u, 0u, 0u);
-#pragma unroll
-      for (int r = 0; r < kBrickVox / 4 / kWave; r++) {
-        ((uint4*)sc)[r * kWave + lane_id()] = v[r];
-        if (v[r].x | v[r].y | v[r].z | v[r].w) src[r * kWave + lane_id()] = make_uint4(0u, 0u, 0u, 0u);
-      }
-      wave_lds_sync();
-      const uint32_t* mine = sc + lane_id() * 64;  // the cells of the lane's word
-      while (word) {
-        const int bit = __ffsll(word) - 1;
-        winner[pos] = ~mine[bit];
-        codes[pos++] = cb + (uint64_t)bit;
-        word &= word - 1;
-      }
-      wave_lds_sync();  // the next brick's cells overwrite these
-      continue;
-    }
-    uint32_t* cells = units[u].wide ? (uint32_t*)units[u].grid8 + (ti - ubase[u]) * kBrickVox +
-                                          lane_id() * 64
-                                    : nullptr;
     while (word) {
       const int bit = __ffsll(word) - 1;
-      if (cells) {
-        winner[pos] = ~cells[bit];
-        cells[bit] = 0u;
-      }
       codes[pos++] = cb + (uint64_t)bit;
       word &= word - 1;
     }
@@ -1210,7 +1167,190 @@ __global__ void k_unit_voxels(const uint32_t* __restrict__ occ, uint32_t occ_mas
 }
 
 // ---------------------------------------------------------------- payload records
-// BarycentricCoords.h:4-32 for the winning triangle; colour modes of main.cpp:373-382.
+// Exact quotient x / d of a grid coordinate: a power of two d (a unit bbox) needs no division.
+__device__ __forceinline__ float coord_over(uint32_t x, float d, float inv_d, bool pow2) {
+  return pow2 ? (float)(int)x * inv_d : (float)(int)x / d;
+}
+// The record of voxel 'code' won by triangle t: BarycentricCoords.h:4-32; colour modes of
+// main.cpp:373-382.
+__device__ __forceinline__ void put_payload_record(const JobDev& J, uint64_t code, uint32_t t,
+                                                   float* __restrict__ r) {
+  float col0, col1, col2, nr0, nr1, nr2;
+  const gfloat_t* p = (const gfloat_t*)J.tris + (uint64_t)t * 21;
+  const float v0x = p[0], v0y = p[1], v0z = p[2];
+  const float v1x = p[3], v1y = p[4], v1z = p[5];
+  const float v2x = p[6], v2y = p[7], v2z = p[8];
+  nr0 = p[9];
+  nr1 = p[10];
+  nr2 = p[11];
+  uint32_t x, y, z;
+  unmorton3(code, x, y, z);
+  const int color_mode = J.color_mode;
+  const float unit_div = J.unit_div;
+  if (color_mode == 0) {
+    // n = normalize(cross(e0, e1)) exactly as in the voxelizer
+    const float e0x = v1x - v0x, e0y = v1y - v0y, e0z = v1z - v0z;
+    const float e1x = v2x - v1x, e1y = v2y - v1y, e1z = v2z - v1z;
+    const float cx = e0y * e1z - e1y * e0z;
+    const float cy = e0z * e1x - e1z * e0x;
+    const float cz = e0x * e1y - e1x * e0y;
+    const float inv = 1.0f / sqrtf((cx * cx + cy * cy) + cz * cz);
+    const float nx = cx * inv, ny = cy * inv, nz = cz * inv;
+    // (a power of two in the middle of the exponent range: its reciprocal is exact)
+    const uint32_t ub = __float_as_uint(unit_div);
+    const bool pow2 = (ub & 0x807FFFFFu) == 0u && (ub >> 23) > 64u && (ub >> 23) < 190u;
+    const float inv_div = __builtin_amdgcn_ldexpf(1.0f, 127 - (int)(ub >> 23));
+    const float vx = coord_over(x, unit_div, inv_div, pow2);
+    const float vy = coord_over(y, unit_div, inv_div, pow2);
+    const float vz = coord_over(z, unit_div, inv_div, pow2);
+    const float coeffD = -((v0x * nx + v0y * ny) + v0z * nz);
+    const float k = (((vx * nx + vy * ny) + vz * nz) + coeffD) / ((nx * nx + ny * ny) + nz * nz);
+    const float qx = vx - k * nx, qy = vy - k * ny, qz = vz - k * nz;
+    // glm::inverse(mat3(v0, v1, v2)), m[c][r]
+    const float m00 = v0x, m01 = v0y, m02 = v0z;
+    const float m10 = v1x, m11 = v1y, m12 = v1z;
+    const float m20 = v2x, m21 = v2y, m22 = v2z;
+    const float det = (m00 * (m11 * m22 - m21 * m12) - m10 * (m01 * m22 - m21 * m02)) +
+                      m20 * (m01 * m12 - m11 * m02);
+    const float o = 1.0f / det;
+    const float i00 = (m11 * m22 - m21 * m12) * o;
+    const float i10 = (-(m10 * m22 - m20 * m12)) * o;
+    const float i20 = (m10 * m21 - m20 * m11) * o;
+    const float i01 = (-(m01 * m22 - m21 * m02)) * o;
+    const float i11 = (m00 * m22 - m20 * m02) * o;
+    const float i21 = (-(m00 * m21 - m20 * m01)) * o;
+    const float i02 = (m01 * m12 - m11 * m02) * o;
+    const float i12 = (-(m00 * m12 - m10 * m02)) * o;
+    const float i22 = (m00 * m11 - m10 * m01) * o;
+    const float bx = (i00 * qx + i10 * qy) + i20 * qz;
+    const float by = (i01 * qx + i11 * qy) + i21 * qz;
+    const float bz = (i02 * qx + i12 * qy) + i22 * qz;
+    col0 = (bx * p[12] + by * p[15]) + bz * p[18];
+    col1 = (bx * p[13] + by * p[16]) + bz * p[19];
+    col2 = (bx * p[14] + by * p[17]) + bz * p[20];
+  } else if (color_mode == 1) {  // fixed white
+    col0 = col1 = col2 = 1.0f;
+  } else if (color_mode == 2) {  // mortonToRGB: (z, y, x) / gridsize
+    const float g = (float)J.gridsize;
+    col0 = (float)z / g;
+    col1 = (float)y / g;
+    col2 = (float)x / g;
+  } else {  // normal -> colour
+    const float inv = 1.0f / sqrtf((nr0 * nr0 + nr1 * nr1) + nr2 * nr2);
+    const float a = nr0 * inv, b = nr1 * inv, c = nr2 * inv;
+    col0 = (a + 1.0f) / 2.0f;
+    col1 = (b + 1.0f) / 2.0f;
+    col2 = (c + 1.0f) / 2.0f;
+  }
+  uint4 q0, q1;
+  q0.x = (uint32_t)code;
+  q0.y = (uint32_t)(code >> 32);
+  q0.z = __float_as_uint(canon_nan(col0));
+  q0.w = __float_as_uint(canon_nan(col1));
+  q1.x = __float_as_uint(canon_nan(col2));
+  q1.y = __float_as_uint(canon_nan(nr0));
+  q1.z = __float_as_uint(canon_nan(nr1));
+  q1.w = __float_as_uint(canon_nan(nr2));
+  ((uint4*)r)[0] = q0;
+  ((uint4*)r)[1] = q1;
+}
+
+// Position of the n-th set bit of w (n below its count)
+__device__ __forceinline__ uint32_t nth_set_bit(uint64_t w, uint32_t n) {
+  uint32_t lo = (uint32_t)w, at = 0;
+  const uint32_t c = (uint32_t)__popc(lo);
+  if (n >= c) {
+    n -= c;
+    lo = (uint32_t)(w >> 32);
+    at = 32;
+  }
+#pragma unroll
+  for (int h = 16; h; h >>= 1) {
+    const uint32_t k = (uint32_t)__popc(lo & ((1u << h) - 1u));
+    const bool up = n >= k;
+    n -= up ? k : 0u;
+    lo = up ? lo >> h : lo;
+    at += up ? h : 0;
+  }
+  return at;
+}
+
+// The records of a dense pass's payload units, straight from their bricks: a wave per brick,
+// its voxels 64 at a time in Morton order, so that neighbouring lanes read neighbouring cells
+// (~the winning triangle, 0 = unmarked) and write neighbouring records. The cells of non-empty
+// words are zeroed afterwards, whole 256-byte words at once. Codes and winners are not written
+// (ensure_codes expands the codes for readers that want them).
+//
+// Bound by memory: 32 bytes written a voxel, the cells' words, and the winners' records
+// gathered. A pass that wrote every voxel's code and winner (a lane per word, its voxels one
+// after the other) and one that read them back took 242 + 336 us on 17M voxels of a rough
+// sphere; this one 403 (1.9M voxels of a fine terrain: 34 + 71 us, 81).
+__global__ __launch_bounds__(256) void k_payload_bricks(
+    const uint32_t* __restrict__ occ, const ull* __restrict__ n_occ_ptr,
+    const VoxParams* __restrict__ units, const uint64_t* __restrict__ ubase, uint32_t n_units,
+    const ull* __restrict__ words, const uint64_t* __restrict__ boff,
+    const JobDev* __restrict__ jobs, uint64_t s0, float* __restrict__ out, ull* ctr) {
+  __shared__ uint8_t s_slot[256];
+  uint8_t* slot = s_slot + (threadIdx.x / kWave) * kWave;
+  const int lane = lane_id();
+  const uint64_t n_occ = *n_occ_ptr;
+  for (uint64_t wv = wave_global(); wv < n_occ; wv += waves_total()) {
+    const uint32_t ti = (uint32_t)__builtin_amdgcn_readfirstlane((int)occ[wv]) & kOccMask;
+    const uint32_t u = upper_index<uint64_t>(ubase, n_units + 1, (uint64_t)ti);
+    if (!units[u].wide) continue;
+    const ull word = words[wv * kBrickWords + lane];
+    gword_t* cells = (gword_t*)units[u].grid8 + (ti - ubase[u]) * kBrickVox;
+    const uint64_t code0 = units[u].bstart + ((ti - ubase[u]) << kBrickBits);
+    const JobDev& J = jobs[units[u].job];
+    const uint64_t pos0 = boff[wv] & kVoxMask;  // the brick's first voxel in the pass
+    float* rec = out + (J.dbase + 1 + (s0 + pos0 - J.voff)) * 8;
+    const uint32_t c = (uint32_t)__popcll(word);
+    const uint32_t inc = wave_incl_scan<uint32_t>(c), pre = inc - c;
+    const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)inc, kWave - 1);
+    // (the next window's cells are on their way while this one's records are made)
+    uint32_t carry = 0, v = 0, cell = 0;
+    auto fetch = [&](uint32_t k0, uint32_t& vo, uint32_t& co) {
+      const uint32_t wi = locate(slot, pre, c != 0, k0, carry) & 63u;
+      const uint32_t wlo = (uint32_t)__shfl((int)(uint32_t)word, (int)wi, kWave);
+      const uint32_t whi = (uint32_t)__shfl((int)(uint32_t)(word >> 32), (int)wi, kWave);
+      const uint32_t wpre = (uint32_t)__shfl((int)pre, (int)wi, kWave);
+      const uint32_t k = k0 + lane;
+      if (k < n) {
+        vo = wi * 64u + nth_set_bit(((uint64_t)whi << 32) | wlo, k - wpre);
+        co = cells[vo];
+      }
+    };
+    if (n) fetch(0, v, cell);
+    for (uint32_t k0 = 0; k0 < n; k0 += kWave) {
+      uint32_t v2 = 0, cell2 = 0;
+      if (k0 + kWave < n) fetch(k0 + kWave, v2, cell2);
+      const uint32_t k = k0 + lane;
+      if (k < n) {
+        if (cell == 0u)  // cannot happen: the words were made from the cells
+          atomicAdd(&ctr[kCtrError], 1ull);
+        else
+          put_payload_record(J, code0 + v, ~cell, rec + (uint64_t)k * 8);
+      }
+      v = v2;
+      cell = cell2;
+    }
+    // (every cell has been read: the records were made from them)
+    uint64_t ne = __ballot(word != 0ull);
+    while (ne) {  // four words at a time, 16 lanes each
+      uint32_t mine = 64u;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const uint32_t wi = ne ? (uint32_t)__ffsll((long long)ne) - 1u : 64u;
+        if ((lane >> 4) == q) mine = wi;
+        ne &= ne - 1ull;
+      }
+      if (mine < 64u) ((gquad_t*)(cells + mine * 64u))[lane & 15] = u32x4{0u, 0u, 0u, 0u};
+    }
+  }
+}
+
+// Touched-brick passes: one thread per payload voxel, its code and winner from the arrays that
+// k_brick_emit and the winner walk wrote.
 // Voxel i of the pass (stream index s0 + i) belongs to the unit whose voxel range holds
 // it, and to that unit's job; its record goes to dbase[job] + 1 + (s0 + i - voff[job]).
 // Voxels of geometry-only jobs have no record here.
@@ -1239,82 +1379,10 @@ __global__ __launch_bounds__(256) void k_payload_records(
   if (!J.payload) return;
   const uint64_t code = tagged & kCodeMask;
   const uint32_t t = winner[i];
-  float col0, col1, col2, nr0, nr1, nr2;
-  if (t == 0xFFFFFFFFu) {  // cannot happen: both passes evaluate the same predicates
+  if (t == 0xFFFFFFFFu)  // cannot happen: both passes evaluate the same predicates
     atomicAdd(&ctr[kCtrError], 1ull);
-    col0 = col1 = col2 = nr0 = nr1 = nr2 = 0.0f;
-  } else {
-    const float* p = J.tris + (uint64_t)t * 21;
-    const float v0x = p[0], v0y = p[1], v0z = p[2];
-    const float v1x = p[3], v1y = p[4], v1z = p[5];
-    const float v2x = p[6], v2y = p[7], v2z = p[8];
-    nr0 = p[9];
-    nr1 = p[10];
-    nr2 = p[11];
-    uint32_t x, y, z;
-    unmorton3(code, x, y, z);
-    const int color_mode = J.color_mode;
-    const float unit_div = J.unit_div;
-    if (color_mode == 0) {
-      // n = normalize(cross(e0, e1)) exactly as in the voxelizer
-      const float e0x = v1x - v0x, e0y = v1y - v0y, e0z = v1z - v0z;
-      const float e1x = v2x - v1x, e1y = v2y - v1y, e1z = v2z - v1z;
-      const float cx = e0y * e1z - e1y * e0z;
-      const float cy = e0z * e1x - e1z * e0x;
-      const float cz = e0x * e1y - e1x * e0y;
-      const float inv = 1.0f / sqrtf((cx * cx + cy * cy) + cz * cz);
-      const float nx = cx * inv, ny = cy * inv, nz = cz * inv;
-      const float vx = (float)(int)x / unit_div;
-      const float vy = (float)(int)y / unit_div;
-      const float vz = (float)(int)z / unit_div;
-      const float coeffD = -((v0x * nx + v0y * ny) + v0z * nz);
-      const float k = (((vx * nx + vy * ny) + vz * nz) + coeffD) / ((nx * nx + ny * ny) + nz * nz);
-      const float qx = vx - k * nx, qy = vy - k * ny, qz = vz - k * nz;
-      // glm::inverse(mat3(v0, v1, v2)), m[c][r]
-      const float m00 = v0x, m01 = v0y, m02 = v0z;
-      const float m10 = v1x, m11 = v1y, m12 = v1z;
-      const float m20 = v2x, m21 = v2y, m22 = v2z;
-      const float det = (m00 * (m11 * m22 - m21 * m12) - m10 * (m01 * m22 - m21 * m02)) +
-                        m20 * (m01 * m12 - m11 * m02);
-      const float o = 1.0f / det;
-      const float i00 = (m11 * m22 - m21 * m12) * o;
-      const float i10 = (-(m10 * m22 - m20 * m12)) * o;
-      const float i20 = (m10 * m21 - m20 * m11) * o;
-      const float i01 = (-(m01 * m22 - m21 * m02)) * o;
-      const float i11 = (m00 * m22 - m20 * m02) * o;
-      const float i21 = (-(m00 * m21 - m20 * m01)) * o;
-      const float i02 = (m01 * m12 - m11 * m02) * o;
-      const float i12 = (-(m00 * m12 - m10 * m02)) * o;
-      const float i22 = (m00 * m11 - m10 * m01) * o;
-      const float bx = (i00 * qx + i10 * qy) + i20 * qz;
-      const float by = (i01 * qx + i11 * qy) + i21 * qz;
-      const float bz = (i02 * qx + i12 * qy) + i22 * qz;
-      col0 = (bx * p[12] + by * p[15]) + bz * p[18];
-      col1 = (bx * p[13] + by * p[16]) + bz * p[19];
-      col2 = (bx * p[14] + by * p[17]) + bz * p[20];
-    } else if (color_mode == 1) {  // fixed white
-      col0 = col1 = col2 = 1.0f;
-    } else if (color_mode == 2) {  // mortonToRGB: (z, y, x) / gridsize
-      const float g = (float)J.gridsize;
-      col0 = (float)z / g;
-      col1 = (float)y / g;
-      col2 = (float)x / g;
-    } else {  // normal -> colour
-      const float inv = 1.0f / sqrtf((nr0 * nr0 + nr1 * nr1) + nr2 * nr2);
-      const float a = nr0 * inv, b = nr1 * inv, c = nr2 * inv;
-      col0 = (a + 1.0f) / 2.0f;
-      col1 = (b + 1.0f) / 2.0f;
-      col2 = (c + 1.0f) / 2.0f;
-    }
-  }
-  float* r = out + (J.dbase + 1 + (s0 + i - J.voff)) * 8;
-  *(uint64_t*)r = code;
-  r[2] = canon_nan(col0);
-  r[3] = canon_nan(col1);
-  r[4] = canon_nan(col2);
-  r[5] = canon_nan(nr0);
-  r[6] = canon_nan(nr1);
-  r[7] = canon_nan(nr2);
+  else
+    put_payload_record(J, code, t, out + (J.dbase + 1 + (s0 + i - J.voff)) * 8);
 }
 
 // ---------------------------------------------------------------- partition kernels
@@ -2024,10 +2092,10 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
       return hipErrorInvalidValue;
     }
     if (winner_walk) SVO_TRY(ensure(c.wprefix, n_occ * kBrickWords * 4));
-    if (any_payload) SVO_TRY(ensure(c.winner, nvox * 4));
-    // geometry-only passes write no codes: the build reads the brick stream, and
+    if (winner_walk) SVO_TRY(ensure(c.winner, nvox * 4));
+    // dense and geometry-only passes write no codes: the build reads the brick stream, and
     // ensure_codes writes the codes for readers that want them
-    const bool codes_now = any_payload;
+    const bool codes_now = winner_walk;
     SVO_TRY(ensure_keep(c.codes, (s0 + nvox) * 8, s0 * 8, c.stream));
     if (!dense) {
       SVO_TRY(ensure_keep(c.bwords, (nb0 + n_occ) * kBrickWords * 8, nb0 * kBrickWords * 8,
@@ -2047,6 +2115,8 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
       // records: each job's first record is its null record
       const uint64_t keep = batch ? c.records.cap : (1 + s0) * 32;
       SVO_TRY(ensure_keep(c.records, n_records * 32, keep, c.stream));
+    }
+    if (winner_walk) {
       std::vector<uint64_t> pr(1, 0), ps, pu;
       for (uint32_t u = 0; u < nu; u++) {
         const uint64_t cnt = uvoff[u + 1] - uvoff[u];
@@ -2072,27 +2142,29 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     }
     // the pass's remaining kernels: one graph segment
     SVO_TRY(run_segment(c, [&]() -> hipError_t {
-      // a dense pass has its brick stream entries already (k_brick_count); the emit pass
-      // writes the codes and winners of its payload units
-      if (!dense || codes_now) {
+      // a dense pass has its brick stream entries already (k_brick_count)
+      if (!dense) {
         ktimer_begin(c, "brick_emit");
-        // dense payload units: their cells are staged through LDS, kBrickVox words per wave
-        const bool stage_cells = codes_now && dense && any_payload;
         SVO_LAUNCH(codes_now ? k_brick_emit<true> : k_brick_emit<false>,
-                   dim3(brick_grid(n_occ)), dim3(256),
-                   stage_cells ? (256 / kWave) * kBrickVox * 4 : 0, c.stream,
+                   dim3(brick_grid(n_occ)), dim3(256), 0, c.stream,
                    c.occ_list.as<uint32_t>(), ctr, d_units, d_ubase, nu, pool_words,
                    c.bcount.as<uint64_t>(), c.codes.as<uint64_t>() + s0,
                    winner_walk ? c.wprefix.as<uint32_t>() : (uint32_t*)nullptr, s0,
                    c.bwords.as<uint64_t>() + nb0 * kBrickWords, c.bcode.as<uint64_t>() + nb0,
-                   c.bvoff.as<uint64_t>() + nb0, c.bshape.as<uint32_t>() + nb0,
-                   any_payload ? c.winner.as<uint32_t>() : (uint32_t*)nullptr,
-                   stage_cells ? 1 : 0, dense ? 0 : 1);
+                   c.bvoff.as<uint64_t>() + nb0, c.bshape.as<uint32_t>() + nb0);
+        ktimer_end(c);
+        SVO_TRY(hipGetLastError());
+      } else if (any_payload) {
+        ktimer_begin(c, "payload_records");
+        SVO_LAUNCH(k_payload_bricks, dim3(brick_grid(n_occ)), dim3(256), 0, c.stream,
+                   c.occ_list.as<uint32_t>(), (const ull*)(ctr + kCtrNumOcc),
+                   (const VoxParams*)d_units, d_ubase, nu, (const ull*)pool_words,
+                   c.bcount.as<uint64_t>(), c.jobdev.as<JobDev>(), s0, c.records.as<float>(), ctr);
         ktimer_end(c);
         SVO_TRY(hipGetLastError());
       }
-      if (any_payload) {
-        if (winner_walk) {
+      if (winner_walk) {
+        {
           SVO_TRY(fill_u32(c.winner.as<uint32_t>(), 0xFFFFFFFFu, nvox, c.stream));
           SVO_TRY(tile_pass(WinnerAction{}, "vox_small_winner", queues + 2 * kQueueWords, 0,
                             kSkipBinary));

@@ -49,9 +49,10 @@ struct Setup {
   double nv0, nc, nm;
 };
 
-// voxelizer.cpp:189-254 (bbox, clamp, normal, critical point, edge functions)
-SVO_HD void setup_tri(const float* __restrict__ p, const VoxParams& P,
-                                          Setup& S) {
+// voxelizer.cpp:189-254 (bbox, clamp, normal, critical point, edge functions) of the nine
+// floats at p
+template <typename FloatPtr>
+SVO_HD void setup_tri(FloatPtr p, const VoxParams& P, Setup& S) {
   const float v0x = p[0], v0y = p[1], v0z = p[2];
   const float v1x = p[3], v1y = p[4], v1z = p[5];
   const float v2x = p[6], v2y = p[7], v2z = p[8];
