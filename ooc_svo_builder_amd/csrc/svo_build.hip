@@ -341,6 +341,11 @@ __device__ __forceinline__ void job_bases(JobDev* jobs, uint32_t n_jobs,
 // carry, a barrier before the next level reads it), then the per-job bases.
 constexpr int kTailBlock = 1024;
 constexpr uint64_t kTailLevelMax = 8192;  // largest level bound the tail block takes
+// The level scans' stores walk a parent's children (dependent loads, and with -levels their
+// averages): one element a thread up to this many keeps enough blocks in flight. With eight,
+// the levels of 487,600 voxels ran on 60 blocks: 375 us for four of them.
+constexpr uint64_t kLevelScanSmall = 1ull << 23;
+constexpr uint64_t kTopLevelMax = 4096;  // largest level bound k_emit_levels_top takes
 __global__ __launch_bounds__(kTailBlock) void k_levels_tail(
     Arena A, LevelMeta M, Tags T, JobDev* jobs, uint32_t n_jobs, const uint64_t* leaves,
     uint32_t* leaf_parent, unsigned long long* root_size, unsigned long long* root_isize,
@@ -392,15 +397,11 @@ __device__ __forceinline__ void put_data(float* rec, uint64_t idx, const float* 
 // own record (children_base relative to its job's node array) and start; with -levels
 // also its data record. Consecutive nodes land in consecutive records, so the stores
 // coalesce.
-__global__ __launch_bounds__(256) void k_emit_level(Arena A, LevelMeta M, Tags T,
-                                                    const JobDev* __restrict__ jobs, int h,
-                                                    uint64_t node_cap,
-                                                    uint64_t* __restrict__ nodes,
-                                                    float* __restrict__ out_rec) {
-  if (M.flag[0]) return;  // arena overflow: the build is redone with a larger arena
-  const uint64_t nc = M.n[h];
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nc) return;
+__device__ __forceinline__ void emit_level_node(const Arena& A, const LevelMeta& M, const Tags& T,
+                                                const JobDev* __restrict__ jobs, int h,
+                                                uint64_t i, uint64_t node_cap,
+                                                uint64_t* __restrict__ nodes,
+                                                float* __restrict__ out_rec) {
   const uint64_t co = M.off[h];
   const uint64_t code = A.code[co + i];
   const JobDev& J = jobs[T.job(code)];
@@ -443,6 +444,30 @@ __global__ __launch_bounds__(256) void k_emit_level(Arena A, LevelMeta M, Tags T
     put_data(out_rec, J.dbase + idx, A.cache + (co + i) * 6);
   }
   put_node(J, nodes, gpos, data, st + sz - 1 - (uint32_t)__popc(cm), offsets_of(cm));
+}
+__global__ __launch_bounds__(256) void k_emit_level(Arena A, LevelMeta M, Tags T,
+                                                    const JobDev* __restrict__ jobs, int h,
+                                                    uint64_t node_cap,
+                                                    uint64_t* __restrict__ nodes,
+                                                    float* __restrict__ out_rec) {
+  if (M.flag[0]) return;  // arena overflow: the build is redone with a larger arena
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < M.n[h]) emit_level_node(A, M, T, jobs, h, i, node_cap, nodes, out_rec);
+}
+// Heights H .. h_lo, all small, in one block (a height reads what the one above it wrote):
+// a launch each took 5 us whatever it did.
+__global__ __launch_bounds__(kTailBlock) void k_emit_levels_top(Arena A, LevelMeta M, Tags T,
+                                                                const JobDev* __restrict__ jobs,
+                                                                int h_lo, int H, uint64_t node_cap,
+                                                                uint64_t* __restrict__ nodes,
+                                                                float* __restrict__ out_rec) {
+  if (M.flag[0]) return;
+  for (int h = H; h >= h_lo; h--) {
+    const uint64_t n = M.n[h];
+    for (uint64_t i = threadIdx.x; i < n; i += kTailBlock)
+      emit_level_node(A, M, T, jobs, h, i, node_cap, nodes, out_rec);
+    __syncthreads();
+  }
 }
 
 // Every node of heights hs..H in one launch (geometry records, no -levels data): one
@@ -1093,7 +1118,7 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
       }
     const int h_scan_end = up_once ? h0 : h_tail;  // level scans for h0 .. h_scan_end-1
     uint64_t st_words = 0;
-    for (int h = h0; h < h_scan_end; h++) st_words += scan_single_words(bound[h]);
+    for (int h = h0; h < h_scan_end; h++) st_words += scan_single_words(bound[h], kLevelScanSmall);
     SVO_TRY(ensure(c.lvl_aux, (meta_words + st_words) * 8));
     if (levels) {
       SVO_TRY(ensure(c.lvl_isize, cap * 8));
@@ -1171,8 +1196,8 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
                        root_size, root_isize, c.records.as<float>() + 8, h};
         SVO_TRY((scan_single<uint32_t>(ld, st, bound[h], status,
                                        c.counters.as<unsigned long long>() + kCtrError, c.stream,
-                                       M.n + h)));
-        status += scan_single_words(bound[h]);
+                                       M.n + h, kLevelScanSmall)));
+        status += scan_single_words(bound[h], kLevelScanSmall);
       }
       SVO_LAUNCH(k_levels_tail, dim3(1), dim3(kTailBlock), 0, c.stream, A, M, T, d_jobs,
                          n_jobs, c.codes.as<uint64_t>(), c.lvl_leafp.as<uint32_t>(), root_size,
@@ -1192,7 +1217,16 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
         ktimer_end(c);
         SVO_TRY(hipGetLastError());
       }
-      for (int h = H; levels && h >= hs; h--) {
+      int h_top = H + 1;  // heights from here up in one launch
+      while (levels && h_top > hs && bound[h_top - 1] <= kTopLevelMax) h_top--;
+      if (h_top <= H) {
+        ktimer_begin(c, "emit_children");
+        SVO_LAUNCH(k_emit_levels_top, dim3(1), dim3(kTailBlock), 0, c.stream, A, M, T,
+                   (const JobDev*)d_jobs, h_top, H, node_cap, nodes, out_rec);
+        ktimer_end(c);
+        SVO_TRY(hipGetLastError());
+      }
+      for (int h = h_top - 1; levels && h >= hs; h--) {
         ktimer_begin(c, "emit_children");
         SVO_LAUNCH(k_emit_level, dim3((unsigned)std::max<uint64_t>((bound[h] + 255) / 256, 1)),
                            dim3(256), 0, c.stream, A, M, T, (const JobDev*)d_jobs, h, node_cap,

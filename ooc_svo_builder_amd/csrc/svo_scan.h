@@ -292,21 +292,25 @@ __global__ __launch_bounds__(kSingleBlock) void k_scan_single(Load ld, Store st,
   }
 }
 
-// Items per thread of the single-pass scan for n elements, and its status words.
-inline int scan_single_items(uint64_t n) { return n >= kSingleSmall ? kScanItems : 1; }
-inline uint64_t scan_single_words(uint64_t n) {
-  const uint64_t tile = (uint64_t)kSingleBlock * scan_single_items(n);
+// Items per thread of the single-pass scan for n elements, and its status words: one item below
+// 'small' elements.
+inline int scan_single_items(uint64_t n, uint64_t small = kSingleSmall) {
+  return n >= small ? kScanItems : 1;
+}
+inline uint64_t scan_single_words(uint64_t n, uint64_t small = kSingleSmall) {
+  const uint64_t tile = (uint64_t)kSingleBlock * scan_single_items(n, small);
   return 1 + (n + tile - 1) / tile;
 }
 
-// Exclusive scan in one launch; 'status' holds scan_single_words(n) zero words. n is an
+// Exclusive scan in one launch; 'status' holds scan_single_words(n, small) zero words. n is an
 // upper bound when n_dev is given (as for scan_exclusive).
 template <typename T, typename Load, typename Store>
 hipError_t scan_single(Load ld, Store st, uint64_t n, unsigned long long* status,
                        unsigned long long* err, hipStream_t s,
-                       const unsigned long long* n_dev = nullptr) {
+                       const unsigned long long* n_dev = nullptr,
+                       uint64_t small = kSingleSmall) {
   if (n == 0) return hipSuccess;
-  const int items = scan_single_items(n);
+  const int items = scan_single_items(n, small);
   const uint64_t tile = (uint64_t)kSingleBlock * items;
   const unsigned nb = (unsigned)((n + tile - 1) / tile);
   if (items == kScanItems)
