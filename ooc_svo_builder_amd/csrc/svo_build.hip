@@ -251,15 +251,21 @@ struct ParentStore {
 };
 
 // Level bookkeeping before a build: all zero, n[0] = V and, when the four lowest levels
-// come from the brick stream, n[4] = NB and off[5] = NB.
+// come from the brick stream, n[4] = NB and off[5] = NB; the device clock in flag[3]; a single
+// job's descriptor (job, unless null) from the arguments.
+constexpr int kStampWord = 2 * 64 + 3;
 __global__ __launch_bounds__(256) void k_build_init(unsigned long long* meta, uint64_t words,
-                                                    uint64_t V, uint64_t NB, int fast) {
+                                                    uint64_t V, uint64_t NB, uint64_t fast,
+                                                    JobDev* job, JobDev j0) {
+  const unsigned long long now = wall_clock64();
   for (uint64_t i = threadIdx.x; i < words; i += blockDim.x) {
     unsigned long long v = 0;
     if (i == 0) v = V;
     if (fast && (i == 4 || i == 64 + 5)) v = NB;
+    if (i == kStampWord) v = now;
     meta[i] = v;
   }
+  if (job && threadIdx.x == 0) *job = j0;
 }
 
 // Per job, after the bottom-up passes: node count (a single null root for an empty
@@ -1080,10 +1086,17 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
     bound[h] = std::min(bound[h - 1], b);
     if (fast && h == 4) bound[h] = NB;
   }
-  // the voxelizer's last upload usually holds these already
-  if (c.jobdev_img.size() != jd.size() ||
+  // a batch's last upload usually holds these already; a single job goes by kernel argument
+  // (not into a graph, whose launches are compared by their argument bytes)
+  const bool job_arg = n_jobs == 1 && !c.graphs;
+  SVO_TRY(ensure(c.jobdev, n_jobs * sizeof(JobDev)));
+  if (c.clear_counters) {  // no pass came first
+    SVO_TRY(fill_u64(c.counters.as<uint64_t>(), 0, kNumCounters, c.stream));
+    c.clear_counters = false;
+  }
+  if (job_arg) {
+  } else if (c.jobdev_img.size() != jd.size() ||
       memcmp(c.jobdev_img.data(), jd.data(), n_jobs * sizeof(JobDev)) != 0) {
-    SVO_TRY(ensure(c.jobdev, n_jobs * sizeof(JobDev)));
     SVO_TRY(upload_async(c, c.jobdev.p, jd.data(), n_jobs * sizeof(JobDev)));
   }
   c.jobdev_img.clear();  // the job bases are written into it
@@ -1160,7 +1173,8 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
       // n[0] = V, off[1] = 0, flags = 0, root sizes = 0, hazard flags = 0, scan status = 0
       // (fast: n[4] = NB, off[4] = 0, off[5] = NB)
       SVO_LAUNCH(k_build_init, dim3(1), dim3(256), 0, c.stream, meta,
-                         meta_words + st_words, V, NB, fast ? 1 : 0);
+                         meta_words + st_words, V, NB, (uint64_t)(fast ? 1 : 0),
+                         job_arg ? d_jobs : (JobDev*)nullptr, jd[0]);
       SVO_TRY(hipGetLastError());
 
       if (up_once) {
@@ -1258,14 +1272,15 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
       }
       return hipSuccess;
     }));
-    unsigned long long flags[3] = {0, 0, 0};
+    unsigned long long flags[4] = {0, 0, 0, 0};
     if (c.build_done_ev) SVO_TRY(hipEventRecord(c.build_done_ev, c.stream));
     {
-      const ReadReq rq[3] = {{flags, M.flag, 24},
+      const ReadReq rq[3] = {{flags, M.flag, 32},
                              {jd.data(), d_jobs, n_jobs * sizeof(JobDev)},
                              {&c.err_count, c.counters.as<unsigned long long>() + kCtrError, 8}};
       SVO_TRY(read_back(c, rq, 3));
     }
+    c.stamp_build = flags[3];
     ktimer_flush(c);
     if (flags[1] && !flags[0]) {
       set_error("internal: node record out of range");

@@ -106,6 +106,7 @@ enum Counter : int {
   kCtrLargeJobs = 6,  // jobs of the large tier past its triangles' first ones
   kCtrError = 15,     // sticky: internal consistency failures (cleared per job)
   kCtrPartTotal = 16, // partition list length
+  kCtrStamp = 17,     // device clock at the start of the pass
   kNumCounters = 32
 };
 constexpr int kCtrPassClear = 15;  // counters 0..14 are cleared at the start of a pass
@@ -328,6 +329,12 @@ struct Context {
   uint32_t hread_seq = 0;
 
   StageTimes times;
+  // the run's counters are still to be cleared (the first pass does it, or the build)
+  bool clear_counters = false;
+  // device clock (wall_khz ticks a millisecond) at the start of the last pass, the start of the
+  // last build, and the last read-back
+  uint64_t stamp_pass = 0, stamp_build = 0, stamp_read = 0;
+  int wall_khz = 100000;
   hipEvent_t ev0 = nullptr, ev1 = nullptr, ev2 = nullptr, ev3 = nullptr;
   hipEvent_t build_done_ev = nullptr;  // when set, the build records it before its read-back
 
@@ -439,6 +446,9 @@ struct ReadReq {
   size_t bytes;
 };
 hipError_t read_back(Context& c, const ReadReq* reqs, int n);
+
+// Device-to-device copy on c.stream by a kernel; pointers and size are multiples of 8 bytes.
+hipError_t copy_records(Context& c, void* dst, const void* src, size_t bytes);
 
 // Stage drivers (return hipSuccess or an error; message in last error).
 // Partition job j's mesh into n_parts Morton-range partitions; lists appended to

@@ -1438,8 +1438,9 @@ __global__ void k_fill_u64(uint64_t* p, uint64_t v, uint64_t n) {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = v;
 }
-// two small ranges zeroed by one launch
-__global__ void k_zero2_u64(uint64_t* a, uint64_t na, uint64_t* b, uint64_t nb) {
+// start of a pass: two small ranges zeroed, the device clock in *stamp
+__global__ void k_pass_begin(uint64_t* a, uint64_t na, uint64_t* b, uint64_t nb, uint64_t* stamp) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *stamp = wall_clock64();
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < na + nb; i += stride) {
     if (i < na)
@@ -1448,6 +1449,8 @@ __global__ void k_zero2_u64(uint64_t* a, uint64_t na, uint64_t* b, uint64_t nb) 
       b[i - na] = 0;
   }
 }
+// one job's descriptor by kernel argument (a small copy costs more than a launch)
+__global__ void k_put_job(JobDev* dst, JobDev job) { *dst = job; }
 static unsigned fill_grid(uint64_t n) {
   uint64_t b = (n + 255) / 256;
   return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(b, 8192));
@@ -1501,12 +1504,13 @@ struct GatherArgs {
   uint32_t words[kGatherMax];
   int n;
 };
-// Then it raises *flag = seq (after a system-scope fence), which the host polls: a
-// shorter wait than a stream synchronization.
+// Then it leaves the device clock after the flag and raises *flag = seq (after a system-scope
+// fence), which the host polls: a shorter wait than a stream synchronization.
 __global__ __launch_bounds__(256) void k_gather_host(GatherArgs g, volatile uint32_t* flag,
                                                      uint32_t seq) {
   for (int k = 0; k < g.n; k++)
     for (uint32_t i = threadIdx.x; i < g.words[k]; i += blockDim.x) g.dst[k][i] = g.src[k][i];
+  if (threadIdx.x == 0) *(volatile uint64_t*)(flag + 2) = wall_clock64();
   __threadfence_system();
   __syncthreads();
   if (threadIdx.x == 0) *flag = seq;
@@ -1565,6 +1569,7 @@ hipError_t read_back(Context& c, const ReadReq* reqs, int n) {
       std::atomic_thread_fence(std::memory_order_acquire);
     else
       SVO_TRY(hipStreamSynchronize(c.stream));
+    c.stamp_read = ((volatile uint64_t*)c.hread)[1];
   } else {
     for (int k = 0; k < n; k++) {
       if (reqs[k].bytes)
@@ -1580,6 +1585,33 @@ hipError_t read_back(Context& c, const ReadReq* reqs, int n) {
     off += (reqs[k].bytes + 255) & ~(size_t)255;
   }
   return hipSuccess;
+}
+
+// n elements of 16 or 8 bytes, four in flight a thread; streamed past the caches
+template <typename T>
+__global__ __launch_bounds__(256) void k_copy(T* __restrict__ dst, const T* __restrict__ src,
+                                              uint64_t n) {
+  const uint64_t step = (uint64_t)gridDim.x * 256;
+  uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+  for (; i + 3 * step < n; i += 4 * step) {
+    T v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = __builtin_nontemporal_load(src + i + k * step);
+#pragma unroll
+    for (int k = 0; k < 4; k++) __builtin_nontemporal_store(v[k], dst + i + k * step);
+  }
+  for (; i < n; i += step) __builtin_nontemporal_store(__builtin_nontemporal_load(src + i), dst + i);
+}
+hipError_t copy_records(Context& c, void* dst, const void* src, size_t bytes) {
+  const bool wide = ((uintptr_t)dst | (uintptr_t)src | bytes) % 16 == 0;
+  const uint64_t n = bytes / (wide ? 16 : 8);
+  const unsigned grid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((n + 255) / 256, 8192));
+  if (wide)
+    SVO_LAUNCH(k_copy<u32x4>, dim3(grid), dim3(256), 0, c.stream, (u32x4*)dst, (const u32x4*)src, n);
+  else
+    SVO_LAUNCH(k_copy<uint64_t>, dim3(grid), dim3(256), 0, c.stream, (uint64_t*)dst,
+               (const uint64_t*)src, n);
+  return hipGetLastError();
 }
 
 static hipError_t ensure_scan_scratch(Context& c, uint64_t n, size_t elem) {
@@ -1927,9 +1959,10 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     SVO_TRY(run_segment(c, [&]() -> hipError_t {
       {  // pass counters, scan status words and tile queues
         const uint64_t ns = w_occ + w_bc + 3 * kQueueWords;
-        SVO_LAUNCH(k_zero2_u64, dim3(fill_grid(kCtrPassClear + ns)), dim3(256), 0,
-                           c.stream, (uint64_t*)ctr, (uint64_t)kCtrPassClear,
-                           c.scan_status.as<uint64_t>(), ns);
+        const uint64_t nc = c.clear_counters ? (uint64_t)kCtrStamp : (uint64_t)kCtrPassClear;
+        SVO_LAUNCH(k_pass_begin, dim3(fill_grid(nc + ns)), dim3(256), 0, c.stream,
+                   (uint64_t*)ctr, nc, c.scan_status.as<uint64_t>(), ns,
+                   (uint64_t*)(ctr + kCtrStamp));
         SVO_TRY(hipGetLastError());
       }
       // first pass: dense units mark directly, touch units flag their bricks; both collect
@@ -2010,6 +2043,8 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
                              {hc, c.counters.p, kNumCounters * sizeof(ull)}};
       SVO_TRY(read_back(c, rq, 2));
     }
+    c.clear_counters = false;
+    c.stamp_pass = hc[kCtrStamp];
     ktimer_flush(c);
     if (dense || (!hc[kCtrOverflow] && hc[kCtrNumOcc] <= c.pool_cap)) break;
     // pool too small for the flagged bricks: clear everything, grow, redo
@@ -2079,8 +2114,14 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     d.dbase = J.dbase;
   }
   SVO_TRY(ensure(c.jobdev, jd.size() * sizeof(JobDev)));
-  SVO_TRY(upload_async(c, c.jobdev.p, jd.data(), jd.size() * sizeof(JobDev)));
-  c.jobdev_img = jd;
+  c.jobdev_img.clear();
+  if (batch) {
+    SVO_TRY(upload_async(c, c.jobdev.p, jd.data(), jd.size() * sizeof(JobDev)));
+    c.jobdev_img = jd;
+  } else if (any_payload) {  // (else the build is its first reader, and writes it)
+    SVO_LAUNCH(k_put_job, dim3(1), dim3(1), 0, c.stream, c.jobdev.as<JobDev>(), jd[0]);
+    SVO_TRY(hipGetLastError());
+  }
 
   // ---- phase B: emit sorted codes, payload, clear; no synchronization
   if (n_occ) {
