@@ -573,26 +573,30 @@ __global__ __launch_bounds__(256) void k_emit_leaves(Arena A, LevelMeta M, Tags 
 // per brick writes every record below the brick node at its post-order position, and
 // the heights above come from the brick codes at once (upper levels, above).
 
-__device__ __forceinline__ BrickShape brick_shape(const uint64_t* __restrict__ bwords,
-                                                  uint64_t b) {
-  return brick_shape_of(bwords[b * kBrickWords + lane_id()]);
-}
-
-// Every record below each brick node, written record by record: the brick's records form
-// the contiguous range [S, S + s4 - 1) laid out as the word groups' subtree ranges, then
-// the group nodes; a group's range is its words' ranges, then its word nodes; a word's
-// range is its bytes' voxels, then its byte nodes. Per brick a wave builds the offsets of
-// these ranges in LDS, then lane r writes records r, r + 64, ... of the range (looking
-// its node up in the offsets), so consecutive lanes store consecutive records.
+// Every record below each brick node, a wave per brick. The brick's records form the contiguous
+// range [S, S + s4 - 1) laid out as the word groups' subtree ranges, then the group nodes; a
+// group's range is its words' ranges, then its word nodes; a word's range is its voxels, then
+// its byte nodes. So the voxels' records come in voxel order, whatever lies between them: the
+// wave lists its inner nodes (first child, child mask) in record order in LDS, with a bitmap of
+// their places, and lane r then writes records r, r + 64, ...: an inner node's from the list
+// (its place there is the count of bitmap bits before it), a voxel's from the count of clear
+// bits before it. Consecutive lanes store consecutive records.
+//
+// Bound by the writes, 24 bytes a node. Finding each record's node by searches in the ranges'
+// offsets took 740 vector instructions a brick, two thirds of the kernel's time.
 constexpr int kEmitWaves = 4;  // waves per block of k_emit_bricks
+constexpr int kInnerMax = 8 + 64 + 512;                        // inner nodes below a brick node
+constexpr int kInnerBits = (kBrickVox + kInnerMax + 63) / 64 * 2;  // bitmap, 32-bit words
 
-// last k in [0, 8) with a[k] <= v (a non-decreasing, a[0] <= v)
-__device__ __forceinline__ int last_le8(const uint32_t* a, uint32_t v) {
-  int k = 0;
-  if (a[k + 4] <= v) k += 4;
-  if (a[k + 2] <= v) k += 2;
-  if (a[k + 1] <= v) k += 1;
-  return k;
+// the child offsets of a mask (offsets_of) in two halves by multiplications: four mask bits
+// spread over the low bits of four bytes, their exclusive prefix sums, 0xFF where clear
+__device__ __forceinline__ uint64_t offsets_fast(uint32_t m) {
+  const uint32_t lo = ((m & 15u) * 0x00204081u) & 0x01010101u;
+  const uint32_t hi = ((m >> 4) * 0x00204081u) & 0x01010101u;
+  const uint32_t below = (uint32_t)__popc(m & 15u) * 0x01010101u;
+  const uint32_t l = (lo * 0x01010100u) | ((lo ^ 0x01010101u) * 0xFFu);
+  const uint32_t h = (hi * 0x01010100u + below) | ((hi ^ 0x01010101u) * 0xFFu);
+  return ((uint64_t)h << 32) | l;
 }
 
 // kPlaced: the job's records go to a larger node stream (a streamed partition), their
@@ -603,92 +607,91 @@ __global__ __launch_bounds__(kWave * kEmitWaves) void k_emit_bricks(
     const uint64_t* __restrict__ bwords, const uint64_t* __restrict__ bcode,
     const uint64_t* __restrict__ bvoff, uint64_t nb, uint64_t node_cap,
     uint64_t* __restrict__ nodes) {
-  __shared__ uint32_t s_go[kEmitWaves][9];    // group ranges (relative to S)
-  __shared__ uint32_t s_gs3[kEmitWaves][8];   // group subtree sizes
-  __shared__ uint32_t s_gm3[kEmitWaves][8];   // group child masks (non-zero words)
-  __shared__ uint32_t s_wo[kEmitWaves][64];   // word ranges (relative to S)
-  __shared__ uint32_t s_s2[kEmitWaves][64];   // word subtree sizes
-  __shared__ uint32_t s_m2[kEmitWaves][64];   // word child masks (non-zero bytes)
-  __shared__ uint32_t s_vw[kEmitWaves][64];   // voxels before the word in the brick
-  __shared__ uint64_t s_wd[kEmitWaves][64];   // the words
-  __shared__ uint32_t s_bo[kEmitWaves][512];  // byte voxel ranges (relative to S)
-  __shared__ uint64_t s_offs[256];            // offsets_of(m) for every child mask m
-  __shared__ uint8_t s_nth[256][8];           // nth_bit(m, n)
-  {
-    const uint32_t m = threadIdx.x;  // the block has 256 threads: one mask each
-    s_offs[m] = offsets_of(m);
-    uint32_t x = m;
-#pragma unroll
-    for (int n = 0; n < 8; n++) {
-      s_nth[m][n] = (uint8_t)(x ? __ffs(x) - 1 : 0);
-      x &= x - 1;
-    }
-  }
+  __shared__ uint32_t s_inner[kEmitWaves][kInnerMax];  // first child (relative to S) | mask << 16
+  __shared__ uint32_t s_bits[kEmitWaves][kInnerBits + 2];
+  __shared__ uint64_t s_offs[256];  // offsets of every child mask
   const int ws = threadIdx.x / kWave;
   const int lane = lane_id();
   const int g = lane >> 3, q = lane & 7;
   const uint64_t w = (uint64_t)blockIdx.x * kEmitWaves + ws;
   const bool live = w < nb && !M.flag[0];
-  // every wave of the block reaches the barrier below; a wave without a brick works on
-  // zeros and writes nothing
-  // the brick's own words first, then its job and offsets: all in flight while the
-  // offset tables are built
-  uint64_t bc = 0, bvo = 0, S = 0;
-  BrickShape B;
+  // the brick's own words and offsets, in flight while the offset table is built
+  uint64_t word = 0, bc = 0, bvo = 0, S = 0;
   if (live) {
-    B = brick_shape(bwords, w);
+    word = bwords[w * kBrickWords + lane];
     bc = bcode[w];
     bvo = bvoff[w];
     S = A.start[M.off[4] + w];
-  } else {
-    B.word = 0;
-    B.m2 = B.s2 = B.mask3 = B.s3 = B.mask4 = 0;
-    B.s4 = 1;
   }
-  const uint32_t v3 = (q == 0 && B.s3) ? B.s3 - 1u : 0u;
-  const uint32_t inc3 = wave_incl_scan<uint32_t>(v3);
-  // only group heads add to inc3, and every lane of a group knows its group's s3: the
-  // group's exclusive prefix is inc3 less the head's own term
-  const uint32_t pre3 = inc3 - (B.s3 ? B.s3 - 1u : 0u);
-  const uint32_t v2 = B.word ? B.s2 - 1u : 0u;
-  // inclusive scan within each group of 8 lanes (DPP row shifts, lanes whose source lies
-  // in the previous group add nothing)
-  int x2 = (int)v2;
-  {
-    const int o1 = __builtin_amdgcn_update_dpp(0, x2, 0x111, 0xf, 0xf, true);  // row_shr:1
-    x2 += (q >= 1) ? o1 : 0;
-    const int o2 = __builtin_amdgcn_update_dpp(0, x2, 0x112, 0xf, 0xf, true);  // row_shr:2
-    x2 += (q >= 2) ? o2 : 0;
-    const int o4 = __builtin_amdgcn_update_dpp(0, x2, 0x114, 0xf, 0xf, true);  // row_shr:4
-    x2 += (q >= 4) ? o4 : 0;
-  }
-  const uint32_t inc2 = (uint32_t)x2;
-  const uint32_t wo = pre3 + (inc2 - v2);
-  const uint32_t pw = (uint32_t)__popcll(B.word);
-  const uint32_t incw = wave_incl_scan<uint32_t>(pw);
-  if (q == 0) {
-    s_go[ws][g] = pre3;
-    s_gs3[ws][g] = B.s3;
-    s_gm3[ws][g] = B.mask3;
-  }
-  if (lane == 0) s_go[ws][8] = B.s4 - 1u - (uint32_t)__popc(B.mask4);
-  s_wo[ws][lane] = wo;
-  s_s2[ws][lane] = B.s2;
-  s_m2[ws][lane] = B.m2;
-  s_vw[ws][lane] = incw - pw;
-  s_wd[ws][lane] = B.word;
-  uint32_t bo = wo;
+  s_offs[threadIdx.x] = offsets_fast(threadIdx.x);  // the block has 256 threads
+  uint32_t* inner = s_inner[ws];
+  uint32_t* bits = s_bits[ws];
 #pragma unroll
-  for (int j = 0; j < 8; j++) {
-    s_bo[ws][lane * 8 + j] = bo;
-    bo += (uint32_t)__popc((uint32_t)(B.word >> (8 * j)) & 0xFFu);
-  }
+  for (int k = 0; k < (kInnerBits + 2 + kWave - 1) / kWave; k++)
+    if (lane + kWave * k < kInnerBits + 2) bits[lane + kWave * k] = 0u;
   __syncthreads();
   if (!live) return;
+  // the word: its voxels, its non-empty bytes (byte nodes)
+  uint32_t m2 = 0;
+#pragma unroll
+  for (int j = 0; j < 8; j++)
+    if ((word >> (8 * j)) & 0xFFull) m2 |= 1u << j;
+  const uint32_t nv = (uint32_t)__popcll(word), nbz = (uint32_t)__popc(m2);
+  const uint64_t nz = __ballot(word != 0ull);
+  const uint32_t mask3 = (uint32_t)(nz >> (8 * g)) & 0xFFu;  // the group's non-empty words
+  const uint32_t nw = (uint32_t)__popc(mask3);
+  uint32_t mask4 = 0;
+#pragma unroll
+  for (int k = 0; k < 8; k++)
+    if ((nz >> (8 * k)) & 0xFFull) mask4 |= 1u << k;
+  // within the group: records of the words before this one (voxels and byte nodes), and byte
+  // nodes of the words before it (upper half)
+  const uint32_t mine = (nv + nbz) | (nbz << 16);
+  int x = (int)mine;
+  {
+    const int o1 = __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);  // row_shr:1
+    x += (q >= 1) ? o1 : 0;
+    const int o2 = __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);  // row_shr:2
+    x += (q >= 2) ? o2 : 0;
+    const int o4 = __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);  // row_shr:4
+    x += (q >= 4) ? o4 : 0;
+  }
+  const uint32_t before = (uint32_t)x - mine;
+  const uint32_t all = group8_sum(mine);  // of the whole group
+  // over the groups: records of a group's range (its words' and the word nodes), inner nodes
+  const uint32_t grp = ((all & 0xFFFFu) + nw) | (((all >> 16) + nw) << 16);
+  const uint32_t ginc = wave_incl_scan<uint32_t>(q == 0 ? grp : 0u);
+  const uint32_t gpre = ginc - grp;  // (only group heads add; every lane knows its group's term)
+  const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)ginc, kWave - 1);
+  const uint32_t RG = tot & 0xFFFFu;                      // records inside the groups' ranges
+  const uint32_t R = RG + (uint32_t)__popc(mask4);        // records below the brick node
+  const uint32_t go = gpre & 0xFFFFu, gi = gpre >> 16;    // the group's range, its inner nodes
+  const uint32_t wo = go + (before & 0xFFFFu);            // the word's range
+  auto set_bits = [&](uint32_t at, uint32_t n) {          // n <= 8 bits
+    const uint64_t v = (uint64_t)((1u << n) - 1u) << (at & 31u);
+    atomicOr(&bits[at >> 5], (uint32_t)v);
+    if (v >> 32) atomicOr(&bits[(at >> 5) + 1], (uint32_t)(v >> 32));
+  };
+  if (word) {
+    uint32_t i = gi + (before >> 16), vo = wo;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const uint32_t byte = (uint32_t)(word >> (8 * j)) & 0xFFu;
+      if (byte) inner[i++] = vo | (byte << 16);  // its voxels start at vo
+      vo += (uint32_t)__popc(byte);
+    }
+    set_bits(wo + nv, nbz);
+    const uint32_t rank = (uint32_t)__popc(mask3 & ((1u << q) - 1u));
+    inner[gi + (all >> 16) + rank] = (wo + nv) | (m2 << 16);  // the word node
+  }
+  if (q == 0 && mask3) {
+    set_bits(go + (all & 0xFFFFu), nw);
+    const uint32_t rank = (uint32_t)__popc(mask4 & ((1u << g) - 1u));
+    inner[(tot >> 16) + rank] = (go + (all & 0xFFFFu)) | (mask3 << 16);  // the group node
+  }
+  if (lane == 0) set_bits(RG, R - RG);
+  wave_lds_sync();
   const JobDev& J = jobs[T.job(bc)];
-  const uint64_t vox0 = bvo - J.voff;
-  const uint32_t R = B.s4 - 1u;        // records below the brick node
-  const uint32_t RG = s_go[ws][8];     // records inside the groups' ranges
   if (S + R > J.n_nodes || J.nbase + S + R > node_cap) {
     if (lane == 0) M.flag[1] = 1;
     return;
@@ -696,55 +699,34 @@ __global__ __launch_bounds__(kWave * kEmitWaves) void k_emit_bricks(
   uint64_t* out = nodes + 3 * (J.nbase + S);
   const int payload = J.payload;
   // the job's placement, read once (the record stores below could alias the job table)
-  const uint64_t cb_add = kPlaced ? J.cb_add : 0, data_add = kPlaced ? J.data_add : 0;
-  const uint64_t d_hdr = payload ? 1ull : 2ull;
-  for (uint32_t r = lane; r < R; r += kWave) {
-    // find the record's node: its child mask m (internal nodes) and the first two words
-    uint64_t d0 = 0, d1;
-    uint32_t m;
-    bool leaf = false;
-    if (r >= RG) {  // a group node
-      const int gg = s_nth[B.mask4][r - RG];
-      m = s_gm3[ws][gg];
-      d1 = S + s_go[ws][gg] + s_gs3[ws][gg] - 1u - (uint32_t)__popc(m);
-    } else {
-      const int gg = last_le8(s_go[ws], r);
-      const uint32_t m3 = s_gm3[ws][gg];
-      const uint32_t r1 = r - s_go[ws][gg];
-      const uint32_t l3 = s_gs3[ws][gg] - 1u, nw = (uint32_t)__popc(m3);
-      if (r1 >= l3 - nw) {  // a word node
-        const int ww = gg * 8 + s_nth[m3][r1 - (l3 - nw)];
-        m = s_m2[ws][ww];
-        d1 = S + s_wo[ws][ww] + s_s2[ws][ww] - 1u - (uint32_t)__popc(m);
+  const uint64_t cb0 = S + (kPlaced ? J.cb_add : 0);
+  // the first voxel's data index; geometry-only voxels share record 1
+  uint64_t leaf0 = payload ? 1ull + (bvo - J.voff) : 1ull;
+  if (kPlaced && leaf0 >= (payload ? 1ull : 2ull)) leaf0 += J.data_add;
+  uint32_t prior = 0;  // inner nodes before the window
+  for (uint32_t r0 = 0; r0 < R; r0 += kWave) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)bits[r0 >> 5]);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)bits[(r0 >> 5) + 1]);
+    const uint32_t below = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+    const bool is_inner = ((lane < 32 ? lo : hi) >> (lane & 31)) & 1u;
+    const uint32_t r = r0 + lane;
+    if (r < R) {
+      uint64_t d0, d1, d2;
+      if (is_inner) {
+        const uint32_t e = inner[prior + below];
+        d0 = 0;
+        d1 = cb0 + (e & 0xFFFFu);
+        d2 = s_offs[e >> 16];
       } else {
-        const int ww = gg * 8 + last_le8(&s_wo[ws][gg * 8], r);
-        const uint32_t m2 = s_m2[ws][ww];
-        const uint32_t r2 = r - s_wo[ws][ww];
-        const uint32_t l2 = s_s2[ws][ww] - 1u, nbz = (uint32_t)__popc(m2);
-        const uint64_t word = s_wd[ws][ww];
-        if (r2 >= l2 - nbz) {  // a byte node: its voxels start at its own range start
-          const int j = s_nth[m2][r2 - (l2 - nbz)];
-          m = (uint32_t)(word >> (8 * j)) & 0xFFu;
-          d1 = S + s_bo[ws][ww * 8 + j];
-        } else {  // a voxel
-          const int j = last_le8(&s_bo[ws][ww * 8], r);
-          const uint32_t k = r - s_bo[ws][ww * 8 + j];
-          const uint32_t before = (uint32_t)__popcll(word & ((1ull << (8 * j)) - 1ull));
-          d0 = payload ? 1ull + vox0 + s_vw[ws][ww] + before + k : 1ull;
-          d1 = 0;
-          m = 0;
-          leaf = true;
-        }
+        d0 = leaf0 + (payload ? r - prior - below : 0u);
+        d1 = 0;
+        d2 = ~0ull;
       }
+      out[3 * (uint64_t)r] = d0;
+      out[3 * (uint64_t)r + 1] = d1;
+      out[3 * (uint64_t)r + 2] = d2;
     }
-    const uint64_t d2 = leaf ? ~0ull : s_offs[m];
-    if constexpr (kPlaced) {
-      d0 = d0 >= d_hdr ? d0 + data_add : d0;
-      d1 = leaf ? d1 : d1 + cb_add;
-    }
-    out[3 * (uint64_t)r] = d0;
-    out[3 * (uint64_t)r + 1] = d1;
-    out[3 * (uint64_t)r + 2] = d2;
+    prior += (uint32_t)__popc(lo) + (uint32_t)__popc(hi);
   }
 }
 
