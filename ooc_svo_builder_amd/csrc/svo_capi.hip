@@ -201,10 +201,8 @@ static bool on_device(const Context& c, const void* p, size_t bytes) {
 // copy command and a stream synchronization).
 static hipError_t copy_sync(Context& c, void* dst, const void* src, size_t bytes) {
   if (!bytes) return hipSuccess;
-  if (bytes % 8 == 0 && (uintptr_t)src % 8 == 0 && on_device(c, dst, bytes)) {
-    hipError_t e = copy_records(c, dst, src, bytes);
-    return e == hipSuccess ? read_back(c, nullptr, 0) : e;
-  }
+  if (bytes % 8 == 0 && (uintptr_t)src % 8 == 0 && on_device(c, dst, bytes))
+    return copy_records(c, dst, src, bytes);
   hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, c.stream);
   if (e != hipSuccess) return e;
   return stream_sync(c.stream);
@@ -276,6 +274,7 @@ int svo_ctx_create(int device, svo_ctx** out) {
   }
   ctx->c.own_stream = true;
   if ((e = ensure(ctx->c.counters, kNumCounters * 8)) != hipSuccess ||
+      (e = fill_u64(ctx->c.counters.as<uint64_t>(), 0, kNumCounters, ctx->c.stream)) != hipSuccess ||
       (e = hipEventCreate(&ctx->c.ev0)) != hipSuccess ||
       (e = hipEventCreate(&ctx->c.ev1)) != hipSuccess ||
       (e = hipEventCreate(&ctx->c.ev2)) != hipSuccess ||

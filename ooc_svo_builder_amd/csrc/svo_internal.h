@@ -107,6 +107,7 @@ enum Counter : int {
   kCtrError = 15,     // sticky: internal consistency failures (cleared per job)
   kCtrPartTotal = 16, // partition list length
   kCtrStamp = 17,     // device clock at the start of the pass
+  kCtrCopyDone = 18,  // finished blocks of a copy that raises the read-back flag (0 between copies)
   kNumCounters = 32
 };
 constexpr int kCtrPassClear = 15;  // counters 0..14 are cleared at the start of a pass
@@ -447,7 +448,8 @@ struct ReadReq {
 };
 hipError_t read_back(Context& c, const ReadReq* reqs, int n);
 
-// Device-to-device copy on c.stream by a kernel; pointers and size are multiples of 8 bytes.
+// Device-to-device copy on c.stream by a kernel, waited for; pointers and size are multiples of 8
+// bytes.
 hipError_t copy_records(Context& c, void* dst, const void* src, size_t bytes);
 
 // Stage drivers (return hipSuccess or an error; message in last error).
