@@ -264,23 +264,25 @@ struct ActArgs {
   uint64_t pool_cap;  // touch path slots
 };
 
+// What an action keeps per wave in LDS.
+struct NoCache {};
+
 // Brick allocation without atomics: the touch pass stores 1 into the table entry of
 // every brick a column's candidate voxels fall in; a scan over the table then numbers the
 // flagged bricks in Morton order (table entry = slot + 1) and lists them.
 struct TouchAction {
   static constexpr bool kTouch = true;
-  // the same action for lanes in no order of their triangles (queued columns)
   using Unordered = TouchAction;
-  // whether a direct walk narrows its rows to their intervals
+  using Cache = NoCache;
   __device__ static bool narrow(const VoxParams&) { return true; }
   uint32_t* table;
   uint64_t brick0;  // first brick of the unit's table segment
-  __device__ static TouchAction make(const ActArgs& A, const VoxParams& P) {
+  __device__ static TouchAction make(const ActArgs& A, const VoxParams& P, Cache*) {
     return TouchAction{A.table + P.table_base, P.bstart >> kBrickBits};
   }
   __device__ __forceinline__ void touch(uint64_t brick_code) { table[brick_code - brick0] = 1u; }
   __device__ __forceinline__ void add(uint64_t, uint32_t) {}
-  __device__ __forceinline__ void flush() {}
+  __device__ static void drain(const ActArgs&, const VoxParams&, Cache*, bool) {}
 };
 
 // Mark voxels with plain byte stores of 1: concurrent marks of one voxel all store the
@@ -298,22 +300,22 @@ struct TouchAction {
 //    (touch pass + table scan), cached per thread.
 // Both store through global (not generic) pointers.
 // kWide: some units of the pass carry payload (4-byte cells; the unit's wide flag decides
-// per voxel); otherwise every cell is a byte. kLaneOrder: the lanes of a wave hold
-// non-decreasing triangle indices (the small tier: tile order, item order), and a lane
-// checks its left neighbour before the atomic; not so in the large tier, whose list is in
-// collection order.
-template <bool kWide, bool kLaneOrder = true>
+// per voxel); otherwise every cell is a byte.
+template <bool kWide>
 struct MarkDenseT {
   static constexpr bool kTouch = false;
-  using Unordered = MarkDenseT<kWide, false>;
-  __device__ static bool narrow(const VoxParams& P) { return !kWide || (!kLaneOrder && !P.wide); }
+  // the same action for lanes in no order of their triangles (queued columns)
+  using Unordered = MarkDenseT<kWide>;
+  using Cache = NoCache;  // per wave, in LDS
+  // whether a direct walk narrows its rows to their intervals
+  __device__ static bool narrow(const VoxParams& P) { return !kWide || !P.wide; }
   gbyte_t* table;  // the unit's table segment, a byte per quarter of a brick
   gbyte_t* words;  // the unit's word flags (payload units)
   gbyte_t* bytes;
   uint64_t base;  // code of the first voxel of the unit's first brick
   int wide;
   uint32_t cquarter = 0xFFFFFFFFu, cword = 0xFFFFFFFFu;  // the last ones marked
-  __device__ static MarkDenseT make(const ActArgs& A, const VoxParams& P) {
+  __device__ static MarkDenseT make(const ActArgs& A, const VoxParams& P, Cache*) {
     MarkDenseT m;
     m.table = (gbyte_t*)(A.table + P.table_base);
     m.words = (gbyte_t*)(A.cflags + P.table_base * kBrickWords);
@@ -327,23 +329,9 @@ struct MarkDenseT {
     const uint64_t rel = code - base;
     const uint32_t q = (uint32_t)(rel >> (kBrickBits - 2));
     if (kWide && wide) {
-      // the lowest covering triangle as the largest ~tri (0 = unmarked). With kLaneOrder
-      // a lane whose left neighbour marks the same cell in the same step holds a triangle
-      // no lower than the neighbour's and leaves the atomic to it: on fine meshes
-      // neighbouring triangles cover the same voxels
-      gword_t* cell = (gword_t*)bytes + rel;
-      bool dup = false;
-      if (kLaneOrder) {
-        const uint64_t addr = (uint64_t)cell;
-        const uint64_t act = __ballot(1);
-        const int ln = lane_id();
-        const uint32_t plo = (uint32_t)__shfl_up((int)(uint32_t)addr, 1, kWave);
-        const uint32_t phi = (uint32_t)__shfl_up((int)(uint32_t)(addr >> 32), 1, kWave);
-        dup = ln > 0 && ((act >> (ln - 1)) & 1ull) && plo == (uint32_t)addr &&
-              phi == (uint32_t)(addr >> 32);
-      }
-      if (!dup)
-        __hip_atomic_fetch_max(cell, ~tri, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      // the lowest covering triangle as the largest ~tri (0 = unmarked)
+      __hip_atomic_fetch_max((gword_t*)bytes + rel, ~tri, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
       const uint32_t w = (uint32_t)(rel >> 6);
       if (w != cword) {
         cword = w;
@@ -356,15 +344,105 @@ struct MarkDenseT {
       table[q] = 1;
     }
   }
-  __device__ __forceinline__ void flush() {}
+  __device__ static void drain(const ActArgs&, const VoxParams&, Cache*, bool) {}
 };
 using MarkDenseAction = MarkDenseT<false>;
 using MarkDenseWideAction = MarkDenseT<true>;
-using MarkDenseWideBatchAction = MarkDenseT<true, false>;
+
+// Payload marks of one mesh, gathered in LDS: a wave keeps kLines lines of 32 cells (128 bytes
+// of the grid), takes the maximum of ~triangle there, and gives a line to memory whole, a half
+// wave a line. A cell whose line's place holds another line goes to memory at once.
+//
+// The winner atomics bound these marks: at agent scope they are not done in the (per XCD) L2
+// but at the memory behind it, ~23 G requests a second whatever they hold (TCC_EA0_ATOMIC =
+// TCC_ATOMIC; 12.7 M of them for 17M voxels of a rough sphere at 1024 in 535 us, 4.3 M for a
+// fine terrain in 218), so what counts is how many requests there are, and neighbouring
+// triangles share both cells and lines.
+constexpr uint32_t kLineBits = 5;
+constexpr uint32_t kLineCells = 1u << kLineBits;
+constexpr uint32_t kLines = 64;
+constexpr uint32_t kLinesFull = 40;  // lines held at which a wave gives them to memory
+struct MarkLines {
+  uint32_t tag[kLines];  // line + 1, 0 = free
+  uint32_t val[kLines][kLineCells];
+};
+struct MarkGatherAction {
+  static constexpr bool kTouch = false;
+  using Unordered = MarkDenseWideAction;
+  using Cache = MarkLines;
+  __device__ static bool narrow(const VoxParams&) { return false; }
+  gbyte_t* table;
+  gbyte_t* words;
+  gword_t* cells;
+  uint64_t base;
+  MarkLines* L;
+  __device__ static MarkGatherAction make(const ActArgs& A, const VoxParams& P, Cache* L) {
+    MarkGatherAction m;
+    m.table = (gbyte_t*)(A.table + P.table_base);
+    m.words = (gbyte_t*)(A.cflags + P.table_base * kBrickWords);
+    m.cells = (gword_t*)P.grid8;
+    m.base = P.bstart;
+    m.L = L;
+    return m;
+  }
+  __device__ __forceinline__ void touch(uint64_t) {}
+  __device__ __forceinline__ void add(uint64_t code, uint32_t tri) {
+    const uint64_t rel = code - base;  // (below 2^35: the dense limit is 2^37 bytes)
+    const uint32_t line = (uint32_t)(rel >> kLineBits);
+    // neighbouring lines in neighbouring places (of a 4 x 4 x 4 block of lines: 6 bits), the
+    // blocks mixed
+    const uint32_t at = (line ^ ((line >> 6) * 0x9E3779B1u >> 26)) % kLines;
+    uint32_t tag = L->tag[at];
+    if (tag == 0u) {
+      tag = atomicCAS(&L->tag[at], 0u, line + 1u);
+      if (tag == 0u) tag = line + 1u;
+    }
+    if (tag == line + 1u) {
+      atomicMax(&L->val[at][(uint32_t)rel % kLineCells], ~tri);
+    } else {
+      __hip_atomic_fetch_max(cells + rel, ~tri, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      words[line >> 1] = 1;
+      table[line >> (kBrickBits - 2 - kLineBits)] = 1;
+    }
+  }
+  // Give the lines to memory (all: else only when there are many). Called by whole waves.
+  __device__ static void drain(const ActArgs& A, const VoxParams& P, Cache* L, bool all) {
+    const int lane = lane_id();
+    wave_lds_sync();
+    const uint32_t tag = L->tag[lane];
+    uint64_t used = __ballot(tag != 0u);
+    if (!used || (!all && (uint32_t)__popcll(used) < kLinesFull)) return;  // uniform
+    const MarkGatherAction m = make(A, P, L);
+    while (used) {  // two lines at a time
+      const int l0 = __ffsll((long long)used) - 1;
+      used &= used - 1ull;
+      const int l1 = used ? __ffsll((long long)used) - 1 : -1;
+      used &= used - 1ull;
+      const int at = lane < kWave / 2 ? l0 : l1;
+      const uint32_t line = (uint32_t)__shfl((int)tag, at & (kWave - 1), kWave) - 1u;
+      if (at >= 0) {
+        const uint32_t cell = (uint32_t)lane % kLineCells;
+        const uint32_t v = L->val[at][cell];
+        L->val[at][cell] = 0u;
+        if (v)
+          __hip_atomic_fetch_max(m.cells + (((uint64_t)line << kLineBits) + cell), v,
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (cell == 0) {
+          m.words[line >> 1] = 1;
+          m.table[line >> (kBrickBits - 2 - kLineBits)] = 1;
+        }
+      }
+    }
+    L->tag[lane] = 0u;
+    wave_lds_sync();
+  }
+};
+static_assert(kLines == kWave && kLineCells == kWave / 2, "drain: a place a lane, two lines a step");
 
 struct MarkPoolAction {
   static constexpr bool kTouch = false;
   using Unordered = MarkPoolAction;
+  using Cache = NoCache;
   __device__ static bool narrow(const VoxParams&) { return true; }
   const gword_t* table;
   gbyte_t* bytes;  // the slot pool
@@ -372,7 +450,7 @@ struct MarkPoolAction {
   uint64_t pool_cap;
   uint64_t base;  // code of the first voxel of the unit's first brick
   uint32_t cbrick = 0xFFFFFFFFu, cslot = 0;
-  __device__ static MarkPoolAction make(const ActArgs& A, const VoxParams& P) {
+  __device__ static MarkPoolAction make(const ActArgs& A, const VoxParams& P, Cache*) {
     MarkPoolAction m;
     m.table = (const gword_t*)(A.table + P.table_base);
     m.bytes = (gbyte_t*)A.pool8;
@@ -398,13 +476,14 @@ struct MarkPoolAction {
     }
     bytes[(uint64_t)(s - 1) * kBrickVox + (rel & (kBrickVox - 1))] = 1;
   }
-  __device__ __forceinline__ void flush() {}
+  __device__ static void drain(const ActArgs&, const VoxParams&, Cache*, bool) {}
 };
 
 // Second payload pass: lowest triangle index per voxel rank.
 struct WinnerAction {
   static constexpr bool kTouch = false;
   using Unordered = WinnerAction;
+  using Cache = NoCache;
   __device__ static bool narrow(const VoxParams&) { return false; }
   const uint32_t* table;
   const ull* pool;  // bit form of the bricks, written by the compaction
@@ -412,7 +491,7 @@ struct WinnerAction {
   uint32_t* winner;
   ull* ctr;
   uint64_t base;  // code of the first voxel of the unit's first brick
-  __device__ static WinnerAction make(const ActArgs& A, const VoxParams& P) {
+  __device__ static WinnerAction make(const ActArgs& A, const VoxParams& P, Cache*) {
     return WinnerAction{A.table + P.table_base, A.pool, A.wprefix, A.winner, A.ctr, P.bstart};
   }
   __device__ __forceinline__ void touch(uint64_t) {}
@@ -432,7 +511,7 @@ struct WinnerAction {
     const uint32_t rank = wprefix[slot] + (uint32_t)__popcll(pool[slot] & (bit - 1ull));
     atomicMin(&winner[rank], tri);
   }
-  __device__ __forceinline__ void flush() {}
+  __device__ static void drain(const ActArgs&, const VoxParams&, Cache*, bool) {}
 };
 
 // last k with a[k] <= v, for a non-decreasing a[0..n) with a[0] <= v
@@ -528,18 +607,18 @@ __device__ __forceinline__ void walk_queued(const VoxParams& P, const ActArgs& A
 #pragma unroll
   for (int f = 0; f < kWalkI; f++) Q.i[f] = __shfl(K.i[f], src, kWave);
   if ((uint32_t)lane_id() >= n) return;
-  typename Act::Unordered act = Act::Unordered::make(A, P);
+  typename Act::Unordered act = Act::Unordered::make(A, P, nullptr);
   const uint32_t col = e & kColMask, na = (uint32_t)(Q.i[I_G1U] - Q.i[I_G0U] + 1);
   const int a = Q.i[I_G0U] + (int)(col % na);
   walk_row_span<false>(Q, P, Q.i[I_G0V] + (int)(row0 + col / na), a, a, act);
-  act.flush();
 }
 
 // Rows [row0, row0 + nrows) of the lanes' triangles (nall rows each; their walks K, their linear forms in
 // L.tri).
 template <typename Act>
-__device__ __forceinline__ void walk_rows(WalkLds& L, const VoxParams& P, const ActArgs& A,
-                                          const Walk& K, uint32_t nall, uint32_t nrows, uint32_t row0) {
+__device__ __forceinline__ void walk_rows(WalkLds& L, typename Act::Cache* cache,
+                                          const VoxParams& P, const ActArgs& A, const Walk& K,
+                                          uint32_t nall, uint32_t nrows, uint32_t row0) {
   uint32_t nq = 0;
   const int lane = lane_id();
   const uint32_t rend = wave_incl_scan<uint32_t>(nrows), rstart = rend - nrows;
@@ -575,7 +654,7 @@ __device__ __forceinline__ void walk_rows(WalkLds& L, const VoxParams& P, const 
     const uint32_t C = (uint32_t)__builtin_amdgcn_readlane((int)cend, kWave - 1);
     L.row[lane][0].x = cstart;
     uint32_t ccarry = 0;
-    Act act = Act::make(A, P);
+    Act act = Act::make(A, P, cache);
     for (uint32_t k0 = 0; k0 < C; k0 += kWave) {
       const uint32_t rr = locate(L.slot, cstart, cnt != 0, k0, ccarry);  // (orders the row stores)
       const uint32_t k = k0 + lane;
@@ -619,6 +698,7 @@ __device__ __forceinline__ void walk_rows(WalkLds& L, const VoxParams& P, const 
           }
         }
       }
+      Act::drain(A, P, cache, false);
       const uint64_t pm = __ballot(push);
       if (pm) {  // uniform
         if (push) L.q[nq + (uint32_t)__popcll(pm & ((1ull << lane) - 1ull))] = e;
@@ -631,7 +711,6 @@ __device__ __forceinline__ void walk_rows(WalkLds& L, const VoxParams& P, const 
         }
       }
     }
-    act.flush();
     wave_lds_sync();  // the next rows overwrite these
   }
   if (nq) walk_queued<Act>(P, A, K, row0, L.q, nq);
@@ -668,8 +747,11 @@ __device__ __forceinline__ uint32_t large_jobs(const LargeList& B, ull* ctr, uin
   return fits ? rows : rows | kAllRows;
 }
 
+// blocks of the small tier on a CU (what an action keeps in LDS leaves room for two)
 template <typename Act>
-__global__ __launch_bounds__(kTile, 4) void k_vox_tile(const VoxParams* __restrict__ units,
+constexpr int kTileBlocks = std::is_same<typename Act::Cache, NoCache>::value ? 4 : 2;
+template <typename Act>
+__global__ __launch_bounds__(kTile, kTileBlocks<Act>) void k_vox_tile(const VoxParams* __restrict__ units,
                                                        uint32_t n_units,
                                                        const uint32_t* __restrict__ tile_off,
                                                        ActArgs A, ull* queue, LargeList B,
@@ -680,6 +762,13 @@ __global__ __launch_bounds__(kTile, 4) void k_vox_tile(const VoxParams* __restri
   fill_spread_table();
   __syncthreads();  // the waves part here
   WalkLds& L = s_walk[threadIdx.x / kWave];
+  typename Act::Cache* cache = nullptr;
+  if constexpr (!std::is_same<typename Act::Cache, NoCache>::value) {
+    __shared__ typename Act::Cache s_cache[kTileWaves];
+    cache = &s_cache[threadIdx.x / kWave];
+    for (uint32_t k = lane_id(); k < sizeof(*cache) / 4; k += kWave) ((uint32_t*)cache)[k] = 0u;
+    wave_lds_sync();
+  }
   ull* ctr = A.ctr;
   const int lane = lane_id();
   const uint32_t total = tile_off[n_units];
@@ -768,15 +857,16 @@ __global__ __launch_bounds__(kTile, 4) void k_vox_tile(const VoxParams* __restri
     }
     if (direct) {
       if (ncols) {
-        Act act = Act::make(A, P);
+        Act act = Act::make(A, P, cache);
         walk_all_columns(K, P, act, Act::narrow(P));
-        act.flush();
       }
+      Act::drain(A, P, cache, true);
       continue;
     }
     if (__ballot(rows != 0)) {
       wave_lds_sync();
-      walk_rows<Act>(L, P, A, K, nv, rows, 0u);
+      walk_rows<Act>(L, cache, P, A, K, nv, rows, 0u);
+      Act::drain(A, P, cache, true);
     }
   }
 }
@@ -833,7 +923,7 @@ __global__ __launch_bounds__(kTile, 3) void k_vox_large(const VoxParams* __restr
     const uint32_t nb = (uint32_t)(K.i[I_G1V] - K.i[I_G0V] + 1);
     const uint32_t rows = B.rows[idx] & ~kAllRows;
     do {
-      walk_rows<Act>(L, P, A, K, nb, lane == 0 ? min(rows, nb - row0) : 0u, row0);
+      walk_rows<Act>(L, nullptr, P, A, K, nb, lane == 0 ? min(rows, nb - row0) : 0u, row0);
       row0 += rows;
     } while ((B.rows[idx] & kAllRows) && row0 < nb);
   }
@@ -2009,21 +2099,19 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
       }
       // first pass: dense units mark directly, touch units flag their bricks; both collect
       // the large triangles
-      // payload passes: the lane-neighbour check before the atomic pays on one mesh (a fine
-      // payload terrain at 1024: mark 357 -> 213 us) but cost the 512-mesh batched mix 11%
       if (dense && geometry_only)
         SVO_TRY(tile_pass(MarkDenseAction{}, "vox_small_mark", queues, 1, 0));
       else if (dense && nu == 1)
-        SVO_TRY(tile_pass(MarkDenseWideAction{}, "vox_small_mark", queues, 1, 0));
+        SVO_TRY(tile_pass(MarkGatherAction{}, "vox_small_mark", queues, 1, 0));
       else if (dense)
-        SVO_TRY(tile_pass(MarkDenseWideBatchAction{}, "vox_small_mark", queues, 1, 0));
+        SVO_TRY(tile_pass(MarkDenseWideAction{}, "vox_small_mark", queues, 1, 0));
       else
         SVO_TRY(tile_pass(TouchAction{}, "vox_small_touch", queues, 1, 0));
       if (dense) {
         if (geometry_only)
           SVO_TRY(large_pass(MarkDenseAction{}, "vox_large_mark", 0));
-        else  // (the large tier's lanes are not in triangle order)
-          SVO_TRY(large_pass(MarkDenseWideBatchAction{}, "vox_large_mark", 0));
+        else
+          SVO_TRY(large_pass(MarkDenseWideAction{}, "vox_large_mark", 0));
         // number the flagged bricks in Morton order: table entry = rank + 1, occ = list
         SVO_TRY(occ_scan());
       } else {
