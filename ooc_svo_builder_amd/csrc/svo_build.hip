@@ -279,11 +279,9 @@ __device__ __forceinline__ void job_bases(JobDev* jobs, uint32_t n_jobs,
                                           const unsigned long long* root_size,
                                           const unsigned long long* root_isize,
                                           const unsigned long long* brick_hazard,
-                                          const uint64_t* __restrict__ codes, Tags T,
-                                          LevelMeta M, uint64_t node_cap,
-                                          uint64_t* __restrict__ nodes,
-                                          const float* __restrict__ in_rec,
-                                          float* __restrict__ records, uint64_t* wsum,
+                                          const uint64_t* codes, Tags T, LevelMeta M,
+                                          uint64_t node_cap, uint64_t* nodes,
+                                          const float* in_rec, float* records, uint64_t* wsum,
                                           uint64_t& carry) {
   if (threadIdx.x == 0) carry = 0;
   __syncthreads();
@@ -991,6 +989,227 @@ __global__ __launch_bounds__(256) void k_up_finish(Arena A, LevelMeta M, Tags T,
   }
 }
 
+// All of the above for few bricks, in one block and one launch, the nodes in LDS: the build's
+// bookkeeping (k_build_init), the upper levels, the per-job bases (k_levels_tail) and the upper
+// nodes' records (k_emit_upper). A thread is a brick, then a node.
+//
+// Bound by its chain of accesses, as are the seven launches it replaces (2 to 5 us each whatever
+// they do; with the nodes in global memory one launch of it took 14 us for 40 bricks, 21 for 900,
+// no less than they did).
+constexpr uint32_t kSmallNodes = 2816;  // nodes of heights 4 .. H, at most
+struct SmallNode {
+  uint64_t code;
+  uint32_t a;          // A_l of its first brick, then its start
+  uint32_t size, sib;
+  uint16_t first, pidx;
+};
+__global__ __launch_bounds__(kTailBlock) void k_up_small(
+    uint64_t* __restrict__ start, LevelMeta M, Tags T, JobDev* jobs, uint32_t n_jobs,
+    const uint64_t* __restrict__ bwords, const uint64_t* __restrict__ bcode,
+    const uint32_t* __restrict__ bshape, uint32_t NB, int H, uint64_t meta_words, int put,
+    JobDev j0, unsigned long long* root_size, unsigned long long* root_isize,
+    unsigned long long* hazard, uint64_t* job_end, uint64_t node_cap, uint64_t* nodes,
+    float* records) {
+  constexpr int kWaves = kTailBlock / kWave;
+  __shared__ SmallNode s_node[kSmallNodes];
+  __shared__ uint8_t s_mask[kSmallNodes];
+  __shared__ uint32_t s_cnt[kUpLevels], s_off[kUpLevels + 2], wpre[kWaves][kUpLevels];
+  __shared__ uint32_t s_end[kUpLevels];  // one job: A_l at its end
+  __shared__ uint32_t ws4[kWaves], s_hazard;
+  __shared__ uint64_t s_scan[kWaves], s_carry;
+  const int w = threadIdx.x / kWave, lane = lane_id();
+  const uint64_t le = (2ull << lane) - 1ull;  // lanes <= this one
+  const bool tagged = T.tag_mask != 0ull;
+  const unsigned long long now = wall_clock64();
+  for (uint64_t i = threadIdx.x; i < meta_words; i += kTailBlock)
+    M.n[i] = i == (uint64_t)kStampWord ? now : 0ull;
+  if (put && threadIdx.x == 0) *jobs = j0;
+  if (threadIdx.x == 0) s_hazard = 0;
+  const uint32_t i = threadIdx.x;
+  const bool live = i < NB;
+  uint64_t c0 = 0, c = 0, cp = 0;
+  uint32_t sh = 0, jb = 0;
+  int D = 4, t = 4;
+  if (live) {
+    c0 = bcode[i];
+    sh = bshape[i];
+    c = brick_node_code(c0, T);
+    if (i) cp = brick_node_code(bcode[i - 1], T);
+    jb = T.job(c0);
+    D = tagged ? jobs[jb].depth : j0.depth;
+    t = brick_top(c, cp, i > 0, T, D);
+  }
+  const uint32_t s4 = sh & 0xFFFFu;
+  for (int k = 0; 5 + k <= H; k++) {
+    const uint64_t m = __ballot(t >= 5 + k);
+    if (lane == 0) wpre[w][k] = (uint32_t)__popcll(m);
+  }
+  const uint32_t s4i = wave_incl_scan<uint32_t>(s4);
+  if (lane == kWave - 1) ws4[w] = s4i;
+  __syncthreads();
+  if (threadIdx.x < kWave) {  // exclusive prefixes over the waves, per height; the heights' offsets
+    uint32_t n = 0;
+    if (5 + lane <= H)
+      for (int q = 0; q < kWaves; q++) {
+        const uint32_t x = wpre[q][lane];
+        wpre[q][lane] = n;
+        n += x;
+      }
+    const uint32_t inc = wave_incl_scan<uint32_t>(n);
+    if (5 + lane <= H) {
+      s_cnt[lane] = n;
+      s_off[lane + 2] = NB + inc;
+    }
+    if (lane == 0) {
+      s_off[0] = 0;
+      s_off[1] = NB;
+    }
+  }
+  uint32_t S4 = s4i - s4, all4 = 0;
+  for (int q = 0; q < kWaves; q++) {
+    if (q < w) S4 += ws4[q];
+    all4 += ws4[q];
+  }
+  __syncthreads();
+  // s_off[l - 4]: first node of height l
+  const uint32_t total = s_off[H - 3];
+  if (live) {
+    SmallNode& B = s_node[i];
+    B.code = c;
+    B.a = S4;
+    B.size = s4;
+    B.first = 0;
+    s_mask[i] = (uint8_t)(sh >> 16);
+    const uint64_t G = tagged ? jobs[jb].gridsize : j0.gridsize;
+    if ((c0 & ~T.tag_mask) == G * G * G - kBrickVox &&
+        (bwords[(uint64_t)i * kBrickWords + kWave - 1] >> 62) == 1ull) {
+      if (tagged) hazard[jb] = 1;
+      s_hazard = 1;
+    }
+  }
+  {
+    const uint64_t tag = c & T.tag_mask, rest = c & ~T.tag_mask;
+    const bool job_first = live && i && (cp & T.tag_mask) != tag;
+    uint32_t a = S4, a_end = all4;
+    uint32_t below = i;  // its ancestor's index a height down
+    for (int k = 0; 5 + k <= H; k++) {
+      const int l = 5 + k;
+      const uint64_t m = __ballot(t >= l);  // (all lanes)
+      const uint32_t incl = wpre[w][k] + (uint32_t)__popcll(m & le);
+      const bool head = t >= l;
+      a += incl - (head ? 1u : 0u);  // A_l(i)
+      a_end += s_cnt[k];             // A_l at the end
+      if (live) {
+        // the node it heads a height down learns its parent
+        if (t >= l - 1 && l <= D) s_node[s_off[k] + below].pidx = (uint16_t)(incl - 1u);
+        if (head && l <= D) {
+          SmallNode& P = s_node[s_off[k + 1] + incl - 1u];
+          P.code = tag | (rest >> (3 * (l - 4)));
+          P.first = (uint16_t)below;
+          P.a = a;
+        }
+        if (job_first) job_end[(uint64_t)T.job(cp) * kUpLevels + k] = a;
+        if (i == NB - 1) {
+          if (tagged) job_end[(uint64_t)jb * kUpLevels + k] = a_end;
+          s_end[k] = a_end;
+        }
+      }
+      below = incl - 1u;
+    }
+  }
+  __syncthreads();
+  auto height = [&](uint32_t g) {
+    int l = 4;
+    while (g >= s_off[l - 3]) l++;
+    return l;
+  };
+  for (uint32_t g = threadIdx.x; g < total; g += kTailBlock) {  // sizes, masks, sibling offsets
+    const int l = height(g);
+    const uint32_t co = s_off[l - 4], n = s_off[l - 3] - co, j = g - co;
+    SmallNode& P = s_node[g];
+    const uint64_t code = P.code;
+    const uint32_t job = T.job(code);
+    const int Dj = tagged ? jobs[job].depth : j0.depth;
+    if (l >= 5) {
+      const bool last = j + 1 == n || T.job(s_node[g + 1].code) != job;
+      const uint32_t a1 = !last ? s_node[g + 1].a
+                          : tagged ? (uint32_t)job_end[(uint64_t)job * kUpLevels + (l - 5)]
+                                   : s_end[l - 5];
+      P.size = a1 - P.a;
+      const uint32_t cco = s_off[l - 5], nch = co - cco, f = P.first;
+      uint32_t m = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < 8; k++) {
+        const uint64_t cc = s_node[cco + min(f + k, nch - 1u)].code;
+        if (f + k < nch && T.parent(cc) == code) m |= 1u << (cc & 7);
+      }
+      s_mask[g] = (uint8_t)m;
+    }
+    if (l == Dj && tagged) root_size[job] = P.size;
+    if (l < Dj) {
+      const uint32_t f = s_node[s_off[l - 3] + P.pidx].first;
+      P.sib = P.a - s_node[co + f].a - (j - f);
+    }
+  }
+  __syncthreads();
+  uint32_t n_nodes = 0;
+  if (tagged) {
+    job_bases<kTailBlock>(jobs, n_jobs, root_size, root_isize, hazard, nullptr, T, M, node_cap,
+                          nodes, records, records, s_scan, s_carry);
+    __syncthreads();
+  } else {  // one job, not trivial (it has bricks): job_bases' results
+    n_nodes = s_node[total - 1].size;
+    if (threadIdx.x == 0) {
+      jobs->n_nodes = n_nodes;
+      jobs->nbase = 0;
+      jobs->hazard = s_hazard;
+      jobs->n_data = j0.payload ? 1 + j0.nvox : 2;
+      M.flag[2] = n_nodes;
+    }
+    // the null record, and the white one of geometry-only builds
+    if (threadIdx.x < (j0.payload ? 8u : 16u))
+      records[j0.dbase * 8 + threadIdx.x] =
+          threadIdx.x >= 10 && threadIdx.x < 13 ? 1.0f : 0.0f;
+  }
+  for (uint32_t g = threadIdx.x; g < total; g += kTailBlock) {  // records
+    int l = height(g);
+    const uint32_t j = g - s_off[l - 4];
+    const SmallNode& P = s_node[g];
+    const uint32_t cm = s_mask[g];
+    uint64_t nbase = 0, nn = n_nodes, cb_add = j0.cb_add;
+    int Dj = j0.depth;
+    if (tagged) {
+      const JobDev& J = jobs[T.job(P.code)];
+      nbase = J.nbase;
+      nn = J.n_nodes;
+      cb_add = J.cb_add;
+      Dj = J.depth;
+    }
+    uint32_t st = 0, pos = P.size - 1;
+    if (l < Dj) {
+      const SmallNode& Q = s_node[s_off[l - 3] + P.pidx];
+      const uint32_t qm = s_mask[s_off[l - 3] + P.pidx];
+      uint32_t sp = 0, cur = P.pidx;  // start of the parent
+      for (l++; l < Dj; l++) {
+        const SmallNode& X = s_node[s_off[l - 4] + cur];
+        sp += X.sib;
+        cur = X.pidx;
+      }
+      st = sp + P.sib;
+      pos = sp + Q.size - 1 - (uint32_t)__popc(qm) + (j - Q.first);
+    }
+    if (pos >= nn || nbase + pos >= node_cap) {
+      M.flag[1] = 1;
+      continue;
+    }
+    if (g < NB) start[g] = st;
+    uint64_t* r = nodes + 3 * (nbase + pos);
+    r[0] = 0;
+    r[1] = st + P.size - 1 - (uint32_t)__popc(cm) + cb_add;
+    r[2] = offsets_of(cm);
+  }
+}
+
 #define SVO_TRY(x)                   \
   do {                               \
     hipError_t _e = (x);             \
@@ -1111,6 +1330,10 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
         h_tail = h;
         break;
       }
+    uint64_t nup = 0;  // nodes from the bricks up, at most
+    for (int h = 4; h <= H && up_once; h++) nup += bound[h];
+    // all of it in one launch
+    const bool up_small = up_once && NB <= kTailBlock && nup <= kSmallNodes;
     const int h_scan_end = up_once ? h0 : h_tail;  // level scans for h0 .. h_scan_end-1
     uint64_t st_words = 0;
     for (int h = h0; h < h_scan_end; h++) st_words += scan_single_words(bound[h], kLevelScanSmall);
@@ -1154,12 +1377,23 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
     SVO_TRY(run_segment(c, [&]() -> hipError_t {
       // n[0] = V, off[1] = 0, flags = 0, root sizes = 0, hazard flags = 0, scan status = 0
       // (fast: n[4] = NB, off[4] = 0, off[5] = NB)
-      SVO_LAUNCH(k_build_init, dim3(1), dim3(256), 0, c.stream, meta,
-                         meta_words + st_words, V, NB, (uint64_t)(fast ? 1 : 0),
-                         job_arg ? d_jobs : (JobDev*)nullptr, jd[0]);
+      if (!up_small)
+        SVO_LAUNCH(k_build_init, dim3(1), dim3(256), 0, c.stream, meta,
+                           meta_words + st_words, V, NB, (uint64_t)(fast ? 1 : 0),
+                           job_arg ? d_jobs : (JobDev*)nullptr, jd[0]);
       SVO_TRY(hipGetLastError());
 
-      if (up_once) {
+      if (up_small) {
+        ktimer_begin(c, "upper_levels");
+        SVO_LAUNCH(k_up_small, dim3(1), dim3(kTailBlock), 0, c.stream, A.start, M, T, d_jobs,
+                   n_jobs, c.bwords.as<uint64_t>(), c.bcode.as<uint64_t>(),
+                   c.bshape.as<uint32_t>(), (uint32_t)NB, H, meta_words, (int)job_arg, jd[0],
+                   root_size, root_isize, brick_hazard,
+                   (uint64_t*)((char*)c.up_tiles.p + b_cnt + b_s4 + b_end), node_cap, nodes,
+                   c.records.as<float>());
+        ktimer_end(c);
+        SVO_TRY(hipGetLastError());
+      } else if (up_once) {
         char* ub = (char*)c.up_tiles.p;
         uint32_t* tile_cnt = (uint32_t*)ub;
         uint64_t* tile_s4 = (uint64_t*)(ub + b_cnt);
@@ -1175,8 +1409,6 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
         SVO_LAUNCH(k_up_apply, dim3(ntiles), dim3(kUpTile), 0, c.stream, A, M, T,
                            (const JobDev*)d_jobs, NB, H, (const uint32_t*)tile_cnt,
                            (const uint64_t*)tile_s4, (const uint64_t*)a_end, job_end);
-        uint64_t nup = 0;
-        for (int h = 4; h <= H; h++) nup += bound[h];
         SVO_LAUNCH(k_up_finish, dim3((unsigned)((nup + 255) / 256)), dim3(256), 0,
                            c.stream, A, M, T, (const JobDev*)d_jobs, H,
                            (const uint64_t*)job_end, root_size);
@@ -1195,7 +1427,8 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
                                        M.n + h, kLevelScanSmall)));
         status += scan_single_words(bound[h], kLevelScanSmall);
       }
-      SVO_LAUNCH(k_levels_tail, dim3(1), dim3(kTailBlock), 0, c.stream, A, M, T, d_jobs,
+      if (!up_small)
+        SVO_LAUNCH(k_levels_tail, dim3(1), dim3(kTailBlock), 0, c.stream, A, M, T, d_jobs,
                          n_jobs, c.codes.as<uint64_t>(), c.lvl_leafp.as<uint32_t>(), root_size,
                          root_isize, c.records.as<float>() + 8, h_tail, H,
                          fast ? brick_hazard : nullptr, node_cap,
@@ -1203,7 +1436,7 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
       SVO_TRY(hipGetLastError());
       // ---- top-down: heights H .. 1 (one launch without -levels), then the leaves
       const int hs = std::max(h0, 1);
-      if (!levels && H >= hs) {
+      if (!levels && !up_small && H >= hs) {
         uint64_t nup = 0;
         for (int h = hs; h <= H; h++) nup += bound[h];
         ktimer_begin(c, "emit_children");
