@@ -349,7 +349,7 @@ struct MarkDenseT {
 using MarkDenseAction = MarkDenseT<false>;
 using MarkDenseWideAction = MarkDenseT<true>;
 
-// Payload marks of one mesh, gathered in LDS: a wave keeps kLines lines of 32 cells (128 bytes
+// Payload marks, gathered in LDS: a wave keeps kLines lines of 32 cells (128 bytes
 // of the grid), takes the maximum of ~triangle there, and gives a line to memory whole, a half
 // wave a line. A cell whose line's place holds another line goes to memory at once.
 //
@@ -754,8 +754,9 @@ template <typename Act>
 __global__ __launch_bounds__(kTile, kTileBlocks<Act>) void k_vox_tile(const VoxParams* __restrict__ units,
                                                        uint32_t n_units,
                                                        const uint32_t* __restrict__ tile_off,
-                                                       ActArgs A, ull* queue, LargeList B,
-                                                       uint32_t tt, int collect, int skip) {
+                                                       uint64_t payload_runs, ActArgs A,
+                                                       ull* queue, LargeList B, uint32_t tt,
+                                                       int collect, int skip) {
   __shared__ WalkLds s_walk[kTileWaves];
   __shared__ volatile uint32_t s_empty[kQueues];  // classes found empty
   if (threadIdx.x < kQueues) s_empty[threadIdx.x] = 0;
@@ -771,7 +772,13 @@ __global__ __launch_bounds__(kTile, kTileBlocks<Act>) void k_vox_tile(const VoxP
   }
   ull* ctr = A.ctr;
   const int lane = lane_id();
-  const uint32_t total = tile_off[n_units];
+  // Runs of geometry-only and of payload tiles, mixed evenly (payload_runs: 2^32 x the payload
+  // runs' share, rounded up): the first are bound by vector instructions, the others by their
+  // atomics. 64 mixed meshes 2.74 ms job by job, 2.52 so.
+  const uint32_t* const off_kind[2] = {tile_off, tile_off + n_units + 1};
+  const uint32_t runs = (off_kind[0][n_units] + kTileRun - 1) / kTileRun +
+                        (off_kind[1][n_units] + kTileRun - 1) / kTileRun;
+  const uint32_t total = runs * kTileRun;
   // Runs of kTileRun tiles are dealt to kQueues classes (one per XCD: blocks are dealt to
   // them in turn), each with its own counter in its own cache line: a run's tiles, neighbours
   // in space, mark lines of one L2, and the classes hold about the same work. One counter's
@@ -796,13 +803,18 @@ __global__ __launch_bounds__(kTile, kTileBlocks<Act>) void k_vox_tile(const VoxP
       }
     }
     // in a scalar register: the unit search and the unit's parameters run on scalar loads
-    const uint32_t tile = (uint32_t)__builtin_amdgcn_readfirstlane((int)next);
-    if (tile >= total) return;
+    const uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)next);
+    if (at >= total) return;
     next = total;
-    const uint32_t u = upper_index<uint32_t>(tile_off, n_units + 1, tile);
+    const uint32_t run = at / kTileRun, pay = (uint32_t)((run * payload_runs) >> 32);
+    const bool is_pay = (uint32_t)(((run + 1ull) * payload_runs) >> 32) > pay;
+    const uint32_t tile = (is_pay ? pay : run - pay) * kTileRun + at % kTileRun;
+    const uint32_t* const off = off_kind[is_pay];
+    if (tile >= off[n_units]) continue;  // the kind's last run, not full
+    const uint32_t u = upper_index<uint32_t>(off, n_units + 1, tile);
     const VoxParams P = units[u];
     if (skipped(P, skip)) continue;
-    const uint32_t i = (tile - tile_off[u]) * tt + lane;
+    const uint32_t i = (tile - off[u]) * tt + lane;
     Walk K;
     uint32_t ncols = 0, nu = 0, nv = 0;  // columns of a triangle of this tier; its sides
     bool large = false;
@@ -1574,7 +1586,8 @@ hipError_t upload_async(Context& c, void* dst, const void* src, size_t bytes) {
       if (c.stage) (void)hipHostFree(c.stage);
       c.stage = nullptr;
       c.stage_cap = 0;
-      const size_t cap = std::max<size_t>(need, 4u << 20);
+      // (pinned pages cost 0.15 us each to get: 4 MB of them 600 us of a new context's first pass)
+      const size_t cap = std::max<size_t>(4 * need, 128u << 10);
       SVO_TRY(hipHostMalloc(&c.stage, cap, hipHostMallocDefault));
       c.stage_cap = cap;
     }
@@ -1613,7 +1626,7 @@ static hipError_t ensure_hread(Context& c, size_t total) {
   if (c.hread) (void)hipHostFree(c.hread);
   c.hread = nullptr;
   c.hread_cap = 0;
-  const size_t cap = std::max<size_t>(total, 1u << 20);
+  const size_t cap = std::max<size_t>(2 * total, 72u << 10);  // (every small read-back fits)
   SVO_TRY(hipHostMalloc(&c.hread, cap, hipHostMallocDefault));
   // memory freed by another context may hold its last flag: a value this one will wait for
   memset(c.hread, 0, 256);
@@ -1865,10 +1878,12 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     if (u.n) units.push_back(u);  // main.cpp:330 skips empty partitions
   const uint32_t nu = (uint32_t)units.size();
   if (nu == 0) return hipSuccess;
-  // unit table: VoxParams[nu] | ubase[nu+1] | tile_off[nu+1] | uvoff[nu+1]
+  // unit table: VoxParams[nu] | ubase[nu+1] | 2 x tile_off[nu+1] | uvoff[nu+1]
   std::vector<VoxParams> P(nu);
   std::vector<uint64_t> ubase(nu + 1);
-  std::vector<uint32_t> toff(nu + 1);
+  // tiles before each unit: of the geometry-only units, of the payload ones
+  std::vector<uint32_t> toff(2 * (nu + 1), 0);
+  uint32_t* const toff_kind[2] = {&toff[0], &toff[nu + 1]};
   uint64_t ntab = 0, ntiles = 0, ntri = 0;
   // triangles per tile: kTileTris once the pass has about four tiles of them per wave of the
   // persistent grid, else fewer; up to 16 a wave, one tile for each wave
@@ -1910,13 +1925,14 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     P[u].small_cols = small_cols;
     P[u].table_base = ntab;
     ubase[u] = ntab;
-    toff[u] = (uint32_t)ntiles;
     ntab += unit_bricks(units[u]);
-    ntiles += (units[u].n + tt - 1) / tt;
+    const uint64_t tiles = (units[u].n + tt - 1) / tt;
+    for (int k = 0; k < 2; k++)
+      toff_kind[k][u + 1] = toff_kind[k][u] + ((units[u].stride == 21) == (k == 1) ? (uint32_t)tiles : 0u);
+    ntiles += tiles;
     ntri += units[u].n;
   }
   ubase[nu] = ntab;
-  toff[nu] = (uint32_t)ntiles;
   if (ntab > 0xFFFFFFF0ull || ntiles > 0xFFFFFFF0ull || ntri > 0xFFFFFFF0ull) {
     set_error("voxelize pass too large for 32-bit brick, tile or triangle indices");
     return hipErrorInvalidValue;
@@ -1934,11 +1950,12 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
   for (uint32_t u = 0; u < nu; u++) geometry_only = geometry_only && units[u].stride == 9;
   // the table, the word flags, the dense grid and the byte pool are all-zero whenever no pass
   // is running
-  if (c.table_entries < ntab) {
-    SVO_TRY(ensure(c.table, ntab * 4));
-    SVO_TRY(fill_u32(c.table.as<uint32_t>(), 0, ntab, c.stream));
-    c.table_entries = ntab;
-  }
+  const bool new_table = c.table_entries < ntab;
+  const bool new_flags = dense && !geometry_only && c.cflags_zeroed < ntab * kBrickWords;
+  // (allocated before the first fill: an allocation while the GPU works waits for it)
+  if (new_table) SVO_TRY(ensure(c.table, ntab * 4));
+  if (new_flags) SVO_TRY(ensure(c.cflags, ntab * kBrickWords));
+  uint64_t grid_fill = 0;
   if (dense) {
     if (c.grid_zeroed < dense_bytes) {
       // grown to at least twice its size (at most the dense limit), so that passes of
@@ -1950,13 +1967,7 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
         release(c.grid8);
         SVO_TRY(ensure(c.grid8, target));
       }
-      SVO_TRY(fill_u64(c.grid8.as<uint64_t>(), 0, target / 8, c.stream));
-      c.grid_zeroed = target;
-    }
-    if (!geometry_only && c.cflags_zeroed < ntab * kBrickWords) {
-      SVO_TRY(ensure(c.cflags, ntab * kBrickWords));
-      SVO_TRY(fill_u64(c.cflags.as<uint64_t>(), 0, ntab * kBrickWords / 8, c.stream));
-      c.cflags_zeroed = ntab * kBrickWords;
+      grid_fill = target;
     }
     for (uint32_t u = 0; u < nu; u++) {
       P[u].dense = 1;
@@ -1972,7 +1983,7 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
   }
   const size_t szP = ((nu * sizeof(VoxParams)) + 255) & ~(size_t)255;
   const size_t szB = (((nu + 1) * 8) + 255) & ~(size_t)255;
-  const size_t szT = (((nu + 1) * 4) + 255) & ~(size_t)255;
+  const size_t szT = ((toff.size() * 4) + 255) & ~(size_t)255;
   {
     const void* prev = c.unitdev.p;
     const size_t prev_cap = c.unitdev.cap;
@@ -1987,7 +1998,7 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     std::vector<uint8_t> img(szP + szB + szT, 0);
     memcpy(img.data(), P.data(), nu * sizeof(VoxParams));
     memcpy(img.data() + szP, ubase.data(), (nu + 1) * 8);
-    memcpy(img.data() + szP + szB, toff.data(), (nu + 1) * 4);
+    memcpy(img.data() + szP + szB, toff.data(), toff.size() * 4);
     // a pass over the same units as the last one (the same mesh again) finds them there
     if (img != c.unit_img) {
       SVO_TRY(upload_async(c, d_units, img.data(), img.size()));
@@ -2015,13 +2026,20 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
   SVO_TRY(ensure(c.large_walk, (size_t)walk_cap * kLargeQuads * sizeof(uint4)));
   SVO_TRY(ensure(c.occ_list, ntab * 4));
   SVO_TRY(ensure_scan_scratch(c, ntab, 8));
+  if (new_table) {
+    SVO_TRY(fill_u32(c.table.as<uint32_t>(), 0, ntab, c.stream));
+    c.table_entries = ntab;
+  }
+  if (grid_fill) {
+    SVO_TRY(fill_u64(c.grid8.as<uint64_t>(), 0, grid_fill / 8, c.stream));
+    c.grid_zeroed = grid_fill;
+  }
+  if (new_flags) {
+    SVO_TRY(fill_u64(c.cflags.as<uint64_t>(), 0, ntab * kBrickWords / 8, c.stream));
+    c.cflags_zeroed = ntab * kBrickWords;
+  }
   ull* ctr = c.counters.as<ull>();
   ull hc[kNumCounters];
-  // (one payload mesh: half the waves, whose winner atomics meet on the same cells less often;
-  // 320,000 triangles at 512: mark 73 -> 67 us)
-  const unsigned tile_grid = (unsigned)std::min<uint64_t>(
-      (ntiles + kTileWaves - 1) / kTileWaves,
-      std::max(1, nu == 1 && !geometry_only ? c.tune.tile_blocks / 2 : c.tune.tile_blocks));
   const unsigned large_grid = (unsigned)c.tune.large_blocks;
   auto brick_grid = [&](uint64_t bricks) {
     return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((bricks * kWave + 255) / 256, 8192));
@@ -2041,11 +2059,18 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
   const LargeList large{c.large_unit.as<uint32_t>(), c.large_tri.as<uint32_t>(),
                         c.large_rows.as<uint32_t>(), c.large_jobs.as<uint2>(),
                         c.large_walk.as<uint4>(),    walk_cap};
+  const uint64_t runs_kind[2] = {(toff_kind[0][nu] + (uint64_t)kTileRun - 1) / kTileRun,
+                                 (toff_kind[1][nu] + (uint64_t)kTileRun - 1) / kTileRun};
+  const uint64_t runs = runs_kind[0] + runs_kind[1];
+  const uint64_t payload_runs = ((runs_kind[1] << 32) + runs - 1) / runs;
   auto tile_pass = [&](auto tag, const char* name, ull* queue, int collect, int skip) {
     using Act = decltype(tag);
+    const unsigned tile_grid = (unsigned)std::min<uint64_t>(
+        runs * kTileRun / kTileWaves,
+        std::max(1, c.tune.tile_blocks * kTileBlocks<Act> / kTileBlocks<MarkDenseAction>));
     ktimer_begin(c, name);
     SVO_LAUNCH((k_vox_tile<Act>), dim3(tile_grid), dim3(kTile), 0, c.stream, d_units, nu,
-                       d_toff, args(), queue, large, tt, collect, skip);
+                       d_toff, payload_runs, args(), queue, large, tt, collect, skip);
     ktimer_end(c);
     return hipGetLastError();
   };
@@ -2099,9 +2124,11 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
       }
       // first pass: dense units mark directly, touch units flag their bricks; both collect
       // the large triangles
+      // (units of both kinds: the payload marks' lines in LDS would leave room for half the waves
+      // of the others; apart, in two launches, 64 mixed meshes took 1.15 + 1.89 ms against 2.74)
       if (dense && geometry_only)
         SVO_TRY(tile_pass(MarkDenseAction{}, "vox_small_mark", queues, 1, 0));
-      else if (dense && nu == 1)
+      else if (dense && !toff_kind[0][nu])
         SVO_TRY(tile_pass(MarkGatherAction{}, "vox_small_mark", queues, 1, 0));
       else if (dense)
         SVO_TRY(tile_pass(MarkDenseWideAction{}, "vox_small_mark", queues, 1, 0));
@@ -2267,7 +2294,7 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     // dense and geometry-only passes write no codes: the build reads the brick stream, and
     // ensure_codes writes the codes for readers that want them
     const bool codes_now = winner_walk;
-    SVO_TRY(ensure_keep(c.codes, (s0 + nvox) * 8, s0 * 8, c.stream));
+    if (codes_now) SVO_TRY(ensure_keep(c.codes, (s0 + nvox) * 8, s0 * 8, c.stream));
     if (!dense) {
       SVO_TRY(ensure_keep(c.bwords, (nb0 + n_occ) * kBrickWords * 8, nb0 * kBrickWords * 8,
                           c.stream));
@@ -2374,6 +2401,7 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
 
 hipError_t ensure_codes(Context& c) {
   if (!c.codes_lazy) return hipSuccess;
+  SVO_TRY(ensure_keep(c.codes, std::max<uint64_t>(c.n_vox, 1) * 8, c.n_vox * 8, c.stream));
   // every brick again (rewriting codes already there with the same values)
   if (c.n_bricks) {
     const unsigned grid =
