@@ -250,18 +250,15 @@ struct ParentStore {
   }
 };
 
-// Level bookkeeping before a build: all zero, n[0] = V and, when the four lowest levels
-// come from the brick stream, n[4] = NB and off[5] = NB; the device clock in flag[3]; a single
-// job's descriptor (job, unless null) from the arguments.
+// Level bookkeeping before a build from the codes: all zero, n[0] = V; the device clock in
+// flag[3]; a single job's descriptor (job, unless null) from the arguments.
 constexpr int kStampWord = 2 * 64 + 3;
 __global__ __launch_bounds__(256) void k_build_init(unsigned long long* meta, uint64_t words,
-                                                    uint64_t V, uint64_t NB, uint64_t fast,
-                                                    JobDev* job, JobDev j0) {
+                                                    uint64_t V, JobDev* job, JobDev j0) {
   const unsigned long long now = wall_clock64();
   for (uint64_t i = threadIdx.x; i < words; i += blockDim.x) {
     unsigned long long v = 0;
     if (i == 0) v = V;
-    if (fast && (i == 4 || i == 64 + 5)) v = NB;
     if (i == kStampWord) v = now;
     meta[i] = v;
   }
@@ -770,6 +767,21 @@ __global__ __launch_bounds__(kWave * kEmitWaves) void k_emit_bricks(
 constexpr int kUpTile = 256;
 constexpr int kUpLevels = 17;  // heights 5 .. 21
 
+// job_bases for one job with bricks: its fields (one thread), and the null record and the white
+// one of geometry-only builds (16 threads).
+__device__ __forceinline__ void put_single_base(JobDev* job, const JobDev& j0, const LevelMeta& M,
+                                                uint64_t n_nodes, uint64_t hazard) {
+  job->n_nodes = n_nodes;
+  job->nbase = 0;
+  job->hazard = hazard;
+  job->n_data = j0.payload ? 1 + j0.nvox : 2;
+  M.flag[2] = n_nodes;
+}
+__device__ __forceinline__ void put_leading_records(float* records, const JobDev& j0) {
+  if (threadIdx.x < (j0.payload ? 8u : 16u))
+    records[j0.dbase * 8 + threadIdx.x] = threadIdx.x >= 10 && threadIdx.x < 13 ? 1.0f : 0.0f;
+}
+
 // T(i) from brick i's node code c and the previous brick's p (has_prev = i > 0)
 __device__ __forceinline__ int brick_top(uint64_t c, uint64_t p, bool has_prev, Tags T, int D) {
   if (D <= 4) return 4;
@@ -788,9 +800,11 @@ __device__ __forceinline__ int job_depth(const JobDev* jobs, Tags T, uint64_t co
 
 // Per brick: its height-4 node (code, subtree size and child mask from the voxelizer's
 // brick shape) and the hazard case (the job's last voxel is code G^3 - 2: bits 62 and 63
-// of the last word of the grid's last brick); per tile: counts of T >= l for l = 5 .. H,
-// and the sum of the brick subtree sizes.
-__global__ __launch_bounds__(kUpTile) void k_up_count(Arena A, Tags T, const JobDev* jobs,
+// of the last word of the grid's last brick; a job's last brick answers for it); per tile: counts
+// of T >= l for l = 5 .. H, and the sum of the brick subtree sizes. The first block also leaves
+// the device clock in *stamp and, with put, the single job's descriptor j0 in *jobs.
+__global__ __launch_bounds__(kUpTile) void k_up_count(Arena A, Tags T, JobDev* jobs, int put,
+                                                      JobDev j0, unsigned long long* stamp,
                                                       const uint64_t* __restrict__ bwords,
                                                       const uint64_t* __restrict__ bcode,
                                                       const uint32_t* __restrict__ bshape,
@@ -803,6 +817,10 @@ __global__ __launch_bounds__(kUpTile) void k_up_count(Arena A, Tags T, const Job
   const uint64_t i = (uint64_t)blockIdx.x * kUpTile + threadIdx.x;
   int t = 4;
   uint64_t s4 = 0;
+  if (i == 0) {
+    *stamp = wall_clock64();
+    if (put) *jobs = j0;
+  }
   if (i < NB) {
     const uint64_t c0 = bcode[i];
     const uint64_t code = brick_node_code(c0, T);
@@ -814,12 +832,13 @@ __global__ __launch_bounds__(kUpTile) void k_up_count(Arena A, Tags T, const Job
     A.mask[i] = (uint8_t)(sh >> 16);
     A.first[i] = 0;
     const uint32_t jb = T.job(c0);
-    const JobDev& J = jobs[jb];
-    const uint64_t G = J.gridsize;
-    if ((c0 & ~T.tag_mask) == G * G * G - kBrickVox &&
-        (bwords[i * kBrickWords + kWave - 1] >> 62) == 1ull)
-      hazard[jb] = 1;
-    t = brick_top(code, prev, i > 0, T, J.depth);
+    // (one job: not from the memory that it is being put into)
+    const uint64_t G = T.tag_mask ? jobs[jb].gridsize : j0.gridsize;
+    const int D = T.tag_mask ? jobs[jb].depth : j0.depth;
+    if (i + 1 == NB || (T.tag_mask && T.job(bcode[i + 1]) != jb))
+      hazard[jb] = (c0 & ~T.tag_mask) == G * G * G - kBrickVox &&
+                   (bwords[i * kBrickWords + kWave - 1] >> 62) == 1ull;
+    t = brick_top(code, prev, i > 0, T, D);
   }
   const int w = threadIdx.x / kWave;
 #pragma unroll
@@ -844,9 +863,12 @@ __global__ __launch_bounds__(kUpTile) void k_up_count(Arena A, Tags T, const Job
 
 // one block, a wave per height (and one for the sizes): the exclusive prefix of the tile
 // counts (in place, 64 tiles at a time); then the node counts and arena offsets of all
-// heights and A_l at the end of the stream; an arena too small is flagged
+// heights and A_l at the end of the stream; an arena too small is flagged. One job (jobs not
+// null; it has bricks, so it is not trivial): job_bases' results as well.
 __global__ __launch_bounds__(1024) void k_up_scan(Arena A, LevelMeta M, uint64_t NB, int H,
-                                                  uint32_t ntiles,
+                                                  JobDev* jobs, JobDev j0,
+                                                  const unsigned long long* hazard,
+                                                  float* records, uint32_t ntiles,
                                                   uint32_t* __restrict__ tile_cnt,
                                                   uint64_t* __restrict__ tile_s4,
                                                   uint64_t* __restrict__ a_end) {
@@ -876,6 +898,8 @@ __global__ __launch_bounds__(1024) void k_up_scan(Arena A, LevelMeta M, uint64_t
   if (threadIdx.x == 0) {
     uint64_t off = NB;  // off[5]
     uint64_t a = s_tot[kUpLevels];  // S4 at the end
+    M.n[4] = M.off[5] = NB;
+    M.off[4] = 0;
     for (int l = 5; l <= H; l++) {
       const uint64_t n = s_tot[l - 5];
       M.n[l] = n;
@@ -885,8 +909,11 @@ __global__ __launch_bounds__(1024) void k_up_scan(Arena A, LevelMeta M, uint64_t
       a += n;
       a_end[l - 5] = a;
     }
-    if (off > A.cap) M.flag[0] = 1;
+    M.flag[0] = off > A.cap;
+    M.flag[1] = 0;
+    if (jobs) put_single_base(jobs, j0, M, a, *hazard);
   }
+  if (jobs) put_leading_records(records, j0);
 }
 
 // Per brick: the parent index of its brick node, the fields of every node it heads, A_l at
@@ -1181,19 +1208,10 @@ __global__ __launch_bounds__(kTailBlock) void k_up_small(
     job_bases<kTailBlock>(jobs, n_jobs, root_size, root_isize, hazard, nullptr, T, M, node_cap,
                           nodes, records, records, s_scan, s_carry);
     __syncthreads();
-  } else {  // one job, not trivial (it has bricks): job_bases' results
+  } else {
     n_nodes = s_node[total - 1].size;
-    if (threadIdx.x == 0) {
-      jobs->n_nodes = n_nodes;
-      jobs->nbase = 0;
-      jobs->hazard = s_hazard;
-      jobs->n_data = j0.payload ? 1 + j0.nvox : 2;
-      M.flag[2] = n_nodes;
-    }
-    // the null record, and the white one of geometry-only builds
-    if (threadIdx.x < (j0.payload ? 8u : 16u))
-      records[j0.dbase * 8 + threadIdx.x] =
-          threadIdx.x >= 10 && threadIdx.x < 13 ? 1.0f : 0.0f;
+    if (threadIdx.x == 0) put_single_base(jobs, j0, M, n_nodes, s_hazard);
+    put_leading_records(records, j0);
   }
   for (uint32_t g = threadIdx.x; g < total; g += kTailBlock) {  // records
     int l = height(g);
@@ -1329,6 +1347,9 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
   SVO_TRY(ensure_keep(c.records, n_records * 32, n_records * 32, c.stream));
   JobDev* d_jobs = c.jobdev.as<JobDev>();
   const Tags T{tagged ? ~kCodeMask : 0ull};
+  JobDev job0;  // a single job's descriptor, for the kernels' arguments
+  memset(&job0, 0, sizeof(job0));
+  if (!tagged) job0 = jd[0];
 
   // arena: the internal nodes the level scans produce (heights >= h0)
   uint64_t cap = fast ? NB + NB / 2 + 4096 : std::max<uint64_t>(V / 2 + 1024, 4096);
@@ -1400,18 +1421,17 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
     // the build's kernels up to its read-back: one graph segment
     SVO_TRY(run_segment(c, [&]() -> hipError_t {
       // n[0] = V, off[1] = 0, flags = 0, root sizes = 0, hazard flags = 0, scan status = 0
-      // (fast: n[4] = NB, off[4] = 0, off[5] = NB)
-      if (!up_small)
-        SVO_LAUNCH(k_build_init, dim3(1), dim3(256), 0, c.stream, meta,
-                           meta_words + st_words, V, NB, (uint64_t)(fast ? 1 : 0),
-                           job_arg ? d_jobs : (JobDev*)nullptr, jd[0]);
+      // (the brick path writes what it reads itself)
+      if (!up_once)
+        SVO_LAUNCH(k_build_init, dim3(1), dim3(256), 0, c.stream, meta, meta_words + st_words, V,
+                   job_arg ? d_jobs : (JobDev*)nullptr, job0);
       SVO_TRY(hipGetLastError());
 
       if (up_small) {
         ktimer_begin(c, "upper_levels");
         SVO_LAUNCH(k_up_small, dim3(1), dim3(kTailBlock), 0, c.stream, A.start, M, T, d_jobs,
                    n_jobs, c.bwords.as<uint64_t>(), c.bcode.as<uint64_t>(),
-                   c.bshape.as<uint32_t>(), (uint32_t)NB, H, meta_words, (int)job_arg, jd[0],
+                   c.bshape.as<uint32_t>(), (uint32_t)NB, H, meta_words, (int)job_arg, job0,
                    root_size, root_isize, brick_hazard,
                    (uint64_t*)((char*)c.up_tiles.p + b_cnt + b_s4 + b_end), node_cap, nodes,
                    c.records.as<float>());
@@ -1425,10 +1445,12 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
         uint64_t* job_end = (uint64_t*)(ub + b_cnt + b_s4 + b_end);
         ktimer_begin(c, "upper_levels");
         SVO_LAUNCH(k_up_count, dim3(ntiles), dim3(kUpTile), 0, c.stream, A, T,
-                           (const JobDev*)d_jobs, c.bwords.as<uint64_t>(),
+                           d_jobs, (int)job_arg, job0, M.flag + 3, c.bwords.as<uint64_t>(),
                            c.bcode.as<uint64_t>(), c.bshape.as<uint32_t>(), NB, H, tile_cnt,
                            tile_s4, brick_hazard);
-        SVO_LAUNCH(k_up_scan, dim3(1), dim3(1024), 0, c.stream, A, M, NB, H, ntiles,
+        SVO_LAUNCH(k_up_scan, dim3(1), dim3(1024), 0, c.stream, A, M, NB, H,
+                           tagged ? (JobDev*)nullptr : d_jobs, job0,
+                           (const unsigned long long*)brick_hazard, c.records.as<float>(), ntiles,
                            tile_cnt, tile_s4, a_end);
         SVO_LAUNCH(k_up_apply, dim3(ntiles), dim3(kUpTile), 0, c.stream, A, M, T,
                            (const JobDev*)d_jobs, NB, H, (const uint32_t*)tile_cnt,
@@ -1451,7 +1473,7 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
                                        M.n + h, kLevelScanSmall)));
         status += scan_single_words(bound[h], kLevelScanSmall);
       }
-      if (!up_small)
+      if (!up_once || (tagged && !up_small))
         SVO_LAUNCH(k_levels_tail, dim3(1), dim3(kTailBlock), 0, c.stream, A, M, T, d_jobs,
                          n_jobs, c.codes.as<uint64_t>(), c.lvl_leafp.as<uint32_t>(), root_size,
                          root_isize, c.records.as<float>() + 8, h_tail, H,

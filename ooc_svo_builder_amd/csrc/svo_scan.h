@@ -214,6 +214,14 @@ __device__ __forceinline__ unsigned long long status_get(const unsigned long lon
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// What a Store does for an empty input, if it has a say in that: none().
+template <typename Store>
+__device__ __forceinline__ auto scan_none(const Store& st, int) -> decltype(st.none()) {
+  st.none();
+}
+template <typename Store>
+__device__ __forceinline__ void scan_none(const Store&, long) {}
+
 template <typename T, typename Load, typename Store, int ITEMS>
 __global__ __launch_bounds__(kSingleBlock) void k_scan_single(Load ld, Store st, uint64_t n,
                                                               const unsigned long long* n_dev,
@@ -227,6 +235,7 @@ __global__ __launch_bounds__(kSingleBlock) void k_scan_single(Load ld, Store st,
   const uint32_t tile = s_tile;
   unsigned long long* tiles = status + 1;
   if (n_dev) n = min(n, (uint64_t)*n_dev);
+  if (n == 0 && tile == 0 && threadIdx.x == 0) scan_none(st, 0);
   if ((uint64_t)tile * kSingleBlock * ITEMS >= n) return;  // uniform per block
   const uint64_t first = striped_first<ITEMS>(tile, kSingleBlock);
   T v[ITEMS], ex[ITEMS];

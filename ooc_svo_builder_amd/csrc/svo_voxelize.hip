@@ -1146,16 +1146,33 @@ struct CountStore {
     if (last) *total = (ull)(ex + v);
   }
 };
-// Brick counts of a dense pass: also each brick's first voxel in the stream (s0 + offset).
+// Brick counts of a dense pass: also each brick's first voxel in the stream (s0 + offset). With
+// host (a pass of one unit), the thread that has the total gives the pass's counters to the host,
+// which waits for them: the launch that would follow for it took 4 us.
 struct BrickOffStore {
   uint64_t* off;
-  ull* total;
+  ull* ctr;
   uint64_t* bvoff;
   uint64_t s0;
+  uint64_t* host;  // pinned: kNumCounters words, or nullptr
+  volatile uint32_t* flag;
+  uint64_t seq;
   __device__ void operator()(uint64_t i, uint64_t ex, uint64_t v, bool last) const {
     off[i] = ex;
     bvoff[i] = s0 + (ex & kVoxMask);
-    if (last) *total = (ull)(ex + v);
+    if (last) done(ex + v);
+  }
+  __device__ void none() const { done(0); }  // no bricks
+  __device__ void done(uint64_t total) const {
+    ctr[kCtrNumVox] = total;
+    if (!host) return;
+    uint64_t h[kNumCounters];
+#pragma unroll
+    for (int k = 0; k < kNumCounters; k++) h[k] = k == kCtrNumVox ? total : (uint64_t)ctr[k];
+#pragma unroll
+    for (int k = 0; k < kNumCounters; k++) host[k] = h[k];
+    __threadfence_system();
+    *flag = (uint32_t)seq;
   }
 };
 
@@ -1381,7 +1398,7 @@ __device__ __forceinline__ uint32_t nth_set_bit(uint64_t w, uint32_t n) {
 // its voxels 64 at a time in Morton order, so that neighbouring lanes read neighbouring cells
 // (~the winning triangle, 0 = unmarked) and write neighbouring records. The cells of non-empty
 // words are zeroed afterwards, whole 256-byte words at once. Codes and winners are not written
-// (ensure_codes expands the codes for readers that want them).
+// (ensure_codes expands the codes for readers that want them). jobs = nullptr: the job is j0.
 //
 // Bound by memory: 32 bytes written a voxel, the cells' words, and the winners' records
 // gathered. A pass that wrote every voxel's code and winner (a lane per word, its voxels one
@@ -1391,7 +1408,7 @@ __global__ __launch_bounds__(256) void k_payload_bricks(
     const uint32_t* __restrict__ occ, const ull* __restrict__ n_occ_ptr,
     const VoxParams* __restrict__ units, const uint64_t* __restrict__ ubase, uint32_t n_units,
     const ull* __restrict__ words, const uint64_t* __restrict__ boff,
-    const JobDev* __restrict__ jobs, uint64_t s0, float* __restrict__ out, ull* ctr) {
+    const JobDev* __restrict__ jobs, JobDev j0, uint64_t s0, float* __restrict__ out, ull* ctr) {
   __shared__ uint8_t s_slot[256];
   uint8_t* slot = s_slot + (threadIdx.x / kWave) * kWave;
   const int lane = lane_id();
@@ -1403,7 +1420,7 @@ __global__ __launch_bounds__(256) void k_payload_bricks(
     const ull word = words[wv * kBrickWords + lane];
     gword_t* cells = (gword_t*)units[u].grid8 + (ti - ubase[u]) * kBrickVox;
     const uint64_t code0 = units[u].bstart + ((ti - ubase[u]) << kBrickBits);
-    const JobDev& J = jobs[units[u].job];
+    const JobDev J = jobs ? jobs[units[u].job] : j0;
     const uint64_t pos0 = boff[wv] & kVoxMask;  // the brick's first voxel in the pass
     float* rec = out + (J.dbase + 1 + (s0 + pos0 - J.voff)) * 8;
     const uint32_t c = (uint32_t)__popcll(word);
@@ -2112,6 +2129,16 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     st_occ = c.scan_status.as<ull>();
     st_bc = st_occ + w_occ;
     queues = st_bc + w_bc;
+    // one unit: the scan of the brick counts reads back (not in a graph, whose arguments stay)
+    uint64_t* host_ctr = nullptr;
+    volatile uint32_t* host_flag = nullptr;
+    uint64_t seq = 0;
+    if (nu == 1 && dense && bc_single && !c.graphs) {
+      SVO_TRY(ensure_hread(c, 256 + kNumCounters * sizeof(ull)));
+      host_ctr = (uint64_t*)((char*)c.hread + 256);
+      host_flag = (volatile uint32_t*)c.hread;
+      seq = ++c.hread_seq;
+    }
     // the pass's kernels up to its read-back: one graph segment
     SVO_TRY(run_segment(c, [&]() -> hipError_t {
       {  // pass counters, scan status words and tile queues
@@ -2161,8 +2188,8 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
       if (bc_single && dense)
         SVO_TRY((scan_single<uint64_t>(
             ArrayLoad<uint64_t>{c.bcount.as<uint64_t>()},
-            BrickOffStore{c.bcount.as<uint64_t>(), ctr + kCtrNumVox,
-                          c.bvoff.as<uint64_t>() + nb0, s0},
+            BrickOffStore{c.bcount.as<uint64_t>(), ctr, c.bvoff.as<uint64_t>() + nb0, s0,
+                          host_ctr, host_flag, seq},
             bc_bound, st_bc, ctr + kCtrError, c.stream, ctr + kCtrNumOcc)));
       else if (bc_single)
         SVO_TRY((scan_single<uint64_t>(
@@ -2172,15 +2199,15 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
       else if (dense)
         SVO_TRY((scan_exclusive<uint64_t>(
             ArrayLoad<uint64_t>{c.bcount.as<uint64_t>()},
-            BrickOffStore{c.bcount.as<uint64_t>(), ctr + kCtrNumVox,
-                          c.bvoff.as<uint64_t>() + nb0, s0},
+            BrickOffStore{c.bcount.as<uint64_t>(), ctr, c.bvoff.as<uint64_t>() + nb0, s0, nullptr,
+                          nullptr, 0},
             bc_bound, c.scan_scratch.as<uint64_t>(), c.stream, ctr + kCtrNumOcc)));
       else
         SVO_TRY((scan_exclusive<uint64_t>(
             ArrayLoad<uint64_t>{c.bcount.as<uint64_t>()},
             CountStore{c.bcount.as<uint64_t>(), ctr + kCtrNumVox}, bc_bound,
             c.scan_scratch.as<uint64_t>(), c.stream, ctr + kCtrNumOcc)));
-      if (!(nu == 1 && geometry_only)) {
+      if (nu > 1) {
         SVO_LAUNCH(k_unit_voxels, dim3((nu + 256) / 256), dim3(256), 0, c.stream,
                    c.occ_list.as<uint32_t>(), dense ? kOccMask : 0xFFFFFFFFu, ctr, d_ubase, nu,
                    c.bcount.as<uint64_t>(), d_uvoff);
@@ -2188,11 +2215,16 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
       }
       return hipSuccess;
     }));
-    if (nu == 1 && geometry_only) {
-      // one unit and no payload records (the only device reader of the unit offsets):
-      // its voxels are the whole pass, [0, voxel count)
-      const ReadReq rq = {hc, c.counters.p, kNumCounters * sizeof(ull)};
-      SVO_TRY(read_back(c, &rq, 1));
+    if (nu == 1) {
+      // one unit: its voxels are the whole pass, [0, voxel count)
+      if (host_ctr) {
+        t_syncs++;
+        SVO_TRY(wait_flag(c, (uint32_t)seq));
+        memcpy(hc, host_ctr, sizeof(hc));
+      } else {
+        const ReadReq rq = {hc, c.counters.p, kNumCounters * sizeof(ull)};
+        SVO_TRY(read_back(c, &rq, 1));
+      }
       uvoff[0] = 0;
       uvoff[1] = hc[kCtrNumVox] & kVoxMask;
     } else {
@@ -2275,10 +2307,14 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
   if (batch) {
     SVO_TRY(upload_async(c, c.jobdev.p, jd.data(), jd.size() * sizeof(JobDev)));
     c.jobdev_img = jd;
-  } else if (any_payload) {  // (else the build is its first reader, and writes it)
+  } else if (any_payload && !dense) {  // (else the build is its first reader, and writes it)
     SVO_LAUNCH(k_put_job, dim3(1), dim3(1), 0, c.stream, c.jobdev.as<JobDev>(), jd[0]);
     SVO_TRY(hipGetLastError());
   }
+
+  JobDev job0;  // a single job's descriptor, for the kernels' arguments
+  memset(&job0, 0, sizeof(job0));
+  if (!batch) job0 = jd[0];
 
   // ---- phase B: emit sorted codes, payload, clear; no synchronization
   if (n_occ) {
@@ -2357,7 +2393,9 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
         SVO_LAUNCH(k_payload_bricks, dim3(brick_grid(n_occ)), dim3(256), 0, c.stream,
                    c.occ_list.as<uint32_t>(), (const ull*)(ctr + kCtrNumOcc),
                    (const VoxParams*)d_units, d_ubase, nu, (const ull*)pool_words,
-                   c.bcount.as<uint64_t>(), c.jobdev.as<JobDev>(), s0, c.records.as<float>(), ctr);
+                   c.bcount.as<uint64_t>(),
+                   batch ? (const JobDev*)c.jobdev.p : (const JobDev*)nullptr, job0, s0,
+                   c.records.as<float>(), ctr);
         ktimer_end(c);
         SVO_TRY(hipGetLastError());
       }
