@@ -98,51 +98,47 @@ struct Arena {
 };
 
 // -levels data record of an internal node (OctreeBuilder.cpp:82-99): the caches of its
-// 8 children summed in child order (a null child adds zeros), divided by the number of
-// non-null children, the normal then normalized (glm::normalize = v * (1 / sqrt(dot))).
-// Children j in [i, je) of the child level, in child order; leaf caches are the voxels'
-// own records (payload) or zero (geometry-only builds: leaves carry no data).
+// children summed in child order (a null child adds zeros, which change no sum that started
+// from +0), divided by the number of non-null children, the normal then normalized
+// (glm::normalize = v * (1 / sqrt(dot))). Children i .. i + cnt - 1 of the child level; leaf
+// caches are the voxels' own records (payload) or zero (geometry-only builds: leaves carry no
+// data).
+//
+// Bound by latency: every child's loads are issued before the first sum. One child after the
+// other, the levels of 487,600 payload voxels took 128 us, 116 now.
 __device__ __forceinline__ void average_children(const Arena& A, uint64_t coff, bool leaf,
                                                  const float* __restrict__ leaf_rec,
-                                                 int payload, const uint64_t* code, uint64_t i,
-                                                 uint64_t je, uint64_t& isz, float* out) {
-  float c0 = 0.0f, c1 = 0.0f, c2 = 0.0f, n0 = 0.0f, n1 = 0.0f, n2 = 0.0f;
-  float notnull = 0.0f;
-  isz = 1;
-  uint64_t j = i;
+                                                 int payload, uint64_t i, uint32_t cnt,
+                                                 uint64_t& isz, float* out) {
+  float2 v[8][3];
+  uint64_t inner[8];
+  const bool any = !leaf || payload;
+  // (8-byte aligned: 32-byte records from their third float on, 24-byte caches)
+  const float2* row = (const float2*)(leaf ? leaf_rec + i * 8 + 2 : A.cache + (coff + i) * 6);
+  const uint32_t step = leaf ? 4 : 3;
 #pragma unroll
-  for (int k = 0; k < 8; k++) {
-    float a0 = 0.0f, a1 = 0.0f, a2 = 0.0f, b0 = 0.0f, b1 = 0.0f, b2 = 0.0f;
-    if (j < je && (int)(code[j] & 7) == k) {
-      notnull += 1.0f;
-      const float* r = nullptr;
-      if (!leaf) {
-        isz += A.isize[coff + j];
-        r = A.cache + (coff + j) * 6;
-      } else if (payload) {
-        r = leaf_rec + j * 8 + 2;
-      }
-      if (r) {
-        a0 = r[0];
-        a1 = r[1];
-        a2 = r[2];
-        b0 = r[3];
-        b1 = r[4];
-        b2 = r[5];
-      }
-      j++;
-    }
-    c0 = c0 + a0;
-    c1 = c1 + a1;
-    c2 = c2 + a2;
-    n0 = n0 + b0;
-    n1 = n1 + b1;
-    n2 = n2 + b2;
+  for (uint32_t r = 0; r < 8; r++) {
+    const bool live = r < cnt;
+#pragma unroll
+    for (int q = 0; q < 3; q++) v[r][q] = live && any ? row[r * step + q] : make_float2(0.0f, 0.0f);
+    inner[r] = live && !leaf ? A.isize[coff + i + r] : 0ull;
   }
-  out[0] = c0 / notnull;
-  out[1] = c1 / notnull;
-  out[2] = c2 / notnull;
-  const float t0 = n0 / notnull, t1 = n1 / notnull, t2 = n2 / notnull;
+  float s[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  isz = 1;
+#pragma unroll
+  for (int r = 0; r < 8; r++) {
+    isz += inner[r];
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      s[2 * q] = s[2 * q] + v[r][q].x;
+      s[2 * q + 1] = s[2 * q + 1] + v[r][q].y;
+    }
+  }
+  const float notnull = (float)cnt;
+  out[0] = s[0] / notnull;
+  out[1] = s[1] / notnull;
+  out[2] = s[2] / notnull;
+  const float t0 = s[3] / notnull, t1 = s[4] / notnull, t2 = s[5] / notnull;
   const float inv = 1.0f / sqrtf((t0 * t0 + t1 * t1) + t2 * t2);
   out[3] = t0 * inv;
   out[4] = t1 * inv;
@@ -210,7 +206,7 @@ struct ParentStore {
         }
         const uint64_t pc = T.parent(cj[0]);
         uint32_t m = 0;
-        uint64_t sz = 1, je = i;
+        uint64_t sz = 1;
         bool more = true;
 #pragma unroll
         for (int k = 0; k < 8; k++) {
@@ -219,7 +215,6 @@ struct ParentStore {
             m |= 1u << (cj[k] & 7);
             if (csize) A.sib[M.off[h] + i + k] = sz - 1 - (uint64_t)k;
             sz += sj[k];
-            je = i + k + 1;
           }
         }
         A.code[base + ex] = pc;
@@ -230,8 +225,8 @@ struct ParentStore {
         uint64_t isz = 1;
         if (A.isize) {
           float avg[6];
-          average_children(A, leaf ? 0 : M.off[h], leaf, leaf_rec, jobs[jb].payload, code, i,
-                           je, isz, avg);
+          average_children(A, leaf ? 0 : M.off[h], leaf, leaf_rec, jobs[jb].payload, i,
+                           (uint32_t)__popc(m), isz, avg);
           A.isize[base + ex] = isz;
 #pragma unroll
           for (int q = 0; q < 6; q++) A.cache[(base + ex) * 6 + q] = avg[q];
@@ -419,11 +414,14 @@ __device__ __forceinline__ void emit_level_node(const Arena& A, const LevelMeta&
     const uint32_t pcnt = (uint32_t)__popc((uint32_t)A.mask[po]);
     const uint64_t ps = A.start[po];
     const uint64_t cb = ps + A.size[po] - 1 - pcnt;
-    st = ps;
-    for (uint64_t j = f; j < i; j++) st += A.size[co + j] - 1;
+    const uint64_t sib = A.sib[co + i];
+    st = ps + sib;
     if (lv) {
       pst = A.pstart[po];
-      for (uint64_t j = f; j < i; j++) pst += levels_weight(A, co + j, J.payload);
+      if (J.payload)
+        pst += sib + (i - f);  // the siblings' sizes
+      else
+        for (uint64_t j = f; j < i; j++) pst += A.isize[co + j];
     }
     pos = cb + (i - f);
   }
