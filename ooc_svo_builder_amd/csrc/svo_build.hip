@@ -1327,9 +1327,10 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
     bound[h] = std::min(bound[h - 1], b);
     if (fast && h == 4) bound[h] = NB;
   }
-  // a batch's last upload usually holds these already; a single job goes by kernel argument
+  // a batch's last upload usually holds these already (the kernels of a tagged build read them
+  // there, a batch of one job as well); the plain flow's job goes by kernel argument
   // (not into a graph, whose launches are compared by their argument bytes)
-  const bool job_arg = n_jobs == 1 && !c.graphs;
+  const bool job_arg = !tagged && !c.graphs;
   SVO_TRY(ensure(c.jobdev, n_jobs * sizeof(JobDev)));
   if (c.clear_counters) {  // no pass came first
     SVO_TRY(fill_u64(c.counters.as<uint64_t>(), 0, kNumCounters, c.stream));

@@ -61,6 +61,22 @@ def test_small_jobs_of_a_batch():
                 assert data[r.data_offset:r.data_offset + r.n_data].tobytes() == w_data.tobytes()
 
 
+@pytest.mark.parametrize("graphs", [False, True])
+@pytest.mark.parametrize("payload", [False, True])
+@pytest.mark.parametrize("G,n", [(16, 3), (64, 30), (256, 60), (512, 4000)])
+def test_a_batch_of_one_job(G, n, payload, graphs):
+    """Its descriptor is the uploaded one, with graphs or without, on few bricks and on many."""
+    tris = _mesh(np.random.default_rng(n), n, 2.0 / G, payload)
+    w_nodes, w_data, hz, _, nf = oracle.pipeline(tris, payload, G, 2048)
+    with SvoContext(0) as ctx:
+        ctx.set_graphs(graphs)
+        for _ in range(3):
+            (r,), info = ctx.batch_run([dict(records=tris, payload=payload, gridsize=G)])
+            assert (r.n_nodes, r.n_data, r.nfilled, r.hazard) == (len(w_nodes), len(w_data), nf, hz)
+            assert ctx.nodes(info.n_nodes).tobytes() == w_nodes.tobytes()
+            assert ctx.data(info.n_data).tobytes() == w_data.tobytes()
+
+
 @pytest.mark.parametrize("direct", [0, 16])
 @pytest.mark.parametrize("order", ["as made", "shuffled", "doubled"])
 @pytest.mark.parametrize("mesh", ["terrain", "spikes", "heap"])
