@@ -1293,8 +1293,8 @@ __device__ __forceinline__ float coord_over(uint32_t x, float d, float inv_d, bo
 }
 // The record of voxel 'code' won by triangle t: BarycentricCoords.h:4-32; colour modes of
 // main.cpp:373-382.
-__device__ __forceinline__ void put_payload_record(const JobDev& J, uint64_t code, uint32_t t,
-                                                   float* __restrict__ r) {
+__device__ __forceinline__ void make_payload_record(const JobDev& J, uint64_t code, uint32_t t,
+                                                    uint4& q0, uint4& q1) {
   float col0, col1, col2, nr0, nr1, nr2;
   const gfloat_t* p = (const gfloat_t*)J.tris + (uint64_t)t * 21;
   const float v0x = p[0], v0y = p[1], v0z = p[2];
@@ -1362,7 +1362,6 @@ __device__ __forceinline__ void put_payload_record(const JobDev& J, uint64_t cod
     col1 = (b + 1.0f) / 2.0f;
     col2 = (c + 1.0f) / 2.0f;
   }
-  uint4 q0, q1;
   q0.x = (uint32_t)code;
   q0.y = (uint32_t)(code >> 32);
   q0.z = __float_as_uint(canon_nan(col0));
@@ -1371,8 +1370,6 @@ __device__ __forceinline__ void put_payload_record(const JobDev& J, uint64_t cod
   q1.y = __float_as_uint(canon_nan(nr0));
   q1.z = __float_as_uint(canon_nan(nr1));
   q1.w = __float_as_uint(canon_nan(nr2));
-  ((uint4*)r)[0] = q0;
-  ((uint4*)r)[1] = q1;
 }
 
 // Position of the n-th set bit of w (n below its count)
@@ -1404,14 +1401,21 @@ __device__ __forceinline__ uint32_t nth_set_bit(uint64_t w, uint32_t n) {
 // Bound by memory: 32 bytes written a voxel, the cells' words, and the winners' records
 // gathered. A pass that wrote every voxel's code and winner (a lane per word, its voxels one
 // after the other) and one that read them back took 242 + 336 us on 17M voxels of a rough
-// sphere; this one 403 (1.9M voxels of a fine terrain: 34 + 71 us, 81).
+// sphere; this one 403 (1.9M voxels of a fine terrain: 34 + 71 us, 81). With kStaged (more than
+// kStagePayload bricks) 64 records go through LDS and out in whole KiB past the caches, not as 16
+// bytes of every 32, and cells are zeroed by the 64-byte pieces that hold marks: 392 -> 300 us,
+// the terrain 72 -> 61, 64 mixed meshes 876 -> 682 (2500 bricks: 17, staged 18.6).
+constexpr uint64_t kStagePayload = 4096;
+template <bool kStaged>
 __global__ __launch_bounds__(256) void k_payload_bricks(
     const uint32_t* __restrict__ occ, const ull* __restrict__ n_occ_ptr,
     const VoxParams* __restrict__ units, const uint64_t* __restrict__ ubase, uint32_t n_units,
     const ull* __restrict__ words, const uint64_t* __restrict__ boff,
     const JobDev* __restrict__ jobs, JobDev j0, uint64_t s0, float* __restrict__ out, ull* ctr) {
   __shared__ uint8_t s_slot[256];
+  __shared__ uint4 s_stage[kStaged ? 256 / kWave : 1][2 * kWave];
   uint8_t* slot = s_slot + (threadIdx.x / kWave) * kWave;
+  uint4* stage = s_stage[kStaged ? threadIdx.x / kWave : 0];
   const int lane = lane_id();
   const uint64_t n_occ = *n_occ_ptr;
   for (uint64_t wv = wave_global(); wv < n_occ; wv += waves_total()) {
@@ -1448,8 +1452,23 @@ __global__ __launch_bounds__(256) void k_payload_bricks(
       if (k < n) {
         if (cell == 0u)  // cannot happen: the words were made from the cells
           atomicAdd(&ctr[kCtrError], 1ull);
-        else
-          put_payload_record(J, code0 + v, ~cell, rec + (uint64_t)k * 8);
+        else {
+          uint4 q0, q1;
+          make_payload_record(J, code0 + v, ~cell, q0, q1);
+          uint4* to = kStaged ? stage + 2 * lane : (uint4*)(rec + (uint64_t)k * 8);
+          to[0] = q0;
+          to[1] = q1;
+        }
+      }
+      if constexpr (kStaged) {
+        wave_lds_sync();
+        const uint32_t quads = 2 * min(n - k0, (uint32_t)kWave);
+        u32x4* to = (u32x4*)(rec + (uint64_t)k0 * 8);
+#pragma unroll
+        for (uint32_t q = 0; q < 2; q++)
+          if (lane + kWave * q < quads)
+            __builtin_nontemporal_store(((const u32x4*)stage)[lane + kWave * q], to + lane + kWave * q);
+        wave_lds_sync();
       }
       v = v2;
       cell = cell2;
@@ -1464,7 +1483,12 @@ __global__ __launch_bounds__(256) void k_payload_bricks(
         if ((lane >> 4) == q) mine = wi;
         ne &= ne - 1ull;
       }
-      if (mine < 64u) ((gquad_t*)(cells + mine * 64u))[lane & 15] = u32x4{0u, 0u, 0u, 0u};
+      // (only the 64-byte pieces that hold marks)
+      const uint32_t lo = (uint32_t)__shfl((int)(uint32_t)word, (int)(mine & 63u), kWave);
+      const uint32_t hi = (uint32_t)__shfl((int)(uint32_t)(word >> 32), (int)(mine & 63u), kWave);
+      const uint32_t piece = ((lane & 8) ? hi : lo) >> ((lane & 4) ? 16 : 0);
+      if (mine < 64u && (piece & 0xFFFFu))
+        ((gquad_t*)(cells + mine * 64u))[lane & 15] = u32x4{0u, 0u, 0u, 0u};
     }
   }
 }
@@ -1501,8 +1525,13 @@ __global__ __launch_bounds__(256) void k_payload_records(
   const uint32_t t = winner[i];
   if (t == 0xFFFFFFFFu)  // cannot happen: both passes evaluate the same predicates
     atomicAdd(&ctr[kCtrError], 1ull);
-  else
-    put_payload_record(J, code, t, out + (J.dbase + 1 + (s0 + i - J.voff)) * 8);
+  else {
+    uint4* r = (uint4*)(out + (J.dbase + 1 + (s0 + i - J.voff)) * 8);
+    uint4 q0, q1;
+    make_payload_record(J, code, t, q0, q1);
+    r[0] = q0;
+    r[1] = q1;
+  }
 }
 
 // ---------------------------------------------------------------- partition kernels
@@ -2544,7 +2573,8 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
         SVO_TRY(hipGetLastError());
       } else if (any_payload) {
         ktimer_begin(c, "payload_records");
-        SVO_LAUNCH(k_payload_bricks, dim3(brick_grid(n_occ)), dim3(256), 0, c.stream,
+        SVO_LAUNCH(n_occ > kStagePayload ? k_payload_bricks<true> : k_payload_bricks<false>,
+                   dim3(brick_grid(n_occ)), dim3(256), 0, c.stream,
                    c.occ_list.as<uint32_t>(), (const ull*)(ctr + kCtrNumOcc),
                    (const VoxParams*)d_units, d_ubase, nu, (const ull*)pool_words,
                    c.bcount.as<uint64_t>(),
