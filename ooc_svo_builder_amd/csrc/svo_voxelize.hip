@@ -1860,27 +1860,36 @@ hipError_t read_back(Context& c, const ReadReq* reqs, int n) {
 }
 
 // n elements of 16 bytes (8-byte aligned: wide accesses need no more) and, with tail, one of 8
-// after them; four in flight a thread, streamed past the caches. A copy of few blocks also
-// raises the read-back flag: the block that finishes last, by a counter it leaves at zero for
-// the next copy (flag = nullptr: no flag).
+// after them: a block copies kItems x 4 KB in one piece, a wave's load or store 1 KB of it. A copy
+// of few blocks also raises the read-back flag: the block that finishes last, by a counter it
+// leaves at zero for the next copy (flag = nullptr: no flag).
 //
-// Bound by memory: 5.1 TB/s read and written at 0.7 GB.
+// Bound by memory: 6.2 TB/s read and written at 0.5 GB, 6.3 at 2.4 GB, 7.0 at 0.25 GB, a thread an
+// element, streamed past the caches on the way out only. Four elements a thread a grid apart (32
+// MB: the same channels) and streamed both ways reached 5.2, 5.1 and 5.0; four in one piece 6.2,
+// 5.7 and 6.2.
 typedef u32x4 u32x4_u __attribute__((aligned(8)));
+template <int kItems>
 __global__ __launch_bounds__(256) void k_copy(u32x4_u* __restrict__ dst,
                                               const u32x4_u* __restrict__ src, uint64_t n,
                                               int tail, volatile uint32_t* flag, uint32_t seq,
                                               ull* done) {
-  const uint64_t step = (uint64_t)gridDim.x * 256;
-  uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-  if (tail && i == 0) *(uint64_t*)(dst + n) = *(const uint64_t*)(src + n);
-  for (; i + 3 * step < n; i += 4 * step) {
-    u32x4 v[4];
+  if (tail && blockIdx.x == 0 && threadIdx.x == 0)
+    *(uint64_t*)(dst + n) = *(const uint64_t*)(src + n);
+  for (uint64_t b = (uint64_t)blockIdx.x * 256 * kItems; b < n;
+       b += (uint64_t)gridDim.x * 256 * kItems) {
+    u32x4 v[kItems];
 #pragma unroll
-    for (int k = 0; k < 4; k++) v[k] = __builtin_nontemporal_load(src + i + k * step);
+    for (int k = 0; k < kItems; k++) {
+      const uint64_t i = b + 256 * k + threadIdx.x;
+      if (i < n) v[k] = src[i];
+    }
 #pragma unroll
-    for (int k = 0; k < 4; k++) __builtin_nontemporal_store(v[k], dst + i + k * step);
+    for (int k = 0; k < kItems; k++) {
+      const uint64_t i = b + 256 * k + threadIdx.x;
+      if (i < n) __builtin_nontemporal_store(v[k], dst + i);
+    }
   }
-  for (; i < n; i += step) __builtin_nontemporal_store(__builtin_nontemporal_load(src + i), dst + i);
   if (!flag) return;
   __builtin_amdgcn_s_waitcnt(0);  // the wave's stores have reached the L2
   __syncthreads();
@@ -1898,21 +1907,23 @@ __global__ __launch_bounds__(256) void k_copy(u32x4_u* __restrict__ dst,
 constexpr unsigned kCopyFlagBlocks = 128;
 hipError_t copy_records(Context& c, void* dst, const void* src, size_t bytes) {
   const uint64_t n = bytes / 16;
-  const unsigned grid =
-      n <= kCopyFlagBlocks * 1024ull
-          ? (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((n + 255) / 256, kCopyFlagBlocks))
-          : (unsigned)std::min<uint64_t>((n + 255) / 256, 8192);
-  const bool flagged = grid <= kCopyFlagBlocks;
-  uint32_t seq = 0;
-  if (flagged) {
-    SVO_TRY(ensure_hread(c, 256));
-    seq = ++c.hread_seq;
+  const int tail = bytes % 16 != 0;
+  if (n > kCopyFlagBlocks * 1024ull) {
+    SVO_LAUNCH(k_copy<1>, dim3((unsigned)std::min<uint64_t>((n + 255) / 256, 1u << 24)), dim3(256),
+               0, c.stream, (u32x4_u*)dst, (const u32x4_u*)src, n, tail,
+               (volatile uint32_t*)nullptr, 0u, (ull*)nullptr);
+    SVO_TRY(hipGetLastError());
+    return read_back(c, nullptr, 0);
   }
-  SVO_LAUNCH(k_copy, dim3(grid), dim3(256), 0, c.stream, (u32x4_u*)dst, (const u32x4_u*)src, n,
-             (int)(bytes % 16 != 0), flagged ? (volatile uint32_t*)c.hread : nullptr, seq,
-             c.counters.as<ull>() + kCtrCopyDone);
+  SVO_TRY(ensure_hread(c, 256));
+  const uint32_t seq = ++c.hread_seq;
+  auto copy = [&](auto kernel, uint64_t per_block) {
+    SVO_LAUNCH(kernel, dim3((unsigned)std::max<uint64_t>(1, (n + per_block - 1) / per_block)),
+               dim3(256), 0, c.stream, (u32x4_u*)dst, (const u32x4_u*)src, n, tail,
+               (volatile uint32_t*)c.hread, seq, c.counters.as<ull>() + kCtrCopyDone);
+  };
+  n <= kCopyFlagBlocks * 256ull ? copy(k_copy<1>, 256) : copy(k_copy<4>, 1024);
   SVO_TRY(hipGetLastError());
-  if (!flagged) return read_back(c, nullptr, 0);
   t_syncs++;
   return wait_flag(c, seq);
 }
