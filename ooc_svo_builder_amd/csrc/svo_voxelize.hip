@@ -266,6 +266,11 @@ struct ActArgs {
 
 // What an action keeps per wave in LDS.
 struct NoCache {};
+// The action of a tile whose lanes walk their own triangles.
+template <typename Act>
+struct DirectOf {
+  using type = Act;
+};
 
 // Brick allocation without atomics: the touch pass stores 1 into the table entry of
 // every brick a column's candidate voxels fall in; a scan over the table then numbers the
@@ -349,35 +354,41 @@ struct MarkDenseT {
 using MarkDenseAction = MarkDenseT<false>;
 using MarkDenseWideAction = MarkDenseT<true>;
 
-// Payload marks, gathered in LDS: a wave keeps kLines lines of 32 cells (128 bytes
-// of the grid), takes the maximum of ~triangle there, and gives a line to memory whole, a half
-// wave a line. A cell whose line's place holds another line goes to memory at once.
+// Payload marks, gathered in LDS: a wave keeps kLines lines of 32 cells (128 bytes of the grid),
+// takes the maximum of ~triangle there, and gives a line to memory whole, a half wave a line. A
+// cell whose line's place holds another line goes to memory at once.
 //
 // The winner atomics bound these marks: at agent scope they are not done in the (per XCD) L2
 // but at the memory behind it, ~23 G requests a second whatever they hold (TCC_EA0_ATOMIC =
 // TCC_ATOMIC; 12.7 M of them for 17M voxels of a rough sphere at 1024 in 535 us, 4.3 M for a
 // fine terrain in 218), so what counts is how many requests there are, and neighbouring
 // triangles share both cells and lines.
+//
+// Lanes walking their own triangles have 64 lines, in the memory that rows and columns are laid
+// out in otherwise; a tile laid out so (triangles of more columns, whose lines are few hits each)
+// has 16 of its own. With 64 lines besides that memory two blocks fitted a CU instead of three:
+// the fine terrain 153 us, 134 so; 320,000 triangles at 512 73 and 61; the rough sphere 453 and 457.
 constexpr uint32_t kLineBits = 5;
 constexpr uint32_t kLineCells = 1u << kLineBits;
-constexpr uint32_t kLines = 64;
-constexpr uint32_t kLinesFull = 40;  // lines held at which a wave gives them to memory
+template <uint32_t kLines>
 struct MarkLines {
   uint32_t tag[kLines];  // line + 1, 0 = free
   uint32_t val[kLines][kLineCells];
 };
-struct MarkGatherAction {
+template <uint32_t kLines>
+struct MarkGather {
   static constexpr bool kTouch = false;
+  static constexpr uint32_t kFull = kLines * 5 / 8;  // lines held at which they go to memory
   using Unordered = MarkDenseWideAction;
-  using Cache = MarkLines;
+  using Cache = MarkLines<kLines>;
   __device__ static bool narrow(const VoxParams&) { return false; }
   gbyte_t* table;
   gbyte_t* words;
   gword_t* cells;
   uint64_t base;
-  MarkLines* L;
-  __device__ static MarkGatherAction make(const ActArgs& A, const VoxParams& P, Cache* L) {
-    MarkGatherAction m;
+  Cache* L;
+  __device__ static MarkGather make(const ActArgs& A, const VoxParams& P, Cache* L) {
+    MarkGather m;
     m.table = (gbyte_t*)(A.table + P.table_base);
     m.words = (gbyte_t*)(A.cflags + P.table_base * kBrickWords);
     m.cells = (gword_t*)P.grid8;
@@ -409,10 +420,10 @@ struct MarkGatherAction {
   __device__ static void drain(const ActArgs& A, const VoxParams& P, Cache* L, bool all) {
     const int lane = lane_id();
     wave_lds_sync();
-    const uint32_t tag = L->tag[lane];
+    const uint32_t tag = lane < (int)kLines ? L->tag[lane] : 0u;
     uint64_t used = __ballot(tag != 0u);
-    if (!used || (!all && (uint32_t)__popcll(used) < kLinesFull)) return;  // uniform
-    const MarkGatherAction m = make(A, P, L);
+    if (!used || (!all && (uint32_t)__popcll(used) < kFull)) return;  // uniform
+    const MarkGather m = make(A, P, L);
     while (used) {  // two lines at a time
       const int l0 = __ffsll((long long)used) - 1;
       used &= used - 1ull;
@@ -433,11 +444,16 @@ struct MarkGatherAction {
         }
       }
     }
-    L->tag[lane] = 0u;
+    if (lane < (int)kLines) L->tag[lane] = 0u;
     wave_lds_sync();
   }
 };
-static_assert(kLines == kWave && kLineCells == kWave / 2, "drain: a place a lane, two lines a step");
+static_assert(kLineCells == kWave / 2, "drain: two lines a step");
+using MarkGatherAction = MarkGather<16>;
+template <>
+struct DirectOf<MarkGatherAction> {
+  using type = MarkGather<64>;
+};
 
 struct MarkPoolAction {
   static constexpr bool kTouch = false;
@@ -747,9 +763,9 @@ __device__ __forceinline__ uint32_t large_jobs(const LargeList& B, ull* ctr, uin
   return fits ? rows : rows | kAllRows;
 }
 
-// blocks of the small tier on a CU (what an action keeps in LDS leaves room for two)
+// blocks of the small tier on a CU (what an action keeps in LDS leaves room for three)
 template <typename Act>
-constexpr int kTileBlocks = std::is_same<typename Act::Cache, NoCache>::value ? 4 : 2;
+constexpr int kTileBlocks = std::is_same<typename Act::Cache, NoCache>::value ? 4 : 3;
 template <typename Act>
 __global__ __launch_bounds__(kTile, kTileBlocks<Act>) void k_vox_tile(const VoxParams* __restrict__ units,
                                                        uint32_t n_units,
@@ -770,6 +786,11 @@ __global__ __launch_bounds__(kTile, kTileBlocks<Act>) void k_vox_tile(const VoxP
     for (uint32_t k = lane_id(); k < sizeof(*cache) / 4; k += kWave) ((uint32_t*)cache)[k] = 0u;
     wave_lds_sync();
   }
+  using Direct = typename DirectOf<Act>::type;
+  constexpr bool kOverlay = !std::is_same<typename Direct::Cache, NoCache>::value;
+  static_assert(!kOverlay || sizeof(typename Direct::Cache) <= sizeof(WalkLds), "overlay");
+  typename Direct::Cache* const overlay = kOverlay ? (typename Direct::Cache*)&L : nullptr;
+  bool clean = false;  // the overlay is zero (as a drain leaves it)
   ull* ctr = A.ctr;
   const int lane = lane_id();
   // Runs of geometry-only and of payload tiles, mixed evenly (payload_runs: 2^32 x the payload
@@ -868,13 +889,19 @@ __global__ __launch_bounds__(kTile, kTileBlocks<Act>) void k_vox_tile(const VoxP
       }
     }
     if (direct) {
-      if (ncols) {
-        Act act = Act::make(A, P, cache);
-        walk_all_columns(K, P, act, Act::narrow(P));
+      if (kOverlay && !clean) {
+        for (uint32_t k = lane; k < sizeof(*overlay) / 4; k += kWave) ((uint32_t*)overlay)[k] = 0u;
+        wave_lds_sync();
+        clean = true;
       }
-      Act::drain(A, P, cache, true);
+      if (ncols) {
+        Direct act = Direct::make(A, P, overlay);
+        walk_all_columns(K, P, act, Direct::narrow(P));
+      }
+      Direct::drain(A, P, overlay, true);
       continue;
     }
+    clean = false;
     if (__ballot(rows != 0)) {
       wave_lds_sync();
       walk_rows<Act>(L, cache, P, A, K, nv, rows, 0u);
