@@ -577,7 +577,7 @@ constexpr uint32_t kQueues = 8;        // tile queues per persistent launch
 constexpr uint32_t kTileRun = 16;      // neighbouring tiles in one queue
 constexpr uint32_t kQueueStride = 16;  // words between their counters (own cache lines)
 constexpr uint32_t kQueueWords = kQueues * kQueueStride;
-constexpr uint64_t kLargeWalkMax = 1u << 18;  // large triangles with stored constants
+constexpr uint64_t kLargeWalkMax = 1u << 16;  // large triangles with stored constants (19 MB)
 constexpr int kSkipDense = 1;   // units voxelized in a dense grid (touch pass)
 constexpr int kSkipBinary = 2;  // geometry-only units (payload winner pass)
 
