@@ -577,13 +577,15 @@ __global__ __launch_bounds__(256) void k_emit_leaves(Arena A, LevelMeta M, Tags 
 //
 // Bound by the writes, 24 bytes a node. Finding each record's node by searches in the ranges'
 // offsets took 740 vector instructions a brick, two thirds of the kernel's time. With kStaged
-// (more than kStageBricks bricks) a window's records go through LDS and out 16 bytes a lane, a
-// third of the write requests of three 8-byte stores a record: 3.6 -> 4.4 TB/s on 30M nodes
-// (198 -> 165 us), 64 mixed meshes 1107 -> 955 us, a 6M-triangle soup in 8 partitions 1660 ->
-// 1567. A few bricks wait for the LDS longer than for the stores: 900 of them 11.3 us, staged 13.2.
+// (more than kStageBricks bricks) a window's records go through LDS and out by whole 128-byte
+// lines, past the caches; a line shared with another brick goes through them. Three 8-byte stores
+// a record, 16 bytes a lane staged but not by lines, by lines: 30M nodes 198, 165, 143 us (5.0
+// TB/s), 64 mixed meshes 1107, 955, 894, a 6M-triangle soup in 8 partitions 1660, 1501, 1242 (past
+// the caches without regard to lines the mixed meshes took 1190). A few bricks wait for the LDS
+// longer than for the stores: 900 of them 11.3 us, staged 13.2.
 constexpr int kEmitWaves = 4;  // waves per block of k_emit_bricks
 typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
-typedef u64x2 u64x2_u __attribute__((aligned(8)));
+constexpr uint32_t kLineWords = 16;  // 64-bit words of a memory line
 constexpr int kInnerMax = 8 + 64 + 512;                        // inner nodes below a brick node
 constexpr int kInnerBits = (kBrickVox + kInnerMax + 63) / 64 * 2;  // bitmap, 32-bit words
 
@@ -610,7 +612,7 @@ __global__ __launch_bounds__(kWave * kEmitWaves) void k_emit_bricks(
   __shared__ uint32_t s_inner[kEmitWaves][kInnerMax];  // first child (relative to S) | mask << 16
   __shared__ uint32_t s_bits[kEmitWaves][kInnerBits + 2];
   __shared__ uint64_t s_offs[256];  // offsets of every child mask
-  __shared__ __attribute__((aligned(16))) uint64_t s_rec[kStaged ? kEmitWaves : 1][3 * kWave];
+  __shared__ __attribute__((aligned(16))) uint64_t s_rec[kStaged ? kEmitWaves : 1][kLineWords + 3 * kWave];
   const int ws = threadIdx.x / kWave;
   const int lane = lane_id();
   const int g = lane >> 3, q = lane & 7;
@@ -706,6 +708,11 @@ __global__ __launch_bounds__(kWave * kEmitWaves) void k_emit_bricks(
   uint64_t leaf0 = payload ? 1ull + (bvo - J.voff) : 1ull;
   if (kPlaced && leaf0 >= (payload ? 1ull : 2ull)) leaf0 += J.data_add;
   uint32_t prior = 0;  // inner nodes before the window
+  // staged words lie in rec as in their 128-byte lines: 'fill' words wait there for their line's
+  // others, the first 'skip' of them not the brick's; line = the first one's place
+  const uint32_t lead = (uint32_t)((uintptr_t)out >> 3) % kLineWords;
+  uint32_t fill = lead, skip = lead;
+  uint64_t* line = out - lead;
   for (uint32_t r0 = 0; r0 < R; r0 += kWave) {
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)bits[r0 >> 5]);
     const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)bits[(r0 >> 5) + 1]);
@@ -724,23 +731,42 @@ __global__ __launch_bounds__(kWave * kEmitWaves) void k_emit_bricks(
         d1 = 0;
         d2 = ~0ull;
       }
-      uint64_t* to = kStaged ? rec + 3 * lane : out + 3 * (uint64_t)r;
+      uint64_t* to = kStaged ? rec + fill + 3 * lane : out + 3 * (uint64_t)r;
       to[0] = d0;
       to[1] = d1;
       to[2] = d2;
     }
     if constexpr (kStaged) {
       wave_lds_sync();
-      const uint32_t words = 3 * min(R - r0, (uint32_t)kWave);
-      uint64_t* to = out + 3 * (uint64_t)r0;
+      const uint32_t total = fill + 3 * min(R - r0, (uint32_t)kWave);
+      const uint32_t whole = total / kLineWords * kLineWords;
+      const uint32_t words = r0 + kWave >= R ? total : whole;  // to store now
 #pragma unroll
       for (uint32_t k = 0; k < 2; k++) {
         const uint32_t at = 2 * (lane + kWave * k);
-        if (at + 1 < words)
-          *(u64x2_u*)(to + at) = *(const u64x2*)(rec + at);
-        else if (at < words)
-          to[at] = rec[at];
+        if (at < words) {
+          const u64x2 v = *(const u64x2*)(rec + at);
+          const bool first = at >= skip, second = at + 1 < words && at + 1 >= skip;
+          if (at >= whole || at / kLineWords < (skip + kLineWords - 1) / kLineWords) {
+            // a line shared with another brick: through the cache
+            if (first && second)
+              *(u64x2*)(line + at) = v;
+            else if (first)
+              line[at] = v.x;
+            else if (second)
+              line[at + 1] = v.y;
+          } else {
+            __builtin_nontemporal_store(v, (u64x2*)(line + at));
+          }
+        }
       }
+      uint64_t rest = 0;
+      if (lane < (int)kLineWords) rest = rec[whole + lane];
+      wave_lds_sync();
+      if (lane < (int)kLineWords) rec[lane] = rest;
+      line += whole;
+      fill = total - whole;
+      skip = 0;
       wave_lds_sync();
     }
     prior += (uint32_t)__popc(lo) + (uint32_t)__popc(hi);
