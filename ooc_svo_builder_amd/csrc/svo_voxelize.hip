@@ -305,19 +305,23 @@ struct TouchAction {
 //    (touch pass + table scan), cached per thread.
 // Both store through global (not generic) pointers.
 // kWide: some units of the pass carry payload (4-byte cells; the unit's wide flag decides
-// per voxel); otherwise every cell is a byte.
-template <bool kWide>
+// per voxel); otherwise every cell is a byte. kSmall: no unit spans more than 2^32 voxels, so a
+// voxel's place is 32 bits: the upper half of the Morton stepping goes, and a store takes it as
+// its offset from a scalar address (64 mixed meshes 2500 -> 2467 us, payload terrain at 1024 134 ->
+// 130).
+template <bool kWide, bool kSmall>
 struct MarkDenseT {
   static constexpr bool kTouch = false;
-  // the same action for lanes in no order of their triangles (queued columns)
-  using Unordered = MarkDenseT<kWide>;
+  using Rel = std::conditional_t<kSmall, uint32_t, uint64_t>;
+  // the same action for queued columns
+  using Unordered = MarkDenseT<kWide, kSmall>;
   using Cache = NoCache;  // per wave, in LDS
   // whether a direct walk narrows its rows to their intervals
   __device__ static bool narrow(const VoxParams& P) { return !kWide || !P.wide; }
   gbyte_t* table;  // the unit's table segment, a byte per quarter of a brick
   gbyte_t* words;  // the unit's word flags (payload units)
   gbyte_t* bytes;
-  uint64_t base;  // code of the first voxel of the unit's first brick
+  Rel base;  // code of the first voxel of the unit's first brick
   int wide;
   uint32_t cquarter = 0xFFFFFFFFu, cword = 0xFFFFFFFFu;  // the last ones marked
   __device__ static MarkDenseT make(const ActArgs& A, const VoxParams& P, Cache*) {
@@ -325,13 +329,13 @@ struct MarkDenseT {
     m.table = (gbyte_t*)(A.table + P.table_base);
     m.words = (gbyte_t*)(A.cflags + P.table_base * kBrickWords);
     m.bytes = (gbyte_t*)P.grid8;
-    m.base = P.bstart;
+    m.base = (Rel)P.bstart;
     m.wide = kWide ? P.wide : 0;
     return m;
   }
   __device__ __forceinline__ void touch(uint64_t) {}
   __device__ __forceinline__ void add(uint64_t code, uint32_t tri) {
-    const uint64_t rel = code - base;
+    const Rel rel = (Rel)code - base;
     const uint32_t q = (uint32_t)(rel >> (kBrickBits - 2));
     if (kWide && wide) {
       // the lowest covering triangle as the largest ~tri (0 = unmarked)
@@ -351,8 +355,6 @@ struct MarkDenseT {
   }
   __device__ static void drain(const ActArgs&, const VoxParams&, Cache*, bool) {}
 };
-using MarkDenseAction = MarkDenseT<false>;
-using MarkDenseWideAction = MarkDenseT<true>;
 
 // Payload marks, gathered in LDS: a wave keeps kLines lines of 32 cells (128 bytes of the grid),
 // takes the maximum of ~triangle there, and gives a line to memory whole, a half wave a line. A
@@ -375,30 +377,31 @@ struct MarkLines {
   uint32_t tag[kLines];  // line + 1, 0 = free
   uint32_t val[kLines][kLineCells];
 };
-template <uint32_t kLines>
+template <uint32_t kLines, bool kSmall>
 struct MarkGather {
   static constexpr bool kTouch = false;
+  using Rel = std::conditional_t<kSmall, uint32_t, uint64_t>;
   static constexpr uint32_t kFull = kLines * 5 / 8;  // lines held at which they go to memory
-  using Unordered = MarkDenseWideAction;
+  using Unordered = MarkDenseT<true, kSmall>;
   using Cache = MarkLines<kLines>;
   __device__ static bool narrow(const VoxParams&) { return false; }
   gbyte_t* table;
   gbyte_t* words;
   gword_t* cells;
-  uint64_t base;
+  Rel base;
   Cache* L;
   __device__ static MarkGather make(const ActArgs& A, const VoxParams& P, Cache* L) {
     MarkGather m;
     m.table = (gbyte_t*)(A.table + P.table_base);
     m.words = (gbyte_t*)(A.cflags + P.table_base * kBrickWords);
     m.cells = (gword_t*)P.grid8;
-    m.base = P.bstart;
+    m.base = (Rel)P.bstart;
     m.L = L;
     return m;
   }
   __device__ __forceinline__ void touch(uint64_t) {}
   __device__ __forceinline__ void add(uint64_t code, uint32_t tri) {
-    const uint64_t rel = code - base;  // (below 2^35: the dense limit is 2^37 bytes)
+    const Rel rel = (Rel)code - base;  // (below 2^35: the dense limit is 2^37 bytes)
     const uint32_t line = (uint32_t)(rel >> kLineBits);
     // neighbouring lines in neighbouring places (of a 4 x 4 x 4 block of lines: 6 bits), the
     // blocks mixed
@@ -449,10 +452,9 @@ struct MarkGather {
   }
 };
 static_assert(kLineCells == kWave / 2, "drain: two lines a step");
-using MarkGatherAction = MarkGather<16>;
-template <>
-struct DirectOf<MarkGatherAction> {
-  using type = MarkGather<64>;
+template <bool kSmall>
+struct DirectOf<MarkGather<16, kSmall>> {
+  using type = MarkGather<64, kSmall>;
 };
 
 struct MarkPoolAction {
@@ -2184,7 +2186,11 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
   const uint64_t dense_bytes = goff[nu];
   const bool dense = dense_bytes <= c.dense_limit;
   bool geometry_only = true;  // no unit carries payload records
-  for (uint32_t u = 0; u < nu; u++) geometry_only = geometry_only && units[u].stride == 9;
+  bool small_units = true;    // no unit spans more than 2^32 voxels
+  for (uint32_t u = 0; u < nu; u++) {
+    geometry_only = geometry_only && units[u].stride == 9;
+    small_units = small_units && (ubase[u + 1] - ubase[u]) <= (1ull << (32 - kBrickBits));
+  }
   // the table, the word flags, the dense grid and the byte pool are all-zero whenever no pass
   // is running
   const bool new_table = c.table_entries < ntab;
@@ -2304,7 +2310,7 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     using Act = decltype(tag);
     const unsigned tile_grid = (unsigned)std::min<uint64_t>(
         runs * kTileRun / kTileWaves,
-        std::max(1, c.tune.tile_blocks * kTileBlocks<Act> / kTileBlocks<MarkDenseAction>));
+        std::max(1, c.tune.tile_blocks * kTileBlocks<Act> / kTileBlocks<TouchAction>));
     ktimer_begin(c, name);
     SVO_LAUNCH((k_vox_tile<Act>), dim3(tile_grid), dim3(kTile), 0, c.stream, d_units, nu,
                        d_toff, payload_runs, args(), queue, large, tt, collect, skip);
@@ -2373,22 +2379,23 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
       // the large triangles
       // (units of both kinds: the payload marks' lines in LDS would leave room for half the waves
       // of the others; apart, in two launches, 64 mixed meshes took 1.15 + 1.89 ms against 2.74)
-      if (dense && geometry_only)
-        SVO_TRY(tile_pass(MarkDenseAction{}, "vox_small_mark", queues, 1, 0));
-      else if (dense && !toff_kind[0][nu])
-        SVO_TRY(tile_pass(MarkGatherAction{}, "vox_small_mark", queues, 1, 0));
-      else if (dense)
-        SVO_TRY(tile_pass(MarkDenseWideAction{}, "vox_small_mark", queues, 1, 0));
-      else
-        SVO_TRY(tile_pass(TouchAction{}, "vox_small_touch", queues, 1, 0));
-      if (dense) {
+      auto mark_dense = [&](auto small) -> hipError_t {
+        constexpr bool kSmall = decltype(small)::value;
         if (geometry_only)
-          SVO_TRY(large_pass(MarkDenseAction{}, "vox_large_mark", 0));
+          SVO_TRY(tile_pass(MarkDenseT<false, kSmall>{}, "vox_small_mark", queues, 1, 0));
+        else if (!toff_kind[0][nu])
+          SVO_TRY(tile_pass(MarkGather<16, kSmall>{}, "vox_small_mark", queues, 1, 0));
         else
-          SVO_TRY(large_pass(MarkDenseWideAction{}, "vox_large_mark", 0));
+          SVO_TRY(tile_pass(MarkDenseT<true, kSmall>{}, "vox_small_mark", queues, 1, 0));
+        if (geometry_only) return large_pass(MarkDenseT<false, kSmall>{}, "vox_large_mark", 0);
+        return large_pass(MarkDenseT<true, kSmall>{}, "vox_large_mark", 0);
+      };
+      if (dense) {
+        SVO_TRY(small_units ? mark_dense(std::true_type{}) : mark_dense(std::false_type{}));
         // number the flagged bricks in Morton order: table entry = rank + 1, occ = list
         SVO_TRY(occ_scan());
       } else {
+        SVO_TRY(tile_pass(TouchAction{}, "vox_small_touch", queues, 1, 0));
         SVO_TRY(large_pass(TouchAction{}, "vox_large_touch", 0));
         SVO_TRY(occ_scan());
         // mark pass: byte stores into the slots

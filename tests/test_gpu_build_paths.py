@@ -121,6 +121,22 @@ def test_tiles_of_both_kinds_in_one_pass():
                 assert data[r.data_offset:r.data_offset + r.n_data].tobytes() == w_data.tobytes()
 
 
+@pytest.mark.parametrize("payload", [False, True])
+def test_units_past_32_bits(payload):
+    """A unit of 2^33 voxels takes 64-bit places, one of 2^30 (the same in 8 partitions) 32-bit
+    ones; triangles in every octant, some of many columns."""
+    G = 2048
+    rng = np.random.default_rng(9)
+    tris = np.concatenate([_mesh(rng, 150, 2.0 / G, payload, spread=0.49),
+                           _mesh(rng, 20, 30.0 / G, payload)])
+    want = oracle.pipeline(tris, payload, G, 1024)[:2]
+    with SvoContext(0) as ctx:
+        for limit in (8192, 1024):
+            info = ctx.run(tris, payload, G, limit)
+            assert ctx.nodes(info.n_nodes).tobytes() == want[0].tobytes()
+            assert ctx.data(info.n_data).tobytes() == want[1].tobytes()
+
+
 @pytest.mark.parametrize("n_parts", [8, 64, 512])
 @pytest.mark.parametrize("n", [1, 64, 2047, 2048, 2049, 300001])
 def test_partition_lists(n_parts, n):
