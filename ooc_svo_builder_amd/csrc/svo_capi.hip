@@ -311,13 +311,13 @@ void svo_ctx_destroy(svo_ctx* ctx) {
   c.gexec.clear();
   c.glog.clear();
   DevBuf* bufs[] = {&c.tris, &c.jobdev, &c.batch_tris, &c.hitbox, &c.part_lists, &c.unitdev,
-                    &c.table, &c.pool, &c.pool8, &c.grid8, &c.cflags, &c.counters, &c.large_unit,
-                    &c.large_tri, &c.large_rows, &c.large_jobs, &c.occ_list, &c.bcount,
+                    &c.table, &c.pool, &c.pool8, &c.grid8, &c.cflags, &c.counters, &c.large,
+                    &c.occ_list, &c.bcount,
                     &c.wprefix, &c.winner, &c.scan_scratch, &c.codes, &c.records, &c.nodes,
                     &c.lvl_code, &c.lvl_size, &c.lvl_mask, &c.lvl_first, &c.lvl_start,
                     &c.lvl_aux, &c.lvl_leafp, &c.lvl_pidx, &c.lvl_isize, &c.lvl_cache,
                     &c.lvl_pstart, &c.records2, &c.bwords, &c.bcode, &c.bvoff,
-                    &c.scan_status, &c.lvl_sib, &c.up_tiles, &c.bshape, &c.large_walk,
+                    &c.scan_status, &c.lvl_sib, &c.up_tiles, &c.bshape,
                     &c.payload_map};
   for (DevBuf* b : bufs) release(*b);
   stream_release(c);

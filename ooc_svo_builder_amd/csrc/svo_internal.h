@@ -269,8 +269,7 @@ struct Context {
   uint64_t pool_cap = 0;        // slots of pool8 (and of pool) on the touch path
   uint64_t dense_limit = 0;     // largest dense grid in bytes (set from free HBM)
   DevBuf counters;
-  DevBuf large_unit, large_tri, large_rows, large_jobs;
-  DevBuf large_walk;  // set-up of large triangles (capped)
+  DevBuf large;  // large triangles: unit, index, rows per job, jobs, set-ups (capped)
   DevBuf occ_list, bcount, wprefix, winner;
   DevBuf scan_scratch;
   DevBuf scan_status;  // status words of the single-pass scans of a voxelize pass

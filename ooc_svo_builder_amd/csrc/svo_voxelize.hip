@@ -580,11 +580,10 @@ constexpr uint32_t kTileRun = 16;      // neighbouring tiles in one queue
 constexpr uint32_t kQueueStride = 16;  // words between their counters (own cache lines)
 constexpr uint32_t kQueueWords = kQueues * kQueueStride;
 constexpr uint64_t kLargeWalkMax = 1u << 16;  // large triangles with stored constants (19 MB)
-constexpr int kSkipDense = 1;   // units voxelized in a dense grid (touch pass)
-constexpr int kSkipBinary = 2;  // geometry-only units (payload winner pass)
+constexpr int kSkipBinary = 1;  // geometry-only units (payload winner pass)
 
 __device__ __forceinline__ bool skipped(const VoxParams& P, int skip) {
-  return ((skip & kSkipDense) && P.dense) || ((skip & kSkipBinary) && P.stride == 9);
+  return (skip & kSkipBinary) && P.stride == 9;
 }
 
 // Per wave: the tile's triangles, the current rows, a 64-entry slot array and the queue of
@@ -2261,12 +2260,11 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     SVO_TRY(ensure_keep(c.bshape, (nb0 + ntab) * 4, nb0 * 4, c.stream));
   }
   ull* pool_words = dense ? c.bwords.as<ull>() + nb0 * kBrickWords : c.pool.as<ull>();
-  SVO_TRY(ensure(c.large_unit, ntri * 4));
-  SVO_TRY(ensure(c.large_tri, ntri * 4));
-  SVO_TRY(ensure(c.large_rows, ntri * 4));
-  SVO_TRY(ensure(c.large_jobs, (size_t)kLargeJobs * sizeof(uint2)));
+  // (one allocation: a large one the runtime has to map takes 250 us)
   const uint64_t walk_cap = std::min<uint64_t>(ntri, kLargeWalkMax);
-  SVO_TRY(ensure(c.large_walk, (size_t)walk_cap * kLargeQuads * sizeof(uint4)));
+  const size_t b_tri = ((size_t)ntri * 4 + 255) & ~(size_t)255;
+  const size_t b_jobs = (size_t)kLargeJobs * sizeof(uint2);
+  SVO_TRY(ensure(c.large, 3 * b_tri + b_jobs + (size_t)walk_cap * kLargeQuads * sizeof(uint4)));
   SVO_TRY(ensure(c.occ_list, ntab * 4));
   SVO_TRY(ensure_scan_scratch(c, ntab, 8));
   if (new_table) {
@@ -2299,9 +2297,13 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     A.pool_cap = c.pool_cap;
     return A;
   };
-  const LargeList large{c.large_unit.as<uint32_t>(), c.large_tri.as<uint32_t>(),
-                        c.large_rows.as<uint32_t>(), c.large_jobs.as<uint2>(),
-                        c.large_walk.as<uint4>(),    walk_cap};
+  char* const lb = (char*)c.large.p;
+  const LargeList large{(uint32_t*)lb,
+                        (uint32_t*)(lb + b_tri),
+                        (uint32_t*)(lb + 2 * b_tri),
+                        (uint2*)(lb + 3 * b_tri),
+                        (uint4*)(lb + 3 * b_tri + b_jobs),
+                        walk_cap};
   const uint64_t runs_kind[2] = {(toff_kind[0][nu] + (uint64_t)kTileRun - 1) / kTileRun,
                                  (toff_kind[1][nu] + (uint64_t)kTileRun - 1) / kTileRun};
   const uint64_t runs = runs_kind[0] + runs_kind[1];
@@ -2310,7 +2312,8 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     using Act = decltype(tag);
     const unsigned tile_grid = (unsigned)std::min<uint64_t>(
         runs * kTileRun / kTileWaves,
-        std::max(1, c.tune.tile_blocks * kTileBlocks<Act> / kTileBlocks<TouchAction>));
+        std::max<uint64_t>(
+            1, (uint64_t)std::max(1, c.tune.tile_blocks) * kTileBlocks<Act> / kTileBlocks<TouchAction>));
     ktimer_begin(c, name);
     SVO_LAUNCH((k_vox_tile<Act>), dim3(tile_grid), dim3(kTile), 0, c.stream, d_units, nu,
                        d_toff, payload_runs, args(), queue, large, tt, collect, skip);

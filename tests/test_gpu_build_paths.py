@@ -137,6 +137,19 @@ def test_units_past_32_bits(payload):
             assert ctx.data(info.n_data).tobytes() == want[1].tobytes()
 
 
+@pytest.mark.parametrize("payload", [False, True])
+def test_a_mesh_that_covers_nothing(payload):
+    """No brick is flagged: the scan that reads back has no element, and must still do it; the
+    next mesh of the same context is not affected."""
+    G = 64
+    rng = np.random.default_rng(4)
+    none, some = _mesh(rng, 100, 2.0 / G, payload), _mesh(rng, 100, 2.0 / G, payload)
+    none[:, 3] = 1e12  # a bbox that ends before it starts
+    with SvoContext(0) as ctx:
+        for tris in (none, some, none):
+            _same(ctx, ctx.run(tris, payload, G), tris, payload, G)
+
+
 @pytest.mark.parametrize("n_parts", [8, 64, 512])
 @pytest.mark.parametrize("n", [1, 64, 2047, 2048, 2049, 300001])
 def test_partition_lists(n_parts, n):
