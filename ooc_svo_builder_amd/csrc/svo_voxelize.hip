@@ -550,16 +550,18 @@ __device__ __forceinline__ uint32_t upper_index(const T* __restrict__ a, uint32_
 // device work queues (tile_off[u] = first tile of unit u); tt is smaller for passes with few
 // triangles, so that their tiles still spread over the chip. Lane l sets up triangle l of
 // the tile. A tile whose triangles all have at most direct_cols columns, of about as many
-// each, is walked from registers, a lane a triangle. Triangles with more than small_cols columns (or non-slab triangles with more
-// than small_cols * 8 tests) go to the column-parallel tier. Otherwise a tile is laid out in two
-// steps, each giving every lane of the wave one element whatever the triangles' shapes:
+// each, is walked from registers, a lane a triangle. Triangles with more than small_cols columns
+// (or non-slab triangles with more than small_cols * 8 tests) go to the column-parallel tier.
+// Otherwise a tile is laid out in two steps, each giving every lane of the wave one element
+// whatever the triangles' shapes:
 //   * rows: 64 rows of the tile's triangles at a time; a lane finds its row's interval of
 //     columns, and the terms of its bounds that do not change along it (fast_row);
 //   * columns: the columns of these 64 rows, 64 at a time; a lane finds the run of voxels
 //     its column holds (fast_column) and marks it without testing them one by one.
 // A column whose run is not certain (a bound within its error of an integer: a few in a
 // thousand at 2048; most where faces lie on voxel planes) is queued, and the queue walked
-// with the reference's own tests once 64 are there. Units the pass does not apply to (skip mask) contribute nothing.
+// with the reference's own tests once 64 are there. Units the pass does not apply to (skip mask)
+// contribute nothing.
 //
 // Bound by vector instructions (binary meshes) or by the winner atomics (payload). Testing
 // every candidate voxel of a row segment per lane left 64% of the lanes of a rough mesh's waves
@@ -1431,8 +1433,8 @@ __device__ __forceinline__ uint32_t nth_set_bit(uint64_t w, uint32_t n) {
 // after the other) and one that read them back took 242 + 336 us on 17M voxels of a rough
 // sphere; this one 403 (1.9M voxels of a fine terrain: 34 + 71 us, 81). With kStaged (more than
 // kStagePayload bricks) 64 records go through LDS and out in whole KiB past the caches, not as 16
-// bytes of every 32, and cells are zeroed by the 64-byte pieces that hold marks: 392 -> 300 us,
-// the terrain 72 -> 61, 64 mixed meshes 876 -> 682 (2500 bricks: 17, staged 18.6).
+// bytes of every 32, and cells are zeroed by the 64-byte pieces that hold marks: 392 -> 275 us,
+// the terrain 72 -> 61, 64 mixed meshes 876 -> 680 (2500 bricks: 17, staged 18.6).
 constexpr uint64_t kStagePayload = 4096;
 template <bool kStaged>
 __global__ __launch_bounds__(256) void k_payload_bricks(
