@@ -2196,15 +2196,23 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
   // is running
   const bool new_table = c.table_entries < ntab;
   const bool new_flags = dense && !geometry_only && c.cflags_zeroed < ntab * kBrickWords;
-  // (allocated before the first fill: an allocation while the GPU works waits for it)
-  if (new_table) SVO_TRY(ensure(c.table, ntab * 4));
-  if (new_flags) SVO_TRY(ensure(c.cflags, ntab * kBrickWords));
+  // (allocated before the first fill: an allocation while the GPU works waits for it. What is
+  // replaced counts as zero only once its fill is on the stream: a later allocation may fail)
+  if (new_table) {
+    c.table_entries = 0;
+    SVO_TRY(ensure(c.table, ntab * 4));
+  }
+  if (new_flags) {
+    c.cflags_zeroed = 0;
+    SVO_TRY(ensure(c.cflags, ntab * kBrickWords));
+  }
   uint64_t grid_fill = 0;
   if (dense) {
     if (c.grid_zeroed < dense_bytes) {
       // grown to at least twice its size (at most the dense limit), so that passes of
       // slowly growing spans (a server's batches) reallocate it a few times only
       uint64_t target = dense_bytes;
+      c.grid_zeroed = 0;
       if (c.grid8.cap < dense_bytes) {
         target = std::max<uint64_t>(dense_bytes,
                                     std::min<uint64_t>(c.dense_limit, 2 * (uint64_t)c.grid8.cap));
@@ -2535,8 +2543,8 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     d.nvox = J.nvox;
     d.dbase = J.dbase;
   }
+  c.jobdev_img.clear();  // (before what it tells of may be replaced)
   SVO_TRY(ensure(c.jobdev, jd.size() * sizeof(JobDev)));
-  c.jobdev_img.clear();
   if (batch) {
     SVO_TRY(upload_async(c, c.jobdev.p, jd.data(), jd.size() * sizeof(JobDev)));
     c.jobdev_img = jd;

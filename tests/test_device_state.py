@@ -1,0 +1,143 @@
+"""What the voxelizer keeps on the device between passes, when an allocation fails.
+
+Its brick table, word flags, cells and slots are zero whenever no pass is running, and the
+context remembers how much of each is. A pass that grows them and then fails, or that fails
+with marks in them, must leave that knowledge right for the next one: the server runs the jobs
+of a failed batch one by one on the same context. The library's host side is compiled here
+against a stand-in for the device (tests/native/device_state_check.hip), where every
+allocation of a pass fails in turn and the passes that follow are checked."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from ooc_svo_builder_amd import lib as binding
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "ooc_svo_builder_amd", "csrc")
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+NAMES = ("allocations", "unclean", "outside", "bad_grid", "marks")
+
+
+@pytest.fixture(scope="module")
+def device(tmp_path_factory):
+    tmp = tmp_path_factory.mktemp("state")
+    src = [os.path.join(ROOT, "tests", "native", "device_state_check.hip")] + \
+        [os.path.join(CSRC, f) for f in ("svo_build.hip", "svo_stream.hip", "svo_capi.hip")]
+    runs, objs = [], []
+    for f in src:
+        objs.append(str(tmp / (os.path.basename(f) + ".o")))
+        runs.append(subprocess.Popen([HIPCC, "--offload-host-only", "-O1", "-std=c++17", "-fPIC",
+                                      "-ffp-contract=off", "-fno-fast-math", "-c", f, "-o", objs[-1]]))
+    assert [r.wait() for r in runs] == [0] * len(runs)
+    so = str(tmp / "device_state.so")
+    # (no code for a device is linked in: the registration's references to it are null)
+    names = subprocess.run(["nm", "-u"] + objs, check=True, capture_output=True, text=True).stdout
+    none = ["-Wl,--defsym=%s=0" % w for w in set(names.split()) if w.startswith("__hip_fatbin")]
+    subprocess.run(["g++", "-shared", "-o", so] + objs + ["-Wl,-Bsymbolic", "-lpthread"] + none, check=True)
+    L = C.CDLL(so)
+    for name, (res, args) in binding.SIGNATURES.items():
+        if hasattr(L, name):
+            getattr(L, name).restype, getattr(L, name).argtypes = res, args
+    return L
+
+
+def _arm(L, fail_at=-1, n_occ=5, n_vox=100):
+    L.state_arm(C.c_long(fail_at), C.c_uint64(n_occ), C.c_uint64(n_vox))
+
+
+def _state(L):
+    out = (C.c_uint64 * 5)()
+    L.state_read(out)
+    return dict(zip(NAMES, out))
+
+
+def _mesh(payload, n=40):
+    return np.zeros((n, 21 if payload else 9), np.float32)
+
+
+def _pass(L, ctx, payload, G):
+    t = _mesh(payload)
+    rc = L.svo_mesh_load(ctx, t.ctypes.data_as(C.c_void_p), len(t), int(payload), 0)
+    return rc or L.svo_voxelize(ctx, 0, 0, G ** 3, 1.0 / G, G, 0, None)
+
+
+def _batch(L, ctx, G, kinds):
+    jobs, res, info = (binding.Job * len(kinds))(), (binding.JobResult * len(kinds))(), binding.RunInfo()
+    keep = [binding.fill_job(q, dict(records=_mesh(p), payload=p, gridsize=G))
+            for q, p in zip(jobs, kinds)]
+    rc = L.svo_batch_run(ctx, jobs, len(kinds), res, C.byref(info))
+    del keep
+    return rc
+
+
+def _find(L, n_occ):
+    L.state_found(C.c_uint64(n_occ), C.c_uint64(20 * n_occ))
+
+
+def _fail_each(L, first, grown, after, marked, dense_mb=None):
+    """Passes 'first' on a new context, then 'grown' with its k-th allocation failing, then the
+    passes 'after', for every k up to the allocations it makes. marked: the failures after its
+    marks, else those before them."""
+    failed = 0
+    for k in range(100):
+        ctx = C.c_void_p()
+        L.state_clear()
+        _arm(L)
+        assert L.svo_ctx_create(0, C.byref(ctx)) == 0
+        assert L.svo_ctx_set_graphs(ctx, 0) == 0
+        if dense_mb is not None:
+            assert L.svo_ctx_set_tuning(ctx, 0, dense_mb) == 0
+        for f in first:
+            assert f(ctx) == 0, k
+        _arm(L, fail_at=k)
+        marks = _state(L)["marks"]
+        rc = grown(ctx)
+        s = _state(L)
+        if s["allocations"] <= k:  # it made fewer
+            assert rc == 0 and failed >= 1
+            L.svo_ctx_destroy(ctx)
+            return
+        assert rc in (binding.SVO_ERR_NOMEM, binding.SVO_ERR_DEVICE), (k, rc)
+        if marked == (s["marks"] > marks):
+            failed += 1
+            _arm(L)
+            for f in after:
+                assert f(ctx) == 0, k
+            s = _state(L)
+            assert (s["unclean"], s["outside"], s["bad_grid"]) == (0, 0, 0), (k, s)
+        L.svo_ctx_destroy(ctx)
+    raise AssertionError("the pass still allocates after 100 allocations")
+
+
+def _passes(L, kinds, dense, marked):
+    a, b = kinds
+    _fail_each(L, [lambda c: _pass(L, c, a, 32)], lambda c: (_find(L, 400), _pass(L, c, b, 128))[1],
+               [lambda c: _pass(L, c, a, 32), lambda c: _pass(L, c, b, 32), lambda c: _pass(L, c, b, 64),
+                lambda c: _pass(L, c, a, 64), lambda c: _pass(L, c, b, 128)],
+               marked, None if dense else 0)
+
+
+def _batches(L, marked):
+    kinds = (False, True, False)
+    _fail_each(L, [lambda c: _batch(L, c, 32, kinds)], lambda c: (_find(L, 400), _batch(L, c, 128, kinds))[1],
+               [lambda c: _batch(L, c, 32, kinds), lambda c: _batch(L, c, 128, (False,)),
+                lambda c: _batch(L, c, 128, (True,)), lambda c: _batch(L, c, 128, kinds)], marked)
+
+
+KINDS = [(False, False), (True, True), (False, True), (True, False)]
+
+
+@pytest.mark.parametrize("dense", [True, False])
+@pytest.mark.parametrize("kinds", KINDS)
+def test_a_pass_that_fails_as_it_grows(device, kinds, dense):
+    """A pass, a larger one that fails before its marks, the first again, one in between and the
+    larger again: nothing that was replaced is taken for zero."""
+    _passes(device, kinds, dense, marked=False)
+
+
+def test_a_batch_that_fails_as_it_grows(device):
+    """The server's order: the batch fails, then its jobs run one by one on the same context."""
+    _batches(device, marked=False)
