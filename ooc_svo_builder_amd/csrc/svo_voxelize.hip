@@ -2110,6 +2110,16 @@ static void fill_params(const VoxUnit& h, const Context& c, VoxParams& P) {
   P.grid8 = nullptr;
 }
 
+// What a pass marks is cleared by its later kernels. One that returns before they are all on the
+// stream leaves marks behind: the next pass is to zero everything again.
+struct MarksLeft {
+  Context& c;
+  bool cleared = false;
+  ~MarksLeft() {
+    if (!cleared) c.table_entries = c.cflags_zeroed = c.grid_zeroed = c.pool_cap = 0;
+  }
+};
+
 hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch,
                           uint64_t* nfilled) {
   *nfilled = 0;
@@ -2193,7 +2203,7 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     small_units = small_units && (ubase[u + 1] - ubase[u]) <= (1ull << (32 - kBrickBits));
   }
   // the table, the word flags, the dense grid and the byte pool are all-zero whenever no pass
-  // is running
+  // is running, as far as the context's counts of them go
   const bool new_table = c.table_entries < ntab;
   const bool new_flags = dense && !geometry_only && c.cflags_zeroed < ntab * kBrickWords;
   // (allocated before the first fill: an allocation while the GPU works waits for it. What is
@@ -2357,6 +2367,7 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
   };
 
   // ---- phase A: mark, compact counts; one synchronization at its end
+  MarksLeft marks{c};
   std::vector<uint64_t> uvoff(nu + 1);
   for (int attempt = 0;; attempt++) {
     const uint64_t bc_bound = dense ? ntab : std::min<uint64_t>(ntab, c.pool_cap);
@@ -2674,6 +2685,7 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     for (uint32_t u = 0; u < nu; u++) any_binary |= units[u].stride == 9;
     if (!codes_now || any_binary) c.codes_lazy = true;
   }
+  marks.cleared = true;
   c.n_vox = s0 + nvox;
   *nfilled = nvox;
   return hipSuccess;

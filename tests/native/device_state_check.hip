@@ -214,6 +214,9 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, si
       memcpy(st.host, st.ctr, kNumCounters * 8);
       *st.flag = (uint32_t)st.seq;
     }
+  } else if (is("k_unit_voxels")) {  // the voxels dealt evenly to the units
+    const uint32_t n = arg<uint32_t>(args, 4);
+    for (uint32_t u = 0; u <= n; u++) arg<uint64_t*>(args, 6)[u] = d.n_vox * u / n;
   } else if (is("k_payload_bricks")) {
     each(g_pass.units, g_pass.n, nullptr, nullptr, kCells, 0);
   } else if (is("k_brick_clear")) {

@@ -141,3 +141,22 @@ def test_a_pass_that_fails_as_it_grows(device, kinds, dense):
 def test_a_batch_that_fails_as_it_grows(device):
     """The server's order: the batch fails, then its jobs run one by one on the same context."""
     _batches(device, marked=False)
+
+
+@pytest.mark.parametrize("kinds,dense", [(k, d) for k in KINDS for d in (True, False) if k[1] or not d])
+def test_a_pass_that_fails_with_marks(device, kinds, dense):
+    """The same with failures after the marks (the records' array above all; a dense geometry-only
+    pass allocates nothing then): what they left is cleared before the next marks."""
+    _passes(device, kinds, dense, marked=True)
+
+
+def test_a_batch_that_fails_with_marks(device):
+    _batches(device, marked=True)
+
+
+def test_slots_that_fail_to_grow(device):
+    """A pass on touched bricks that needs more slots than there are (1500 of 1024)."""
+    L = device
+    _fail_each(L, [lambda c: _pass(L, c, False, 256)],
+               lambda c: (_find(L, 1500), _pass(L, c, False, 256))[1],
+               [lambda c: _pass(L, c, False, 64), lambda c: _pass(L, c, True, 256)], True, 0)
