@@ -1528,18 +1528,18 @@ __global__ __launch_bounds__(256) void k_payload_bricks(
 // Voxel i of the pass (stream index s0 + i) belongs to the unit whose voxel range holds
 // it, and to that unit's job; its record goes to dbase[job] + 1 + (s0 + i - voff[job]).
 // Voxels of geometry-only jobs have no record here.
-// Threads cover the payload units' voxels only: payload voxel k lies in the payload unit
-// j with prange[j] <= k < prange[j + 1] (a block searches for its first voxel, a thread
+// Threads cover the payload units' voxels only, from payload voxel 'first' on: payload voxel k
+// lies in the payload unit j with prange[j] <= k < prange[j + 1] (a block searches for its first voxel, a thread
 // steps forward over the rare unit boundaries), unit punit[j], whose voxels start at pass
 // voxel pstart[j].
 __global__ __launch_bounds__(256) void k_payload_records(
     const JobDev* __restrict__ jobs, const VoxParams* __restrict__ units,
     const uint64_t* __restrict__ prange, const uint64_t* __restrict__ pstart,
     const uint32_t* __restrict__ punit, uint32_t n_pu, const uint64_t* __restrict__ codes,
-    uint64_t s0, const uint32_t* __restrict__ winner, uint64_t n_pv, float* __restrict__ out,
-    ull* ctr) {
+    uint64_t s0, const uint32_t* __restrict__ winner, uint64_t first, uint64_t n_pv,
+    float* __restrict__ out, ull* ctr) {
   __shared__ uint32_t s_j0;
-  const uint64_t b0 = (uint64_t)blockIdx.x * blockDim.x;
+  const uint64_t b0 = first + (uint64_t)blockIdx.x * blockDim.x;
   const uint64_t k = b0 + threadIdx.x;
   if (threadIdx.x == 0) s_j0 = upper_index<uint64_t>(prange, n_pu + 1, b0);
   __syncthreads();
@@ -1935,12 +1935,14 @@ __global__ __launch_bounds__(256) void k_copy(u32x4_u* __restrict__ dst,
 }
 // blocks up to which the copy raises the flag itself: 2 MB in four elements a thread
 constexpr unsigned kCopyFlagBlocks = 128;
+// (HIP takes less than 2^32 threads in a launch; the blocks stride)
+constexpr uint64_t kCopyMaxBlocks = (1u << 24) - 1;
 hipError_t copy_records(Context& c, void* dst, const void* src, size_t bytes) {
   const uint64_t n = bytes / 16;
   const int tail = bytes % 16 != 0;
   if (n > kCopyFlagBlocks * 1024ull) {
-    SVO_LAUNCH(k_copy<1>, dim3((unsigned)std::min<uint64_t>((n + 255) / 256, 1u << 24)), dim3(256),
-               0, c.stream, (u32x4_u*)dst, (const u32x4_u*)src, n, tail,
+    SVO_LAUNCH(k_copy<1>, dim3((unsigned)std::min<uint64_t>((n + 255) / 256, kCopyMaxBlocks)),
+               dim3(256), 0, c.stream, (u32x4_u*)dst, (const u32x4_u*)src, n, tail,
                (volatile uint32_t*)nullptr, 0u, (ull*)nullptr);
     SVO_TRY(hipGetLastError());
     return read_back(c, nullptr, 0);
@@ -2661,10 +2663,13 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
         }
         if (n_pv) {
           ktimer_begin(c, "payload_records");
-          SVO_LAUNCH(k_payload_records, dim3((unsigned)((n_pv + 255) / 256)), dim3(256), 0,
-                     c.stream, c.jobdev.as<JobDev>(), (const VoxParams*)d_units, d_prange,
-                     d_pstart, d_punit, n_pu, c.codes.as<uint64_t>(), s0,
-                     c.winner.as<uint32_t>(), n_pv, c.records.as<float>(), ctr);
+          const uint64_t part = 1ull << 31;  // (a launch takes less than 2^32 threads)
+          for (uint64_t first = 0; first < n_pv; first += part)
+            SVO_LAUNCH(k_payload_records,
+                       dim3((unsigned)((std::min(n_pv - first, part) + 255) / 256)), dim3(256), 0,
+                       c.stream, c.jobdev.as<JobDev>(), (const VoxParams*)d_units, d_prange,
+                       d_pstart, d_punit, n_pu, c.codes.as<uint64_t>(), s0,
+                       c.winner.as<uint32_t>(), first, n_pv, c.records.as<float>(), ctr);
           ktimer_end(c);
           SVO_TRY(hipGetLastError());
         }

@@ -5,6 +5,8 @@
 // every launch, that the grid is one HIP accepts.
 #include "../../ooc_svo_builder_amd/csrc/svo_voxelize.hip"
 
+#include <sys/mman.h>
+
 #include <cstdlib>
 #include <map>
 #include <string>
@@ -14,6 +16,7 @@
 using namespace svo;
 
 namespace {
+constexpr size_t kHuge = 256u << 20;  // allocations above are address space, neither filled nor read
 struct Device {
   std::map<uintptr_t, size_t> mem;           // live allocations
   std::map<const void*, std::string> names;  // kernels
@@ -37,14 +40,22 @@ hipError_t allocate(void** p, size_t bytes) {
   Device& d = dev();
   *p = nullptr;
   if (d.allocs++ == d.fail_at) return d.last = hipErrorOutOfMemory;
-  *p = malloc(bytes);
-  memset(*p, 0xA5, bytes);
+  if (bytes > kHuge) {
+    *p = mmap(nullptr, bytes, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+  } else {
+    *p = malloc(bytes);
+    memset(*p, 0xA5, bytes);
+  }
   d.mem[(uintptr_t)*p] = bytes;
   return hipSuccess;
 }
 hipError_t give_back(void* p) {
+  const size_t bytes = dev().mem[(uintptr_t)p];
   dev().mem.erase((uintptr_t)p);
-  free(p);
+  if (bytes > kHuge)
+    munmap(p, bytes);
+  else
+    free(p);
   return hipSuccess;
 }
 void must_be_zero(const void* p, size_t bytes) {
@@ -174,12 +185,12 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, si
     uint32_t* p = arg<uint32_t*>(args, 0);
     const uint64_t n = arg<uint64_t>(args, 2);
     if (!inside(p, n * 4)) d.outside++;
-    else std::fill(p, p + n, arg<uint32_t>(args, 1));
+    else if (n * 4 <= kHuge) std::fill(p, p + n, arg<uint32_t>(args, 1));
   } else if (is("k_fill_u64")) {
     uint64_t* p = arg<uint64_t*>(args, 0);
     const uint64_t n = arg<uint64_t>(args, 2);
     if (!inside(p, n * 8)) d.outside++;
-    else std::fill(p, p + n, arg<uint64_t>(args, 1));
+    else if (n * 8 <= kHuge) std::fill(p, p + n, arg<uint64_t>(args, 1));
   } else if (is("k_gather_host")) {
     const GatherArgs g = arg<GatherArgs>(args, 0);
     for (int k = 0; k < g.n; k++) memcpy(g.dst[k], g.src[k], g.words[k] * 8);
@@ -248,6 +259,13 @@ void state_read(uint64_t out[5]) {
   out[2] = d.outside;
   out[3] = d.bad_grid;
   out[4] = d.marks;
+}
+// A device-to-device copy of records.
+int state_copy(uint64_t bytes) {
+  Context c;
+  const hipError_t e = copy_records(c, (void*)64, (const void*)128, bytes);
+  if (c.hread) (void)hipHostFree(c.hread);
+  return (int)e;
 }
 void state_clear() {
   Device& d = dev();

@@ -160,3 +160,27 @@ def test_slots_that_fail_to_grow(device):
     _fail_each(L, [lambda c: _pass(L, c, False, 256)],
                lambda c: (_find(L, 1500), _pass(L, c, False, 256))[1],
                [lambda c: _pass(L, c, False, 64), lambda c: _pass(L, c, True, 256)], True, 0)
+
+
+@pytest.mark.parametrize("gib", [1, 63, 64, 65, 128, 200])
+def test_copies_of_any_size(device, gib):
+    """A record copy's grid is one that HIP takes (less than 2^32 threads)."""
+    L = device
+    for bytes_ in ((gib << 30) - 24, gib << 30, (gib << 30) + 24):
+        L.state_clear()
+        assert L.state_copy(C.c_uint64(bytes_)) == 0
+        assert _state(L)["bad_grid"] == 0
+
+
+@pytest.mark.parametrize("n_vox", [1 << 31, (1 << 31) + 1, 0xFFFFFF00, 0xFFFFFF01, 0xFFFFFFF0])
+def test_payload_records_of_almost_two_to_the_32_voxels(device, n_vox):
+    """The records of a pass on touched bricks, up to the largest one that is accepted."""
+    L, ctx = device, C.c_void_p()
+    L.state_clear()
+    _arm(L)
+    assert L.svo_ctx_create(0, C.byref(ctx)) == 0
+    assert L.svo_ctx_set_tuning(ctx, 0, 0) == 0
+    L.state_found(C.c_uint64(500), C.c_uint64(n_vox))
+    assert _pass(L, ctx, True, 256) == 0
+    assert _state(L)["bad_grid"] == 0
+    L.svo_ctx_destroy(ctx)
