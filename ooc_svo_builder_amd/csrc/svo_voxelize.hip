@@ -751,19 +751,41 @@ struct LargeList {
   uint4* walk;
   uint64_t walk_cap;
 };
-// Rows per job of a triangle with nu x nv columns, its further jobs appended; with no room
-// for them (kAllRows) its one job takes all rows, that many at a time.
+// Rows per job of a triangle with nu x nv columns, and places for its further jobs: n of them
+// from 'at' on, to be filled with idx and the rows. With no room for all (kAllRows) its one job
+// takes all rows, that many at a time, and the places left are filled with none.
 constexpr uint32_t kAllRows = 1u << 31;
-__device__ __forceinline__ uint32_t large_jobs(const LargeList& B, ull* ctr, uint32_t idx,
-                                               uint32_t nu, uint32_t nv) {
+struct JobPlaces {
+  uint32_t idx, rows, at, n;
+};
+__device__ __forceinline__ uint32_t large_jobs(ull* ctr, uint32_t idx, uint32_t nu, uint32_t nv,
+                                               JobPlaces& J) {
   const uint32_t rows = max(1u, min((uint32_t)kWave, kJobCols / nu));
   const uint32_t more = (nv + rows - 1) / rows - 1;
   if (!more) return rows;
   const ull at = atomicAdd(&ctr[kCtrLargeJobs], (ull)more);
   const bool fits = at + more <= kLargeJobs;
-  for (uint32_t q = 0; q < more && at + q < kLargeJobs; q++)
-    B.jobs[at + q] = make_uint2(fits ? idx : 0xFFFFFFFFu, (q + 1) * rows);
+  J.idx = fits ? idx : 0xFFFFFFFFu;
+  J.rows = rows;
+  J.at = (uint32_t)min(at, (ull)kLargeJobs);
+  J.n = min(more, kLargeJobs - J.at);
   return fits ? rows : rows | kAllRows;
+}
+// Fill the lanes' places (whole waves): a few by their lane, many by the wave, one lane's at a
+// time. Hundreds written by a lane one after the other held up its wave, the last of the launch: a
+// rotated cube's 12 triangles at 1024 225 us in all, 167 so; at 4096 in 8 partitions 2465 and 1603.
+constexpr uint32_t kOwnPlaces = 8;
+__device__ __forceinline__ void put_jobs(uint2* jobs, const JobPlaces& J) {
+  if (J.n <= kOwnPlaces)
+    for (uint32_t q = 0; q < J.n; q++) jobs[J.at + q] = make_uint2(J.idx, (q + 1) * J.rows);
+  for (uint64_t m = __ballot(J.n > kOwnPlaces); m; m &= m - 1ull) {
+    const int src = __ffsll((long long)m) - 1;
+    const uint32_t idx = (uint32_t)__builtin_amdgcn_readlane((int)J.idx, src);
+    const uint32_t rows = (uint32_t)__builtin_amdgcn_readlane((int)J.rows, src);
+    const uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)J.at, src);
+    const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)J.n, src);
+    for (uint32_t q = lane_id(); q < n; q += kWave) jobs[at + q] = make_uint2(idx, (q + 1) * rows);
+  }
 }
 
 // blocks of the small tier on a CU (what an action keeps in LDS leaves room for three)
@@ -868,6 +890,7 @@ __global__ __launch_bounds__(kTile, kTileBlocks<Act>) void k_vox_tile(const VoxP
     most = (uint32_t)__builtin_amdgcn_readlane((int)most, kWave - 1);
     const bool direct = most <= (uint32_t)P.direct_cols && most * 100u <= 1200u + all * 4u;
     uint32_t rows = 0;
+    JobPlaces places{0, 0, 0, 0};
     if ((large && collect) || (ncols && !direct)) {
       FastTri F;
       make_fast(K, P, F);
@@ -880,7 +903,7 @@ __global__ __launch_bounds__(kTile, kTileBlocks<Act>) void k_vox_tile(const VoxP
         const ull idx = atomicAdd(&ctr[kCtrLargeCount], 1ull);
         B.unit[idx] = u;
         B.tri[idx] = (uint32_t)K.i[I_TRI];
-        B.rows[idx] = large_jobs(B, ctr, (uint32_t)idx, nu, nv);
+        B.rows[idx] = large_jobs(ctr, (uint32_t)idx, nu, nv, places);
         if (idx < B.walk_cap) {
           uint4* dst = B.walk + idx * kLargeQuads;
 #pragma unroll
@@ -891,6 +914,7 @@ __global__ __launch_bounds__(kTile, kTileBlocks<Act>) void k_vox_tile(const VoxP
         }
       }
     }
+    if (collect) put_jobs(B.jobs, places);
     if (direct) {
       if (kOverlay && !clean) {
         for (uint32_t k = lane; k < sizeof(*overlay) / 4; k += kWave) ((uint32_t*)overlay)[k] = 0u;
