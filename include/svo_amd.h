@@ -62,6 +62,11 @@ void* svo_ctx_stream(svo_ctx* ctx);
  * touched bricks only (UINT64_MAX keeps the current value; the default is half of the
  * free HBM at context creation, at most 128 GiB). Neither changes the output. */
 int svo_ctx_set_tuning(svo_ctx* ctx, int small_cols, uint64_t dense_limit_mb);
+/* Room of the column-parallel tier's lists (no reference counterpart): triangles whose set-up is
+ * stored (288 B each; 65536), and jobs of some rows past a triangle's first one (8 B each;
+ * 1048576). What finds no room is set up again by each job, or found by the waves themselves;
+ * neither changes the output. */
+int svo_ctx_set_large_tier(svo_ctx* ctx, uint32_t walks, uint32_t jobs);
 
 /* hipGraph use of svo_batch_run on this context (no reference counterpart; on by
  * default): each kernel sequence between two host synchronizations of a batch runs as a

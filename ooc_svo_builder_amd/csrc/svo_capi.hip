@@ -363,6 +363,13 @@ int svo_ctx_set_tuning(svo_ctx* ctx, int small_cols, uint64_t dense_limit_mb) {
   return SVO_OK;
 }
 
+int svo_ctx_set_large_tier(svo_ctx* ctx, uint32_t walks, uint32_t jobs) {
+  CHECK_CTX();
+  ctx->c.tune.large_walks = walks;
+  ctx->c.tune.large_jobs = jobs;
+  return SVO_OK;
+}
+
 int svo_ctx_set_graphs(svo_ctx* ctx, int on) {
   CHECK_CTX();
   ctx->c.graph_policy = on ? 1 : 0;

@@ -135,6 +135,9 @@ struct VoxTuning {
   int direct_cols = 16;     // columns up to which a triangle's own thread walks them
   int tile_blocks = 1024;   // persistent grid of the small tier
   int large_blocks = 1024;  // grid of the large tier (grid-stride)
+  // room of the large tier's lists
+  uint32_t large_walks = 1u << 16;  // triangles with stored constants (19 MB)
+  uint32_t large_jobs = 1u << 20;   // jobs past the triangles' first ones (8 MB)
 };
 
 struct StageTimes {

@@ -581,7 +581,6 @@ constexpr uint32_t kQueues = 8;        // tile queues per persistent launch
 constexpr uint32_t kTileRun = 16;      // neighbouring tiles in one queue
 constexpr uint32_t kQueueStride = 16;  // words between their counters (own cache lines)
 constexpr uint32_t kQueueWords = kQueues * kQueueStride;
-constexpr uint64_t kLargeWalkMax = 1u << 16;  // large triangles with stored constants (19 MB)
 constexpr int kSkipBinary = 1;  // geometry-only units (payload winner pass)
 
 __device__ __forceinline__ bool skipped(const VoxParams& P, int skip) {
@@ -737,10 +736,9 @@ __device__ __forceinline__ void walk_rows(WalkLds& L, typename Act::Cache* cache
 }
 
 // The triangles of the large tier: unit, triangle, rows per job, the linear form and walk of
-// the first walk_cap of them (the others are set up again by each of their jobs), and the jobs
-// after each triangle's first one (triangle's index here, first row).
-constexpr uint32_t kLargeJobs = 1u << 20;  // places for those
-constexpr uint32_t kJobCols = 1024;        // columns of a job, roughly
+// the first walk_cap of them (the others are set up again by each of their jobs), and up to job_cap
+// jobs after each triangle's first one (triangle's index here, first row).
+constexpr uint32_t kJobCols = 1024;  // columns of a job, roughly
 constexpr int kLargeQuads = kTriQuads + kWalkWords / 4;
 static_assert(kWalkWords % 4 == 0 && sizeof(Walk) == kWalkWords * 4, "walk words");
 struct LargeList {
@@ -749,27 +747,29 @@ struct LargeList {
   uint32_t* rows;
   uint2* jobs;
   uint4* walk;
-  uint64_t walk_cap;
+  uint32_t job_cap, walk_cap;
 };
 // Rows per job of a triangle with nu x nv columns, and places for its further jobs: n of them
-// from 'at' on, to be filled with idx and the rows. With no room for all (kAllRows) its one job
-// takes all rows, that many at a time, and the places left are filled with none.
-constexpr uint32_t kAllRows = 1u << 31;
+// from 'at' on, to be filled with idx and the rows. With no room for all, the places left are
+// filled with none, and the number of its jobs stands above the rows (unlisted: below 2^15, as a
+// unit's side): kShareJobs or more are dealt to all waves, fewer are done with its first one.
+constexpr int kUnlistedShift = 8;
+constexpr uint32_t kShareJobs = 8;
 struct JobPlaces {
   uint32_t idx, rows, at, n;
 };
-__device__ __forceinline__ uint32_t large_jobs(ull* ctr, uint32_t idx, uint32_t nu, uint32_t nv,
-                                               JobPlaces& J) {
+__device__ __forceinline__ uint32_t large_jobs(const LargeList& B, ull* ctr, uint32_t idx,
+                                               uint32_t nu, uint32_t nv, JobPlaces& J) {
   const uint32_t rows = max(1u, min((uint32_t)kWave, kJobCols / nu));
   const uint32_t more = (nv + rows - 1) / rows - 1;
   if (!more) return rows;
   const ull at = atomicAdd(&ctr[kCtrLargeJobs], (ull)more);
-  const bool fits = at + more <= kLargeJobs;
+  const bool fits = at + more <= B.job_cap;
   J.idx = fits ? idx : 0xFFFFFFFFu;
   J.rows = rows;
-  J.at = (uint32_t)min(at, (ull)kLargeJobs);
-  J.n = min(more, kLargeJobs - J.at);
-  return fits ? rows : rows | kAllRows;
+  J.at = (uint32_t)min(at, (ull)B.job_cap);
+  J.n = min(more, B.job_cap - J.at);
+  return fits ? rows : rows | (more << kUnlistedShift);
 }
 // Fill the lanes' places (whole waves): a few by their lane, many by the wave, one lane's at a
 // time. Hundreds written by a lane one after the other held up its wave, the last of the launch: a
@@ -903,7 +903,7 @@ __global__ __launch_bounds__(kTile, kTileBlocks<Act>) void k_vox_tile(const VoxP
         const ull idx = atomicAdd(&ctr[kCtrLargeCount], 1ull);
         B.unit[idx] = u;
         B.tri[idx] = (uint32_t)K.i[I_TRI];
-        B.rows[idx] = large_jobs(ctr, (uint32_t)idx, nu, nv, places);
+        B.rows[idx] = large_jobs(B, ctr, (uint32_t)idx, nu, nv, places);
         if (idx < B.walk_cap) {
           uint4* dst = B.walk + idx * kLargeQuads;
 #pragma unroll
@@ -942,27 +942,59 @@ __global__ __launch_bounds__(kTile, kTileBlocks<Act>) void k_vox_tile(const VoxP
 // live on the device, the grid strides. Triangle idx has its first job at idx, its others at
 // n_large + (their place in B.jobs). (A thread per bbox column took 219 us on 20,480 triangles
 // of ~2,200 columns, after a launch that scanned the column counts; in rows 160.)
+// Once there are more jobs than places, every wave looks through the triangles, 64 at a time, for
+// unlisted jobs of its own: job q of triangle idx is wave (idx * jobs + q) mod waves's, which deals
+// out triangles of like size evenly. With all rows of such a triangle in one wave, 700 that span
+// most of a grid of 4096 took 131 ms (39 with a thread per column), 29 so; 1500 at 2048 38 ms, 17
+// and 14.
 template <typename Act>
 __global__ __launch_bounds__(kTile, 3) void k_vox_large(const VoxParams* __restrict__ units,
                                                         ActArgs A, LargeList B, int skip) {
   __shared__ WalkLds s_walk[kTileWaves];
   const ull* ctr = A.ctr;
-  const uint64_t n_large = ctr[kCtrLargeCount];
-  const uint64_t total = n_large + min(ctr[kCtrLargeJobs], (ull)kLargeJobs);
-  if ((uint64_t)blockIdx.x * kTileWaves >= total) return;  // uniform per block
+  const uint64_t n_large = ctr[kCtrLargeCount], n_jobs = ctr[kCtrLargeJobs];
+  const uint64_t total = n_large + min(n_jobs, (uint64_t)B.job_cap);
+  const bool unlisted = n_jobs > B.job_cap;
+  if ((uint64_t)blockIdx.x * kTileWaves >= total && !unlisted) return;  // uniform per block
   fill_spread_table();
   __syncthreads();
   WalkLds& L = s_walk[threadIdx.x / kWave];
   const int lane = lane_id();
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(
       (int)(blockIdx.x * kTileWaves + threadIdx.x / kWave));
-  for (uint64_t g = wave; g < total; g += (uint64_t)gridDim.x * kTileWaves) {
-    uint32_t idx = (uint32_t)g, row0 = 0;
-    if (g >= n_large) {
-      const uint2 e = B.jobs[g - n_large];
-      idx = e.x;
-      row0 = e.y;
+  const uint32_t waves = gridDim.x * kTileWaves;
+  uint64_t g = wave, t0 = unlisted ? 0 : n_large;
+  uint32_t q = 0, more = 0;  // of the lane's triangle, t0 - 64 + lane: this wave's next job, all
+  uint64_t mine = 0;         // lanes whose triangle has a job for this wave
+  for (;;) {
+    uint32_t idx, row0 = 0;
+    if (g < total) {
+      idx = (uint32_t)g;
+      if (g >= n_large) {
+        const uint2 e = B.jobs[g - n_large];
+        idx = e.x;
+        row0 = e.y;
+      }
+      g += waves;
       if (idx == 0xFFFFFFFFu) continue;  // a place left empty
+    } else {
+      while (!mine && t0 < n_large) {
+        more = t0 + lane < n_large ? B.rows[t0 + lane] >> kUnlistedShift : 0u;
+        const uint32_t first = (uint32_t)((t0 + lane) * more % waves);
+        q = wave >= first ? wave - first : wave + waves - first;
+        mine = __ballot(more >= kShareJobs && q < more);
+        t0 += kWave;
+      }
+      if (!mine) break;
+      const int src = __ffsll((long long)mine) - 1;
+      idx = (uint32_t)(t0 - kWave) + (uint32_t)src;
+      const uint32_t job = (uint32_t)__builtin_amdgcn_readlane((int)q, src);
+      row0 = (job + 1u) * (B.rows[idx] & ((1u << kUnlistedShift) - 1u));
+      if (job + waves < (uint32_t)__builtin_amdgcn_readlane((int)more, src)) {
+        if (lane == src) q += waves;
+      } else {
+        mine &= mine - 1ull;
+      }
     }
     const VoxParams P = units[B.unit[idx]];
     if (skipped(P, skip)) continue;
@@ -987,11 +1019,11 @@ __global__ __launch_bounds__(kTile, 3) void k_vox_large(const VoxParams* __restr
     }
     wave_lds_sync();
     const uint32_t nb = (uint32_t)(K.i[I_G1V] - K.i[I_G0V] + 1);
-    const uint32_t rows = B.rows[idx] & ~kAllRows;
-    do {
-      walk_rows<Act>(L, nullptr, P, A, K, nb, lane == 0 ? min(rows, nb - row0) : 0u, row0);
-      row0 += rows;
-    } while ((B.rows[idx] & kAllRows) && row0 < nb);
+    const uint32_t rj = B.rows[idx], rows = rj & ((1u << kUnlistedShift) - 1u);
+    const uint32_t rest = rj >> kUnlistedShift;  // (of a triangle with few of them: all its rows here)
+    const uint32_t end = rest && rest < kShareJobs ? nb : min(row0 + rows, nb);
+    for (; row0 < end; row0 += rows)
+      walk_rows<Act>(L, nullptr, P, A, K, nb, lane == 0 ? min(rows, end - row0) : 0u, row0);
   }
 }
 
@@ -2307,9 +2339,9 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
   }
   ull* pool_words = dense ? c.bwords.as<ull>() + nb0 * kBrickWords : c.pool.as<ull>();
   // (one allocation: a large one the runtime has to map takes 250 us)
-  const uint64_t walk_cap = std::min<uint64_t>(ntri, kLargeWalkMax);
+  const uint32_t walk_cap = (uint32_t)std::min<uint64_t>(ntri, c.tune.large_walks);
   const size_t b_tri = ((size_t)ntri * 4 + 255) & ~(size_t)255;
-  const size_t b_jobs = (size_t)kLargeJobs * sizeof(uint2);
+  const size_t b_jobs = ((size_t)c.tune.large_jobs * sizeof(uint2) + 255) & ~(size_t)255;
   SVO_TRY(ensure(c.large, 3 * b_tri + b_jobs + (size_t)walk_cap * kLargeQuads * sizeof(uint4)));
   SVO_TRY(ensure(c.occ_list, ntab * 4));
   SVO_TRY(ensure_scan_scratch(c, ntab, 8));
@@ -2349,6 +2381,7 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
                         (uint32_t*)(lb + 2 * b_tri),
                         (uint2*)(lb + 3 * b_tri),
                         (uint4*)(lb + 3 * b_tri + b_jobs),
+                        c.tune.large_jobs,
                         walk_cap};
   const uint64_t runs_kind[2] = {(toff_kind[0][nu] + (uint64_t)kTileRun - 1) / kTileRun,
                                  (toff_kind[1][nu] + (uint64_t)kTileRun - 1) / kTileRun};

@@ -83,6 +83,7 @@ SIGNATURES = {
     "svo_ctx_set_stream": (_i32, [_vp, _vp]),
     "svo_ctx_stream": (_vp, [_vp]),
     "svo_ctx_set_tuning": (_i32, [_vp, _i32, _u64]),
+    "svo_ctx_set_large_tier": (_i32, [_vp, C.c_uint32, C.c_uint32]),
     "svo_ctx_set_graphs": (_i32, [_vp, _i32]),
     "svo_estimate_partitions": (_u64, [_u64, _u64]),
     "svo_mesh_load": (_i32, [_vp, _vp, _u64, _i32, _i32]),
@@ -324,6 +325,10 @@ class SvoContext:
         """Voxelizer split threshold and dense-grid limit (output is unchanged)."""
         lim = 0xFFFFFFFFFFFFFFFF if dense_limit_mb is None else int(dense_limit_mb)
         _check(load_library().svo_ctx_set_tuning(self._h, int(small_cols), lim))
+
+    def set_large_tier(self, walks: int = 1 << 16, jobs: int = 1 << 20):
+        """Room of the column-parallel tier's lists (output is unchanged)."""
+        _check(load_library().svo_ctx_set_large_tier(self._h, walks, jobs))
 
     def set_graphs(self, on: bool):
         """hipGraph capture and replay of batch_run's kernel sequences (on by default)."""

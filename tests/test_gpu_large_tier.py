@@ -1,4 +1,5 @@
-"""The column-parallel tier's jobs against the oracle."""
+"""The column-parallel tier's lists at and past their ends, against the oracle: set-ups that are
+not stored, jobs that find no place and are dealt to all waves, triangles left to one wave."""
 import numpy as np
 import pytest
 
@@ -33,3 +34,31 @@ def test_triangles_of_few_and_many_jobs(payload, small_cols):
             assert (info.n_partitions, info.nfilled) == (parts, nf)
             assert ctx.nodes(info.n_nodes).tobytes() == nodes.tobytes()
             assert ctx.data(info.n_data).tobytes() == data.tobytes()
+
+
+@pytest.fixture(scope="module")
+def want():
+    G = 256
+    return {p: (oracle.pipeline(_mesh(p), p, G, 2048), oracle.pipeline(_mesh(p), p, G, 2)) for p in (False, True)}
+
+
+@pytest.mark.parametrize("room", [(1 << 16, 1 << 20), (0, 0), (3, 0), (1 << 16, 0), (1 << 16, 1), (5, 100),
+                                  (0, 300), (20, 400)])
+@pytest.mark.parametrize("dense", [True, False])
+@pytest.mark.parametrize("payload", [False, True])
+def test_lists_past_their_room(payload, dense, room, want):
+    """small_cols 64 and 1: the larger kinds of triangles in jobs, and all of them; one partition
+    and eight. What the lists have no room for gives the same bytes."""
+    G, tris = 256, _mesh(payload)
+    with SvoContext(0) as ctx:
+        ctx.set_tuning(dense_limit_mb=None if dense else 0)
+        ctx.set_large_tier(*room)
+        k = ctx.get_tuning()
+        for small_cols in (64, 1):
+            for blocks in (k[3], 2):
+                ctx.set_knobs(small_cols, 0, k[2], blocks)
+                for (nodes, data, _, parts, nf), limit in zip(want[payload], (2048, 2)):
+                    info = ctx.run(tris, payload, G, limit)
+                    assert (info.n_partitions, info.nfilled) == (parts, nf)
+                    assert ctx.nodes(info.n_nodes).tobytes() == nodes.tobytes()
+                    assert ctx.data(info.n_data).tobytes() == data.tobytes()
