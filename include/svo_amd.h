@@ -167,7 +167,10 @@ typedef struct svo_run_info {
   uint64_t n_nodes;
   uint64_t n_data;
   int hazard;
-  float ms_partition, ms_voxelize, ms_build; /* device time per stage */
+  /* time per stage by the device's clock, from a stage's start to the next one's: waits on the
+   * host and what the sink of a streamed run takes (ms_build) are in it. One partition has no
+   * partition stage (0). */
+  float ms_partition, ms_voxelize, ms_build;
   uint32_t launches;       /* kernel launches the call issued outside graphs */
   uint32_t host_syncs;     /* host waits on the device the call made */
   uint32_t graph_launches; /* hipGraph launches (svo_batch_run with graphs on) */

@@ -862,7 +862,8 @@ static int run_impl(svo_ctx* ctx, const float* records, uint64_t n_triangles, in
   const float u_vox =
       (text_roundtrip(bbox[3]) - text_roundtrip(bbox[0])) / (float)gridsize;  // main.cpp:311
   // stage boundaries: the device clock at the start of a pass, of a build and at its read-back
-  // (an event per boundary costs a barrier packet on the stream)
+  // (an event per boundary costs a barrier packet on the stream). A streamed build's records go
+  // out after its read-back: it lasts until the next partition's pass, the last one to the end
   float ms_p = 0, ms_v = 0, ms_b = 0;
   auto ms_between = [&](uint64_t t0, uint64_t t1) {
     return t0 && t1 > t0 ? (float)((double)(t1 - t0) / c.wall_khz) : 0.0f;
@@ -883,6 +884,7 @@ static int run_impl(svo_ctx* ctx, const float* records, uint64_t n_triangles, in
   if (streamed) {
     r = svo_stream_begin(ctx, gridsize, np, generate_levels, sink, user);
     if (r) return r;
+    uint64_t built = 0;  // since when the last partition is being built
     for (uint64_t i = 0; i < np; i++) {
       if (counts[i] == 0) continue;  // main.cpp:330
       uint64_t nf = 0;
@@ -890,15 +892,18 @@ static int run_impl(svo_ctx* ctx, const float* records, uint64_t n_triangles, in
       r = svo_voxelize(ctx, i, i * morton_part, (i + 1) * morton_part, u_vox, gridsize,
                        color_mode, &nf);
       if (r) return r;
-      const uint64_t counted = c.stamp_read;
+      ms_b += ms_between(built, c.stamp_pass);
+      built = c.stamp_read;
       r = svo_stream_partition(ctx, i);
       if (r) return r;
-      ms_v += ms_between(c.stamp_pass, nf ? c.stamp_build : counted);
-      if (nf) ms_b += ms_between(c.stamp_build, c.stamp_read);
+      if (nf) built = c.stamp_build;
+      ms_v += ms_between(c.stamp_pass, built);
     }
     r = svo_stream_end(ctx, &nn, &nd, &hz);
     if (r) return r;
-    TRYC(stream_sync(c.stream), "svo_run");  // the levels above the partitions are uploads
+    // (the levels above the partitions are uploads)
+    TRYC(read_back(c, nullptr, 0), "svo_run");
+    ms_b += ms_between(built, c.stamp_read);
   } else {
     for (uint64_t i = 0; i < np; i++) {
       if (counts[i] == 0) continue;  // main.cpp:330

@@ -2544,7 +2544,7 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
       SVO_TRY(read_back(c, rq, 2));
     }
     c.clear_counters = false;
-    c.stamp_pass = hc[kCtrStamp];
+    if (attempt == 0) c.stamp_pass = hc[kCtrStamp];
     ktimer_flush(c);
     if (dense || (!hc[kCtrOverflow] && hc[kCtrNumOcc] <= c.pool_cap)) break;
     // pool too small for the flagged bricks: clear everything, grow, redo
