@@ -165,6 +165,8 @@ static int fail(hipError_t e, const char* where) {
     if (_e != hipSuccess) return fail(_e, where); \
   } while (0)
 
+static uint64_t dense_bytes_of(uint64_t mb) { return std::min(mb, kDenseMax >> 20) << 20; }
+
 static int is_pow2_u64(uint64_t x) { return x != 0 && !(x & (x - 1)); }
 
 // What the sticky consistency-failure counter counts (kCtrError): a look-back wait of a
@@ -291,7 +293,7 @@ int svo_ctx_create(int device, svo_ctx** out) {
     if (hipMemGetInfo(&free_b, &total_b) == hipSuccess)
       ctx->c.dense_limit = std::min<uint64_t>((uint64_t)free_b / 2, 128ull << 30);
     const char* env = getenv("SVO_DENSE_LIMIT_MB");
-    if (env) ctx->c.dense_limit = (uint64_t)strtoull(env, nullptr, 10) << 20;
+    if (env) ctx->c.dense_limit = dense_bytes_of(strtoull(env, nullptr, 10));
   }
   int khz = 0;
   if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0)
@@ -359,7 +361,7 @@ void* svo_ctx_stream(svo_ctx* ctx) { return ctx ? (void*)ctx->c.stream : nullptr
 int svo_ctx_set_tuning(svo_ctx* ctx, int small_cols, uint64_t dense_limit_mb) {
   CHECK_CTX();
   if (small_cols > 0) ctx->c.tune.small_cols = small_cols;
-  if (dense_limit_mb != UINT64_MAX) ctx->c.dense_limit = dense_limit_mb << 20;
+  if (dense_limit_mb != UINT64_MAX) ctx->c.dense_limit = dense_bytes_of(dense_limit_mb);
   return SVO_OK;
 }
 

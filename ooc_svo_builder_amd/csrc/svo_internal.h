@@ -91,6 +91,9 @@ inline hipError_t launch_kernel(void (*k)(KArgs...), dim3 g, dim3 b, uint32_t sh
 constexpr int kBrickBits = 12;
 constexpr int kBrickVox = 1 << kBrickBits;
 constexpr int kBrickWords = 1 << (kBrickBits - 6);
+// Bytes of the largest dense grid (128 GiB unless a caller sets another limit): what 32-bit table
+// and line numbers reach. No card holds as much.
+constexpr uint64_t kDenseMax = 1ull << 39;
 // Per-brick counts carry a non-empty flag at bit kNonEmptyShift above the voxel count.
 constexpr int kNonEmptyShift = 40;
 constexpr uint64_t kVoxMask = (1ull << kNonEmptyShift) - 1;

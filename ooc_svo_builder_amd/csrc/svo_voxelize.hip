@@ -401,7 +401,7 @@ struct MarkGather {
   }
   __device__ __forceinline__ void touch(uint64_t) {}
   __device__ __forceinline__ void add(uint64_t code, uint32_t tri) {
-    const Rel rel = (Rel)code - base;  // (below 2^35: the dense limit is 2^37 bytes)
+    const Rel rel = (Rel)code - base;  // (below 2^37: kDensePayloadBricks)
     const uint32_t line = (uint32_t)(rel >> kLineBits);
     // neighbouring lines in neighbouring places (of a 4 x 4 x 4 block of lines: 6 bits), the
     // blocks mixed
@@ -1045,10 +1045,12 @@ struct OccStore {
     if (last) ctr[kCtrNumOcc] = (ull)(ex + v);
   }
 };
-// Dense passes: the list entries carry the brick's flagged quarters above its table index
-// (the dense limit, 2^37 cells, keeps that below 2^25).
+// Dense passes: the list entries carry the brick's flagged quarters above its table index.
 constexpr int kOccBits = 28;
 constexpr uint32_t kOccMask = (1u << kOccBits) - 1u;
+static_assert(kDenseMax >> kBrickBits <= 1ull << kOccBits, "a byte a voxel");
+// (payload units' lines of 32 cells go by number + 1)
+constexpr uint64_t kDensePayloadBricks = 1ull << (32 + kLineBits - kBrickBits);
 struct OccStoreDense {
   uint32_t* occ;
   const uint32_t* table;
@@ -2253,7 +2255,9 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     goff[u + 1] = goff[u] + ((ubase[u + 1] - ubase[u]) << kBrickBits) *
                                 (units[u].stride == 21 ? 4 : 1);
   const uint64_t dense_bytes = goff[nu];
-  const bool dense = dense_bytes <= c.dense_limit;
+  bool dense = dense_bytes <= c.dense_limit;
+  for (uint32_t u = 0; u < nu; u++)
+    dense = dense && (units[u].stride == 9 || ubase[u + 1] - ubase[u] < kDensePayloadBricks);
   bool geometry_only = true;  // no unit carries payload records
   bool small_units = true;    // no unit spans more than 2^32 voxels
   for (uint32_t u = 0; u < nu; u++) {

@@ -22,7 +22,7 @@ struct Device {
   std::map<const void*, std::string> names;  // kernels
   long allocs = 0, fail_at = -1;             // allocations since arming; the one that fails
   uint64_t n_occ = 0, n_vox = 0;             // what a pass is said to find
-  uint64_t unclean = 0, outside = 0, bad_grid = 0, marks = 0;
+  uint64_t unclean = 0, outside = 0, bad_grid = 0, marks = 0, dense = 0;
   hipError_t last = hipSuccess;
 };
 Device& dev() {
@@ -63,6 +63,7 @@ void must_be_zero(const void* p, size_t bytes) {
     dev().outside++;
     return;
   }
+  if (bytes > kHuge) return;
   for (size_t k = 0; k < bytes; k++)
     if (((const uint8_t*)p)[k]) {
       dev().unclean++;
@@ -85,17 +86,17 @@ void each(const VoxParams* units, uint32_t n, uint32_t* table, uint8_t* cflags, 
     const uint64_t nb = bricks_of(P);
     if (what & kTable) {
       if (value < 0) must_be_zero(table + P.table_base, nb * 4);
-      else if (inside(table + P.table_base, nb * 4)) memset(table + P.table_base, value, nb * 4);
+      else if (nb * 4 <= kHuge && inside(table + P.table_base, nb * 4)) memset(table + P.table_base, value, nb * 4);
       if (P.wide) {
         uint8_t* f = cflags + P.table_base * kBrickWords;
         if (value < 0) must_be_zero(f, nb * kBrickWords);
-        else if (inside(f, nb * kBrickWords)) memset(f, value, nb * kBrickWords);
+        else if (nb * kBrickWords <= kHuge && inside(f, nb * kBrickWords)) memset(f, value, nb * kBrickWords);
       }
     }
     if (P.dense && (what & (P.wide ? kCells : kBytes))) {
       const size_t bytes = nb * kBrickVox * (P.wide ? 4 : 1);
       if (value < 0) must_be_zero(P.grid8, bytes);
-      else if (inside(P.grid8, bytes)) memset(P.grid8, value, bytes);
+      else if (bytes <= kHuge && inside(P.grid8, bytes)) memset(P.grid8, value, bytes);
     }
   }
 }
@@ -208,6 +209,7 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, si
       must_be_zero(A.pool8, A.pool_cap * kBrickVox);
       if (inside(A.pool8, A.pool_cap * kBrickVox)) memset(A.pool8, 1, A.pool_cap * kBrickVox);
     } else if (is("MarkDense") || is("MarkGather")) {
+      d.dense++;
       each(g_pass.units, g_pass.n, A.table, A.cflags, kTable | kBytes | kCells, -1);
       each(g_pass.units, g_pass.n, A.table, A.cflags, kTable | kBytes | kCells, 1);
     }
@@ -219,6 +221,8 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, si
       each(g_pass.units, g_pass.n, g_pass.A.table, g_pass.A.cflags, kTable | kBytes, 0);
     else if (inside(g_pass.A.pool8, g_pass.A.pool_cap * kBrickVox))
       memset(g_pass.A.pool8, 0, g_pass.A.pool_cap * kBrickVox);
+  } else if (is("k_scan_single") && is("OccStoreDense")) {
+    if (arg<uint64_t>(args, 2) > 1ull << kOccBits) d.outside++;  // (table indices of kOccBits)
   } else if (is("k_scan_single") && is("BrickOffStore")) {
     const BrickOffStore st = arg<BrickOffStore>(args, 1);
     if (st.host) {
@@ -251,14 +255,15 @@ void state_arm(long fail_at, uint64_t n_occ, uint64_t n_vox) {
   state_found(n_occ, n_vox);
 }
 // out: allocations since arming, memory not zero when marked, accesses outside of allocations,
-// grids that HIP refuses, mark kernels
-void state_read(uint64_t out[5]) {
+// grids that HIP refuses, mark kernels, those of dense passes
+void state_read(uint64_t out[6]) {
   Device& d = dev();
   out[0] = (uint64_t)d.allocs;
   out[1] = d.unclean;
   out[2] = d.outside;
   out[3] = d.bad_grid;
   out[4] = d.marks;
+  out[5] = d.dense;
 }
 // A device-to-device copy of records.
 int state_copy(uint64_t bytes) {
@@ -269,7 +274,7 @@ int state_copy(uint64_t bytes) {
 }
 void state_clear() {
   Device& d = dev();
-  d.unclean = d.outside = d.bad_grid = d.marks = 0;
+  d.unclean = d.outside = d.bad_grid = d.marks = d.dense = 0;
   d.fail_at = -1;
 }
 }

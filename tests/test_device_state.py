@@ -18,7 +18,7 @@ from ooc_svo_builder_amd import lib as binding
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "ooc_svo_builder_amd", "csrc")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-NAMES = ("allocations", "unclean", "outside", "bad_grid", "marks")
+NAMES = ("allocations", "unclean", "outside", "bad_grid", "marks", "dense")
 
 
 @pytest.fixture(scope="module")
@@ -49,7 +49,7 @@ def _arm(L, fail_at=-1, n_occ=5, n_vox=100):
 
 
 def _state(L):
-    out = (C.c_uint64 * 5)()
+    out = (C.c_uint64 * 6)()
     L.state_read(out)
     return dict(zip(NAMES, out))
 
@@ -183,4 +183,19 @@ def test_payload_records_of_almost_two_to_the_32_voxels(device, n_vox):
     L.state_found(C.c_uint64(500), C.c_uint64(n_vox))
     assert _pass(L, ctx, True, 256) == 0
     assert _state(L)["bad_grid"] == 0
+    L.svo_ctx_destroy(ctx)
+
+
+@pytest.mark.parametrize("G,payload", [(8192, False), (16384, False), (4096, True), (8192, True)])
+def test_a_dense_limit_beyond_any_memory(device, G, payload):
+    """A caller's limit does not make a pass dense whose bricks or cells have no 32-bit place."""
+    L, ctx = device, C.c_void_p()
+    L.state_clear()
+    _arm(L)
+    assert L.svo_ctx_create(0, C.byref(ctx)) == 0
+    assert L.svo_ctx_set_tuning(ctx, 0, 1 << 40) == 0
+    assert _pass(L, ctx, payload, G) == 0
+    s = _state(L)
+    assert (s["outside"], s["bad_grid"]) == (0, 0)
+    assert s["dense"] == (G ** 3 <= 1 << (36 if payload else 39))
     L.svo_ctx_destroy(ctx)
