@@ -100,7 +100,6 @@ constexpr uint64_t kVoxMask = (1ull << kNonEmptyShift) - 1;
 
 // Device counters block (one 256-byte line of u64s).
 enum Counter : int {
-  kCtrPoolCount = 0,  // bricks allocated from the pool
   kCtrOverflow = 1,   // pool exhausted during a pass
   kCtrLargeCount = 2, // triangles deferred to the column-parallel tier
   kCtrNumOcc = 3,     // occupied bricks after compaction

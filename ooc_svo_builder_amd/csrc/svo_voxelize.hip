@@ -207,29 +207,20 @@ __device__ __forceinline__ void walk_row_cols(const Walk& K, const VoxParams& P,
   }
 }
 
-// Columns [a_lo, a_hi] of row b of a walk, narrowed to the row's interval when kNarrow
-// (a span of one or a few columns is cheaper to test column by column).
-template <bool kNarrow, typename Act>
-__device__ __forceinline__ void walk_row_span(const Walk& K, const VoxParams& P, int b, int a_lo,
-                                              int a_hi, Act& act) {
-  const ColRow R = col_row(K, P, b);
-  int i0 = a_lo, i1 = a_hi;
-  if constexpr (kNarrow) {
-    row_interval(K, R, P.unit, i0, i1);
-    i0 = max(i0, a_lo);
-    i1 = min(i1, a_hi);
-    if (i0 > i1) return;
-  }
+// Column (a, b) of a walk.
+template <typename Act>
+__device__ __forceinline__ void walk_one_column(const Walk& K, const VoxParams& P, int a, int b,
+                                                Act& act) {
   const int w = K.w();
   const int ua = (w == 0) ? 1 : 0;
   const int va = (w == 2) ? 1 : 2;
-  walk_row_cols(K, P, b, R, i0, i1, spread3_s((uint32_t)i0) << ua,
+  walk_row_cols(K, P, b, col_row(K, P, b), a, a, spread3_s((uint32_t)a) << ua,
                 spread3_s((uint32_t)b) << va, ua, act);
 }
 
 // All columns of a walk, row by row, the Morton parts of a and b stepped incrementally;
-// with 'narrow' (units whose items are segments of several columns) rows are narrowed to
-// their interval (rows narrower than kRowSpanMin columns are walked whole).
+// with 'narrow' rows are narrowed to their interval (rows narrower than kRowSpanMin columns are
+// walked whole).
 template <typename Act>
 __device__ __forceinline__ void walk_all_columns(const Walk& K, const VoxParams& P, Act& act,
                                                  bool narrow) {
@@ -628,7 +619,7 @@ __device__ __forceinline__ void walk_queued(const VoxParams& P, const ActArgs& A
   typename Act::Unordered act = Act::Unordered::make(A, P, nullptr);
   const uint32_t col = e & kColMask, na = (uint32_t)(Q.i[I_G1U] - Q.i[I_G0U] + 1);
   const int a = Q.i[I_G0U] + (int)(col % na);
-  walk_row_span<false>(Q, P, Q.i[I_G0V] + (int)(row0 + col / na), a, a, act);
+  walk_one_column(Q, P, a, Q.i[I_G0V] + (int)(row0 + col / na), act);
 }
 
 // Rows [row0, row0 + nrows) of the lanes' triangles (nall rows each; their walks K, their linear forms in
@@ -2212,12 +2203,11 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
       small_cols = (int)std::max<int64_t>(small_cols, std::min<int64_t>(4ll * small_cols, 1 << 16));
     } else
       tt = (uint32_t)std::min<uint64_t>(kTileTris, (all / (4 * waves) + 7) / 8 * 8);
-    // A pass of one mesh with 16 or more tiles per block of the persistent grid has the
-    // parallelism to walk triangles of up to 16 x small_cols columns in the small tier (rows
-    // narrowed to their intervals, a triangle's segments shared by its block's threads),
-    // which is faster than the large tier's thread per bbox column (the soup of 5x10^7
-    // triangles at 8192, 8 partitions: 68.6 -> 61.1 ms per step). Batches keep their
-    // autotuned threshold.
+    // A pass of one mesh with 12 or more tiles of 64 triangles per wave of the persistent grid
+    // keeps triangles of up to 16 x small_cols columns in the small tier: its waves are busy, and
+    // the large tier would list them and read them again. Soups in 8 partitions, so and with 1024
+    // columns: 6M triangles at 4096 4.8 and 6.6 ms, 50M at 8192 40.5 and 46.4, 50M at 4096 (few such
+    // triangles) 13.4 and 13.5. Batches keep their autotuned threshold.
     if (!batch && all >= 16 * blocks * 192)
       small_cols = std::max(small_cols, (int)std::min<int64_t>(16ll * small_cols, 1 << 16));
   }
@@ -2479,7 +2469,7 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
       };
       if (dense) {
         SVO_TRY(small_units ? mark_dense(std::true_type{}) : mark_dense(std::false_type{}));
-        // number the flagged bricks in Morton order: table entry = rank + 1, occ = list
+        // list the flagged bricks in Morton order, with their flagged quarters
         SVO_TRY(occ_scan());
       } else {
         SVO_TRY(tile_pass(TouchAction{}, "vox_small_touch", queues, 1, 0));
