@@ -2554,6 +2554,7 @@ hipError_t voxelize_units(Context& c, const std::vector<VoxUnit>& hu, bool batch
     SVO_TRY(ensure(c.pool8, want * kBrickVox));
     SVO_TRY(fill_u64(c.pool8.as<uint64_t>(), 0, want * kBrickVox / 8, c.stream));
     c.pool_cap = want;
+    pool_words = c.pool.as<ull>();
   }
   const uint64_t n_occ = hc[kCtrNumOcc];
   const uint64_t nvox = hc[kCtrNumVox] & kVoxMask;

@@ -70,6 +70,9 @@ void must_be_zero(const void* p, size_t bytes) {
       return;
     }
 }
+void must_hold(const void* p, size_t bytes) {
+  if (!inside(p, bytes)) dev().outside++;
+}
 template <typename T>
 T arg(void** args, int k) {
   return *(T*)args[k];
@@ -208,6 +211,10 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, si
     } else if (is("MarkPool")) {
       must_be_zero(A.pool8, A.pool_cap * kBrickVox);
       if (inside(A.pool8, A.pool_cap * kBrickVox)) memset(A.pool8, 1, A.pool_cap * kBrickVox);
+    } else if (is("WinnerAction")) {
+      must_hold(A.pool, d.n_occ * kBrickWords * 8);
+      must_hold(A.wprefix, d.n_occ * kBrickWords * 4);
+      must_hold(A.winner, d.n_vox * 4);
     } else if (is("MarkDense") || is("MarkGather")) {
       d.dense++;
       each(g_pass.units, g_pass.n, A.table, A.cflags, kTable | kBytes | kCells, -1);
@@ -217,7 +224,11 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, si
     ull* ctr = (ull*)g_pass.A.ctr;
     ctr[kCtrNumOcc] = d.n_occ;
     ctr[kCtrNumVox] = d.n_vox | (d.n_occ << kNonEmptyShift);
-    if (arg<uint32_t*>(args, 11))  // a dense pass
+    const uint64_t n = std::min(d.n_occ, arg<uint64_t>(args, 2));
+    must_hold(arg<ull*>(args, 8), n * kBrickWords * 8);  // the bricks' words and counts
+    must_hold(arg<uint64_t*>(args, 9), n * 8);
+    if (arg<uint64_t*>(args, 10)) must_hold(arg<uint64_t*>(args, 10), n * 8);
+    if (arg<uint32_t*>(args, 12))  // a dense pass
       each(g_pass.units, g_pass.n, g_pass.A.table, g_pass.A.cflags, kTable | kBytes, 0);
     else if (inside(g_pass.A.pool8, g_pass.A.pool_cap * kBrickVox))
       memset(g_pass.A.pool8, 0, g_pass.A.pool_cap * kBrickVox);
@@ -234,6 +245,12 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, si
     for (uint32_t u = 0; u <= n; u++) arg<uint64_t*>(args, 6)[u] = d.n_vox * u / n;
   } else if (is("k_payload_bricks")) {
     each(g_pass.units, g_pass.n, nullptr, nullptr, kCells, 0);
+  } else if (is("k_brick_emit")) {
+    must_hold(arg<ull*>(args, 5), d.n_occ * kBrickWords * 8);
+    must_hold(arg<uint64_t*>(args, 6), d.n_occ * 8);
+    must_hold(arg<uint64_t*>(args, 10), d.n_occ * kBrickWords * 8);
+    if (arg<uint32_t*>(args, 8)) must_hold(arg<uint64_t*>(args, 7), d.n_vox * 8);
+    if (arg<uint32_t*>(args, 8)) must_hold(arg<uint32_t*>(args, 8), d.n_occ * kBrickWords * 4);
   } else if (is("k_brick_clear")) {
     each(g_pass.units, g_pass.n, g_pass.A.table, nullptr, kTable, 0);
   } else if (is("k_up_small")) {  // the build's bookkeeping (no nodes, no flags)

@@ -199,3 +199,21 @@ def test_a_dense_limit_beyond_any_memory(device, G, payload):
     assert (s["outside"], s["bad_grid"]) == (0, 0)
     assert s["dense"] == (G ** 3 <= 1 << (36 if payload else 39))
     L.svo_ctx_destroy(ctx)
+
+
+@pytest.mark.parametrize("payload", [False, True])
+def test_slots_that_grow(device, payload):
+    """Passes on touched bricks that need more slots than there are: the redone pass goes through
+    the new ones, and what it writes has room."""
+    L, ctx = device, C.c_void_p()
+    L.state_clear()
+    _arm(L)
+    assert L.svo_ctx_create(0, C.byref(ctx)) == 0
+    assert L.svo_ctx_set_tuning(ctx, 0, 0) == 0
+    for n_occ in (500, 1500, 40000, 90000, 2000):
+        _find(L, n_occ)
+        marks = _state(L)["marks"]
+        assert _pass(L, ctx, payload, 1024) == 0
+        s = _state(L)
+        assert s["marks"] > marks and (s["unclean"], s["outside"], s["bad_grid"]) == (0, 0, 0), (n_occ, s)
+    L.svo_ctx_destroy(ctx)
