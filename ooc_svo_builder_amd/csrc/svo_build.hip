@@ -339,8 +339,12 @@ constexpr int kTailBlock = 1024;
 constexpr uint64_t kTailLevelMax = 8192;  // largest level bound the tail block takes
 // The level scans' stores walk a parent's children (dependent loads, and with -levels their
 // averages): one element a thread up to this many keeps enough blocks in flight. With eight,
-// the levels of 487,600 voxels ran on 60 blocks: 375 us for four of them.
+// the levels of 487,600 voxels ran on 60 blocks: 375 us for four of them. Without -levels a store
+// does less, and the blocks' look-back costs more than their number gives from 2M elements on: added
+// voxels' builds, one and eight a thread, 1.4M 337 and 362 us, 2.0M 304 and 397, 2.5M 1171 and 1094,
+// 4M 1709 and 1402, 8M 1047 and 866.
 constexpr uint64_t kLevelScanSmall = 1ull << 23;
+constexpr uint64_t kPlainScanSmall = 1ull << 21;
 constexpr uint64_t kTopLevelMax = 4096;  // largest level bound k_emit_levels_top takes
 __global__ __launch_bounds__(kTailBlock) void k_levels_tail(
     Arena A, LevelMeta M, Tags T, JobDev* jobs, uint32_t n_jobs, const uint64_t* leaves,
@@ -1417,7 +1421,8 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
     const bool up_small = up_once && NB <= kTailBlock && nup <= kSmallNodes;
     const int h_scan_end = up_once ? h0 : h_tail;  // level scans for h0 .. h_scan_end-1
     uint64_t st_words = 0;
-    for (int h = h0; h < h_scan_end; h++) st_words += scan_single_words(bound[h], kLevelScanSmall);
+    const uint64_t scan_small = levels ? kLevelScanSmall : kPlainScanSmall;
+    for (int h = h0; h < h_scan_end; h++) st_words += scan_single_words(bound[h], scan_small);
     SVO_TRY(ensure(c.lvl_aux, (meta_words + st_words) * 8));
     if (levels) {
       SVO_TRY(ensure(c.lvl_isize, cap * 8));
@@ -1506,8 +1511,8 @@ hipError_t build_jobs(Context& c, uint32_t n_jobs, bool tagged, int levels,
                        root_size, root_isize, c.records.as<float>() + 8, h};
         SVO_TRY((scan_single<uint32_t>(ld, st, bound[h], status,
                                        c.counters.as<unsigned long long>() + kCtrError, c.stream,
-                                       M.n + h, kLevelScanSmall)));
-        status += scan_single_words(bound[h], kLevelScanSmall);
+                                       M.n + h, scan_small)));
+        status += scan_single_words(bound[h], scan_small);
       }
       if (!up_once || (tagged && !up_small))
         SVO_LAUNCH(k_levels_tail, dim3(1), dim3(kTailBlock), 0, c.stream, A, M, T, d_jobs,
