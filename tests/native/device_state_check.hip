@@ -2,7 +2,8 @@
 // garbage, allocations fail on demand, and the few kernels that matter here are imitated (fills,
 // read-backs, and which buffers a pass leaves marked or clears). Checked at every mark kernel: the
 // table, flags, cells and slots that it is given lie in live allocations and are zero; and at
-// every launch, that the grid is one HIP accepts.
+// every launch, that the grid is one HIP accepts and that no argument points into memory that was
+// given back (whose addresses are not used again here).
 #include "../../ooc_svo_builder_amd/csrc/svo_voxelize.hip"
 
 #include <sys/mman.h>
@@ -18,11 +19,13 @@ using namespace svo;
 namespace {
 constexpr size_t kHuge = 256u << 20;  // allocations above are address space, neither filled nor read
 struct Device {
-  std::map<uintptr_t, size_t> mem;           // live allocations
+  std::map<uintptr_t, size_t> mem, gone;     // live allocations, those given back
   std::map<const void*, std::string> names;  // kernels
   long allocs = 0, fail_at = -1;             // allocations since arming; the one that fails
   uint64_t n_occ = 0, n_vox = 0;             // what a pass is said to find
-  uint64_t unclean = 0, outside = 0, bad_grid = 0, marks = 0, dense = 0;
+  uint64_t found = 0;                        // its bricks: no more than there are
+  uint64_t unclean = 0, outside = 0, bad_grid = 0, marks = 0, dense = 0, stale = 0;
+  std::vector<uint8_t> args;  // of the launch (the library's launch log)
   hipError_t last = hipSuccess;
 };
 Device& dev() {
@@ -40,23 +43,32 @@ hipError_t allocate(void** p, size_t bytes) {
   Device& d = dev();
   *p = nullptr;
   if (d.allocs++ == d.fail_at) return d.last = hipErrorOutOfMemory;
-  if (bytes > kHuge) {
-    *p = mmap(nullptr, bytes, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
-  } else {
-    *p = malloc(bytes);
-    memset(*p, 0xA5, bytes);
-  }
+  *p = mmap(nullptr, bytes, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
+  if (bytes <= kHuge) memset(*p, 0xA5, bytes);
   d.mem[(uintptr_t)*p] = bytes;
   return hipSuccess;
 }
 hipError_t give_back(void* p) {
-  const size_t bytes = dev().mem[(uintptr_t)p];
-  dev().mem.erase((uintptr_t)p);
-  if (bytes > kHuge)
-    munmap(p, bytes);
-  else
-    free(p);
+  Device& d = dev();
+  const size_t bytes = d.mem[(uintptr_t)p];
+  d.mem.erase((uintptr_t)p);
+  // the addresses stay taken
+  mmap(p, bytes, PROT_NONE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE | MAP_FIXED, -1, 0);
+  d.gone[(uintptr_t)p] = bytes;
   return hipSuccess;
+}
+// the launch's arguments, word by word: an address in memory that was given back
+void look_for_stale() {
+  Device& d = dev();
+  for (size_t k = 0; k + 8 <= d.args.size(); k += 4) {
+    uintptr_t v;
+    memcpy(&v, d.args.data() + k, 8);
+    auto it = d.gone.upper_bound(v);
+    if (it == d.gone.begin()) continue;
+    --it;
+    if (v < it->first + it->second) d.stale++;
+  }
+  d.args.clear();
 }
 void must_be_zero(const void* p, size_t bytes) {
   if (!inside(p, bytes)) {
@@ -178,6 +190,7 @@ void __hipRegisterFunction(void**, const void* f, char*, const char* name, unsig
 
 hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, size_t, hipStream_t) {
   Device& d = dev();
+  look_for_stale();
   // HIP's limits: 2^32 - 1 threads along x, 1024 in a block
   if (!grid.x || (uint64_t)grid.x * block.x > 0xFFFFFFFFull || block.x > 1024) {
     d.bad_grid++;
@@ -212,8 +225,8 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, si
       must_be_zero(A.pool8, A.pool_cap * kBrickVox);
       if (inside(A.pool8, A.pool_cap * kBrickVox)) memset(A.pool8, 1, A.pool_cap * kBrickVox);
     } else if (is("WinnerAction")) {
-      must_hold(A.pool, d.n_occ * kBrickWords * 8);
-      must_hold(A.wprefix, d.n_occ * kBrickWords * 4);
+      must_hold(A.pool, d.found * kBrickWords * 8);
+      must_hold(A.wprefix, d.found * kBrickWords * 4);
       must_hold(A.winner, d.n_vox * 4);
     } else if (is("MarkDense") || is("MarkGather")) {
       d.dense++;
@@ -222,9 +235,12 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, si
     }
   } else if (is("k_brick_count")) {
     ull* ctr = (ull*)g_pass.A.ctr;
-    ctr[kCtrNumOcc] = d.n_occ;
-    ctr[kCtrNumVox] = d.n_vox | (d.n_occ << kNonEmptyShift);
-    const uint64_t n = std::min(d.n_occ, arg<uint64_t>(args, 2));
+    uint64_t all = 0;
+    for (uint32_t u = 0; u < g_pass.n; u++) all += bricks_of(g_pass.units[u]);
+    d.found = std::min(d.n_occ, all);
+    ctr[kCtrNumOcc] = d.found;
+    ctr[kCtrNumVox] = d.n_vox | (d.found << kNonEmptyShift);
+    const uint64_t n = std::min(d.found, arg<uint64_t>(args, 2));
     must_hold(arg<ull*>(args, 8), n * kBrickWords * 8);  // the bricks' words and counts
     must_hold(arg<uint64_t*>(args, 9), n * 8);
     if (arg<uint64_t*>(args, 10)) must_hold(arg<uint64_t*>(args, 10), n * 8);
@@ -246,15 +262,18 @@ hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, si
   } else if (is("k_payload_bricks")) {
     each(g_pass.units, g_pass.n, nullptr, nullptr, kCells, 0);
   } else if (is("k_brick_emit")) {
-    must_hold(arg<ull*>(args, 5), d.n_occ * kBrickWords * 8);
-    must_hold(arg<uint64_t*>(args, 6), d.n_occ * 8);
-    must_hold(arg<uint64_t*>(args, 10), d.n_occ * kBrickWords * 8);
+    must_hold(arg<ull*>(args, 5), d.found * kBrickWords * 8);
+    must_hold(arg<uint64_t*>(args, 6), d.found * 8);
+    must_hold(arg<uint64_t*>(args, 10), d.found * kBrickWords * 8);
     if (arg<uint32_t*>(args, 8)) must_hold(arg<uint64_t*>(args, 7), d.n_vox * 8);
-    if (arg<uint32_t*>(args, 8)) must_hold(arg<uint32_t*>(args, 8), d.n_occ * kBrickWords * 4);
+    if (arg<uint32_t*>(args, 8)) must_hold(arg<uint32_t*>(args, 8), d.found * kBrickWords * 4);
   } else if (is("k_brick_clear")) {
     each(g_pass.units, g_pass.n, g_pass.A.table, nullptr, kTable, 0);
-  } else if (is("k_up_small")) {  // the build's bookkeeping (no nodes, no flags)
-    memset(*(uint64_t**)args[1], 0, (2 * 64 + 8) * 8);
+  } else if (is("k_up_small") || is("k_up_scan") || is("k_build_init")) {
+    // the build's bookkeeping: no flags, some nodes
+    uint64_t* meta = *(uint64_t**)args[is("k_build_init") ? 0 : 1];
+    memset(meta, 0, (2 * 64 + 8) * 8);
+    meta[2 * 64 + 2] = 1000;
   }
   return hipSuccess;
 }
@@ -272,8 +291,8 @@ void state_arm(long fail_at, uint64_t n_occ, uint64_t n_vox) {
   state_found(n_occ, n_vox);
 }
 // out: allocations since arming, memory not zero when marked, accesses outside of allocations,
-// grids that HIP refuses, mark kernels, those of dense passes
-void state_read(uint64_t out[6]) {
+// grids that HIP refuses, mark kernels, those of dense passes, arguments in memory given back
+void state_read(uint64_t out[7]) {
   Device& d = dev();
   out[0] = (uint64_t)d.allocs;
   out[1] = d.unclean;
@@ -281,6 +300,7 @@ void state_read(uint64_t out[6]) {
   out[3] = d.bad_grid;
   out[4] = d.marks;
   out[5] = d.dense;
+  out[6] = d.stale;
 }
 // A device-to-device copy of records.
 int state_copy(uint64_t bytes) {
@@ -291,7 +311,9 @@ int state_copy(uint64_t bytes) {
 }
 void state_clear() {
   Device& d = dev();
-  d.unclean = d.outside = d.bad_grid = d.marks = d.dense = 0;
+  d.unclean = d.outside = d.bad_grid = d.marks = d.dense = d.stale = 0;
   d.fail_at = -1;
+  d.args.clear();
+  t_launch_log = &d.args;
 }
 }

@@ -18,7 +18,7 @@ from ooc_svo_builder_amd import lib as binding
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "ooc_svo_builder_amd", "csrc")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-NAMES = ("allocations", "unclean", "outside", "bad_grid", "marks", "dense")
+NAMES = ("allocations", "unclean", "outside", "bad_grid", "marks", "dense", "stale")
 
 
 @pytest.fixture(scope="module")
@@ -49,7 +49,7 @@ def _arm(L, fail_at=-1, n_occ=5, n_vox=100):
 
 
 def _state(L):
-    out = (C.c_uint64 * 6)()
+    out = (C.c_uint64 * 7)()
     L.state_read(out)
     return dict(zip(NAMES, out))
 
@@ -107,7 +107,7 @@ def _fail_each(L, first, grown, after, marked, dense_mb=None):
             for f in after:
                 assert f(ctx) == 0, k
             s = _state(L)
-            assert (s["unclean"], s["outside"], s["bad_grid"]) == (0, 0, 0), (k, s)
+            assert (s["unclean"], s["outside"], s["bad_grid"], s["stale"]) == (0, 0, 0, 0), (k, s)
         L.svo_ctx_destroy(ctx)
     raise AssertionError("the pass still allocates after 100 allocations")
 
@@ -215,5 +215,54 @@ def test_slots_that_grow(device, payload):
         marks = _state(L)["marks"]
         assert _pass(L, ctx, payload, 1024) == 0
         s = _state(L)
-        assert s["marks"] > marks and (s["unclean"], s["outside"], s["bad_grid"]) == (0, 0, 0), (n_occ, s)
+        assert s["marks"] > marks and (s["unclean"], s["outside"], s["bad_grid"], s["stale"]) == (0, 0, 0, 0), (n_occ, s)
+    L.svo_ctx_destroy(ctx)
+
+
+def _run(L, ctx, payload, G, limit=2048, levels=0, n=40, sink=None):
+    t, b, info = _mesh(payload, n), np.array([0, 0, 0, 1, 1, 1], np.float32), binding.RunInfo()
+    p = lambda a: a.ctypes.data_as(C.c_void_p)  # noqa: E731
+    if sink is not None:
+        return L.svo_run_stream(ctx, p(t), len(t), int(payload), 0, p(b), G, limit, 0, levels, sink, None,
+                                C.byref(info))
+    return L.svo_run(ctx, p(t), len(t), int(payload), 0, p(b), G, limit, 0, levels, C.byref(info))
+
+
+@pytest.mark.parametrize("dense", [True, False])
+def test_no_launch_is_given_memory_that_is_gone(device, dense):
+    """Whole calls of growing and shrinking sizes on one context, each after every other."""
+    L, ctx = device, C.c_void_p()
+    L.state_clear()
+    _arm(L)
+    assert L.svo_ctx_create(0, C.byref(ctx)) == 0
+    assert L.svo_ctx_set_graphs(ctx, 0) == 0
+    if not dense:
+        assert L.svo_ctx_set_tuning(ctx, 0, 0) == 0
+    sink = binding.SINK_FN(lambda user, kind, p, n: 0)
+    dst = np.zeros(1 << 20, np.uint8)
+    codes = np.arange(5000, dtype=np.uint64)
+
+    def added(c):
+        t = _mesh(False, 0)
+        rc = L.svo_mesh_load(c, t.ctypes.data_as(C.c_void_p), 0, 0, 0)
+        rc = rc or L.svo_add_voxels(c, codes.ctypes.data_as(C.c_void_p), None, len(codes))
+        return rc or L.svo_build(c, 64, 1, None, None, None)
+
+    calls = [lambda c: _run(L, c, False, 64), lambda c: _run(L, c, True, 64), lambda c: _run(L, c, True, 128, levels=1),
+             lambda c: _run(L, c, False, 128, 2, n=3000), lambda c: _run(L, c, True, 128, 2),
+             lambda c: _run(L, c, True, 128, 2, 1), lambda c: _run(L, c, True, 128, 2, 0, 90, sink),
+             lambda c: _batch(L, c, 64, (False, True)), lambda c: _batch(L, c, 128, (True, True, False)), added,
+             lambda c: L.svo_copy_nodes(c, dst.ctypes.data_as(C.c_void_p), 0, 10)]
+    step = 0
+    for n_occ in (5, 1500, 90, 9000):
+        for a in calls:
+            for b in calls:
+                _find(L, n_occ)
+                for f in (a, b):
+                    rc = f(ctx)
+                    s = _state(L)
+                    assert rc == 0 or f is calls[-1], (step, rc, L.svo_last_error())
+                    assert (s["unclean"], s["outside"], s["bad_grid"], s["stale"]) == (0, 0, 0, 0), (step, s)
+                    step += 1
+        _find(L, 20 * n_occ)
     L.svo_ctx_destroy(ctx)
